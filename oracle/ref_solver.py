@@ -45,7 +45,7 @@ def der_available() -> bool:
 def build() -> bool:
     """Build the driver when the reference's sources are present; returns
     whether it is available afterwards."""
-    if os.path.isdir(REF):
+    if os.path.isfile(os.path.join(REF, "src/class_solver/class_solver_3d.f90")):
         subprocess.run(["sh", BUILD], check=True, capture_output=True)
     return available()
 
