@@ -13,10 +13,8 @@
 // * Learned closure: an MLP 10 -> 64 -> 64 -> 6 (tanh) from the filtered
 //   velocity gradients and the filter width to the six SGS stresses.  Weights
 //   are bf16 (rounded from FP32 master weights after every optimiser step),
-//   arithmetic FP32.  One block of 64 threads handles 64 samples: forward in
-//   registers with the activations kept in LDS, backward into per-block
-//   gradient partials that a second kernel sums in a fixed order
-//   (deterministic), then Adam.
+//   arithmetic FP32 (mlp.h: FP32 MFMA; per-block FP64 gradient partials that a
+//   second kernel sums in a fixed order), then Adam.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -28,18 +26,11 @@
 
 #include "gemm.h"
 #include "internal.h"
+#include "mlp.h"
 #include "mflops/mf.h"
 
 namespace mf {
 namespace les {
-
-constexpr int I0 = 10, H = 64, O = 6;
-constexpr int NW1 = H * I0, NW2 = H * H, NW3 = O * H;
-constexpr int OB1 = NW1, OW2 = OB1 + H, OB2 = OW2 + NW2, OW3 = OB2 + H, OB3 = OW3 + NW3;
-constexpr int NPARAM = OB3 + O;  // 5254
-constexpr int SPB = 64;          // samples per block
-
-__device__ __forceinline__ float bf2f(unsigned short b) { return __uint_as_float((unsigned)b << 16); }
 
 __device__ __forceinline__ unsigned short f2bf(float x) {
   unsigned u = __float_as_uint(x);
@@ -54,169 +45,6 @@ __global__ void __launch_bounds__(256) round_kernel(const float *__restrict__ p,
   if (t < NW1) wb[t] = f2bf(p[t]);
   else if (t < NW1 + NW2) wb[t] = f2bf(p[OW2 + (t - NW1)]);
   else if (t < NW1 + NW2 + NW3) wb[t] = f2bf(p[OW3 + (t - NW1 - NW2)]);
-}
-
-struct Net {
-  float w1[NW1], w2[NW2], w3[NW3], b1[H], b2[H], b3[O];
-};
-
-__device__ void load_net(Net &n, const unsigned short *__restrict__ wb, const float *__restrict__ p) {
-  for (int t = threadIdx.x; t < NW1; t += blockDim.x) n.w1[t] = bf2f(wb[t]);
-  for (int t = threadIdx.x; t < NW2; t += blockDim.x) n.w2[t] = bf2f(wb[NW1 + t]);
-  for (int t = threadIdx.x; t < NW3; t += blockDim.x) n.w3[t] = bf2f(wb[NW1 + NW2 + t]);
-  for (int t = threadIdx.x; t < H; t += blockDim.x) { n.b1[t] = p[OB1 + t]; n.b2[t] = p[OB2 + t]; }
-  for (int t = threadIdx.x; t < O; t += blockDim.x) n.b3[t] = p[OB3 + t];
-}
-
-// Y[s][0..5] for samples s < n; X row-major (n x 10)
-__global__ void __launch_bounds__(64) mlp_forward_kernel(const float *__restrict__ X,
-                                                         float *__restrict__ Y, long n,
-                                                         const unsigned short *__restrict__ wb,
-                                                         const float *__restrict__ p) {
-  __shared__ Net net;
-  __shared__ float A[SPB][H + 1];  // h1, one row per sample
-  load_net(net, wb, p);
-  __syncthreads();
-  const int tid = threadIdx.x;
-  const long s = (long)blockIdx.x * SPB + tid;
-  if (s >= n) return;
-  float x[I0];
-#pragma unroll
-  for (int j = 0; j < I0; ++j) x[j] = X[s * I0 + j];
-  for (int i = 0; i < H; ++i) {
-    float a = net.b1[i];
-#pragma unroll
-    for (int j = 0; j < I0; ++j) a = fmaf(net.w1[i * I0 + j], x[j], a);
-    A[tid][i] = tanhf(a);
-  }
-  float y[O];
-#pragma unroll
-  for (int o = 0; o < O; ++o) y[o] = net.b3[o];
-  for (int i = 0; i < H; ++i) {
-    float a = net.b2[i];
-    for (int j = 0; j < H; ++j) a = fmaf(net.w2[i * H + j], A[tid][j], a);
-    const float h2 = tanhf(a);
-    #pragma unroll
-    for (int o = 0; o < O; ++o) y[o] = fmaf(net.w3[o * H + i], h2, y[o]);
-  }
-  for (int o = 0; o < O; ++o) Y[s * O + o] = y[o];
-}
-
-// Gradient of sum_s sum_c (Y - T)^2 / n over the block's samples:
-// part[blk * (NPARAM + 1) + q] (q = NPARAM: the block's loss term).
-__global__ void __launch_bounds__(64) mlp_grad_kernel(const float *__restrict__ X,
-                                                      const float *__restrict__ T, long n,
-                                                      const unsigned short *__restrict__ wb,
-                                                      const float *__restrict__ p,
-                                                      float *__restrict__ part) {
-  __shared__ Net net;
-  __shared__ float A[SPB][H + 1], B[SPB][H + 1];  // h1 -> dh1, h2 -> dh2
-  __shared__ float Xs[SPB][I0], dY[SPB][O];
-  load_net(net, wb, p);
-  const int tid = threadIdx.x;
-  const long s = (long)blockIdx.x * SPB + tid;
-  const bool on = s < n;
-  for (int j = 0; j < I0; ++j) Xs[tid][j] = on ? X[s * I0 + j] : 0.0f;
-  __syncthreads();
-  // forward
-  for (int i = 0; i < H; ++i) {
-    float a = net.b1[i];
-    for (int j = 0; j < I0; ++j) a = fmaf(net.w1[i * I0 + j], Xs[tid][j], a);
-    A[tid][i] = tanhf(a);
-  }
-  float y[O];
-  for (int o = 0; o < O; ++o) y[o] = net.b3[o];
-  for (int i = 0; i < H; ++i) {
-    float a = net.b2[i];
-    for (int j = 0; j < H; ++j) a = fmaf(net.w2[i * H + j], A[tid][j], a);
-    const float h2 = tanhf(a);
-    B[tid][i] = h2;
-    #pragma unroll
-    for (int o = 0; o < O; ++o) y[o] = fmaf(net.w3[o * H + i], h2, y[o]);
-  }
-  const float inv_n = 1.0f / (float)n;
-  float loss = 0.0f;
-  for (int o = 0; o < O; ++o) {
-    const float d = on ? y[o] - T[s * O + o] : 0.0f;
-    loss = fmaf(d, d, loss);
-    dY[tid][o] = 2.0f * d * inv_n;
-  }
-  __syncthreads();
-  float *g = part + (long)blockIdx.x * (NPARAM + 1);
-  // W3 and b3: thread tid owns column j = tid of the six rows
-  for (int o = 0; o < O; ++o) {
-    float a = 0.0f;
-    for (int q = 0; q < SPB; ++q) a = fmaf(dY[q][o], B[q][tid], a);
-    g[OW3 + o * H + tid] = a;
-  }
-  if (tid < O) {
-    float a = 0.0f;
-    for (int q = 0; q < SPB; ++q) a += dY[q][tid];
-    g[OB3 + tid] = a;
-  }
-  __syncthreads();
-  // dh2 = (W3^T dY) (1 - h2^2), in place of h2 (own row)
-  for (int i = 0; i < H; ++i) {
-    float a = 0.0f;
-    for (int o = 0; o < O; ++o) a = fmaf(net.w3[o * H + i], dY[tid][o], a);
-    const float h2 = B[tid][i];
-    B[tid][i] = a * (1.0f - h2 * h2);
-  }
-  __syncthreads();
-  // W2 (row i = tid) and b2
-  {
-    float acc[H];
-    for (int j = 0; j < H; ++j) acc[j] = 0.0f;
-    float gb = 0.0f;
-    for (int q = 0; q < SPB; ++q) {
-      const float d = B[q][tid];
-      gb += d;
-      for (int j = 0; j < H; ++j) acc[j] = fmaf(d, A[q][j], acc[j]);
-    }
-    for (int j = 0; j < H; ++j) g[OW2 + tid * H + j] = acc[j];
-    g[OB2 + tid] = gb;
-  }
-  __syncthreads();
-  // dh1 = (W2^T dh2) (1 - h1^2), in place of h1 (own row)
-  for (int j = 0; j < H; ++j) {
-    float a = 0.0f;
-    for (int i = 0; i < H; ++i) a = fmaf(net.w2[i * H + j], B[tid][i], a);
-    const float h1 = A[tid][j];
-    A[tid][j] = a * (1.0f - h1 * h1);
-  }
-  __syncthreads();
-  // W1 (row i = tid) and b1
-  {
-    float acc[I0];
-    for (int j = 0; j < I0; ++j) acc[j] = 0.0f;
-    float gb = 0.0f;
-    for (int q = 0; q < SPB; ++q) {
-      const float d = A[q][tid];
-      gb += d;
-      for (int j = 0; j < I0; ++j) acc[j] = fmaf(d, Xs[q][j], acc[j]);
-    }
-    for (int j = 0; j < I0; ++j) g[tid * I0 + j] = acc[j];
-    g[OB1 + tid] = gb;
-  }
-  // the block's loss (fixed-order tree over its samples)
-  __shared__ float ls[SPB];
-  ls[tid] = loss * inv_n;
-  __syncthreads();
-  for (int o = SPB / 2; o > 0; o >>= 1) {
-    if (tid < o) ls[tid] += ls[tid + o];
-    __syncthreads();
-  }
-  if (tid == 0) g[NPARAM] = ls[0];
-}
-
-// grad[q] = sum_b part[b (NPARAM + 1) + q], b ascending (FP64 sum)
-__global__ void __launch_bounds__(256) mlp_reduce_kernel(const float *__restrict__ part, int nb,
-                                                         float *__restrict__ grad) {
-  const int q = blockIdx.x * 256 + threadIdx.x;
-  if (q > NPARAM) return;
-  double a = 0.0;
-  for (int b = 0; b < nb; ++b) a += part[(long)b * (NPARAM + 1) + q];
-  grad[q] = (float)a;
 }
 
 // Adam (beta1 0.9, beta2 0.999, eps 1e-8) with bias correction at step t
@@ -776,8 +604,9 @@ extern "C" int mf_les_nu(const double *const *du, const double *gx, int nx, cons
 struct mf_mlp {
   float *p = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;  // NPARAM (+1 for g)
   unsigned short *wb = nullptr;
-  float *part = nullptr;
+  double *part = nullptr;  // per-block gradient partials, grown to the largest grid
   long part_blocks = 0;
+  int ncu = 256;           // compute units of the device the handle was created on
   long step = 0;
 };
 
@@ -809,6 +638,12 @@ extern "C" int mf_mlp_create(const float *params, mf_mlp **out) {
     delete hh;
     return mf::fail(MF_ERR_DEVICE, "mf_mlp_create: rounding kernel");
   }
+  {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
+      h->ncu = cus;
+  }
   *out = h;
   return MF_OK;
 }
@@ -832,7 +667,9 @@ extern "C" int mf_mlp_forward(const mf_mlp *h, const float *X, float *Y, long lo
   using namespace mf::les;
   if (!h || !X || !Y || n < 0) return mf::fail(MF_ERR_ARG, "mf_mlp_forward: invalid argument");
   if (n == 0) return MF_OK;
-  hipLaunchKernelGGL(mlp_forward_kernel, dim3((unsigned)((n + SPB - 1) / SPB)), dim3(SPB), 0,
+  // two resident blocks per CU walk the tiles; fewer samples, fewer blocks
+  const long nb = std::min<long>((n + MLP_TILE - 1) / MLP_TILE, 2L * h->ncu);
+  hipLaunchKernelGGL(mlp_forward_kernel, dim3((unsigned)nb), dim3(64 * MLP_WAVES), 0,
                      (hipStream_t)stream, X, Y, (long)n, (const unsigned short *)h->wb, (const float *)h->p);
   LESCHK(hipGetLastError());
   return MF_OK;
@@ -841,20 +678,20 @@ extern "C" int mf_mlp_forward(const mf_mlp *h, const float *X, float *Y, long lo
 namespace {
 int mlp_grad(mf_mlp *h, const float *X, const float *T, long n, hipStream_t st) {
   using namespace mf::les;
-  const long nb = (n + SPB - 1) / SPB;
+  const long nb = std::min<long>((n + MLP_TILE - 1) / MLP_TILE, 2L * h->ncu);
   if (nb > h->part_blocks) {
     if (h->part) {
       LESCHK(hipStreamSynchronize(st));
       (void)hipFree(h->part);
       h->part = nullptr;
     }
-    LESCHK(hipMalloc(&h->part, (size_t)nb * (NPARAM + 1) * sizeof(float)));
+    LESCHK(hipMalloc(&h->part, (size_t)nb * (NPARAM + 1) * sizeof(double)));
     h->part_blocks = nb;
   }
-  hipLaunchKernelGGL(mlp_grad_kernel, dim3((unsigned)nb), dim3(SPB), 0, st, X, T, n,
+  hipLaunchKernelGGL(mlp_grad_kernel, dim3((unsigned)nb), dim3(64 * MLP_WAVES), 0, st, X, T, n,
                      (const unsigned short *)h->wb, (const float *)h->p, h->part);
-  hipLaunchKernelGGL(mlp_reduce_kernel, dim3(nblk(NPARAM + 1)), dim3(256), 0, st,
-                     (const float *)h->part, (int)nb, h->g);
+  hipLaunchKernelGGL(mlp_reduce_kernel, dim3((NPARAM + 64) / 64), dim3(64 * MLP_RED), 0, st,
+                     (const double *)h->part, (int)nb, h->g);
   LESCHK(hipGetLastError());
   return MF_OK;
 }

@@ -383,6 +383,31 @@ def test_gpu_mlp_forward_and_gradient():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 15, 17, 63, 65, 64 * 512 + 1, 64 * 1100 + 47])
+def test_gpu_mlp_tile_edges(n):
+    """16-sample wave tiles, 64-sample block tiles and more tiles than resident blocks.
+    Bars: 64-term FP32 sums through two layers (64 * 2^-24 * 5 = 2e-5 of the largest)."""
+    mf, torch = _mf()
+    p = L.init_params(31)
+    p[640:704] = np.linspace(-0.2, 0.2, 64)
+    p[4800:4864] = np.linspace(0.3, -0.1, 64)
+    p[L.NPARAM - 6:] = 0.05
+    X, T = _mlp_data(n, 32)
+    net = mf.SGSNet(p)
+    Xd, Td = torch.tensor(X, device="cuda"), torch.tensor(T, device="cuda")
+    print("run mlp edges n=%d" % n, flush=True)
+    guard = torch.full((n + 8, 6), 7.0, device="cuda")
+    Y = net.forward(Xd, out=guard[:n]).cpu().numpy()
+    assert bool((guard[n:] == 7.0).all())
+    Yr = L.forward(p, X)[0]
+    assert np.abs(Y - Yr).max() < 2e-5 * np.abs(Yr).max()
+    loss, g = net.loss_grad(Xd, Td)
+    lr, gr = L.loss_and_grad(p, X, T)
+    assert abs(loss - lr) < 1e-5 * lr
+    assert np.abs(g.cpu().numpy() - gr).max() < 2e-5 * np.abs(gr).max()
+
+
+@pytest.mark.gpu
 def test_gpu_mlp_adam_matches_oracle_and_trains():
     """Three Adam steps track an FP64 restatement of Adam on the oracle's
     gradients; 300 more steps fit a smooth target."""
