@@ -1,6 +1,9 @@
 // Compact finite-difference derivatives on gfx950.
 //
-// One lane owns one grid line and runs the reference's per-line algorithm:
+// Lines of up to 512 points take the segmented solve (der_seg.h), 3-D fields
+// and batches of contiguous lines alike.  Longer ones (and contiguous lines
+// that lie more than 2^25 points apart) take the kernels of this file:
+// one lane owns one grid line and runs the reference's per-line algorithm:
 // the explicit stencil right-hand side (class_derivatives.f90:262-295) fused
 // with the forward recurrence of the packed quasi-pentadiagonal LU solve
 // (pentares, class_derivatives.f90:425-466), then the backward recurrence.
@@ -13,8 +16,10 @@
 // from L2/MALL in the backward sweep.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "der_seg.h"
@@ -276,21 +281,45 @@ __global__ void __launch_bounds__(256) der3d_kernel(FieldSet fs, int nx, int ny,
 // (full scheme), the next nb4.x .. nb4.w blocks the four families of
 // one-boundary-plane lines (sub-line scheme on points 1..n-2), and the last
 // block writes the zeros (two-boundary-plane lines, sub-line end points).
-template <int AXIS>
+template <int AXIS, bool TRI>
 __global__ void __launch_bounds__(64 * SEG_KMAX) der3d_seg_kernel(FieldSet fs, int nx, int ny,
                                                                   int nz, SegTab full,
                                                                   SegTab sub, int mode,
-                                                                  int b_full, int4 nb4) {
+                                                                  int b_full, int4 nb4,
+                                                                  int groups) {
   extern __shared__ double lds[];
-  const double *__restrict__ x = fs.x[blockIdx.y];
-  double *__restrict__ out = fs.out[blockIdx.y];
+  // The boundary-plane blocks come first: at y and z half of them read one
+  // point per cache line and take longest.  Then the full-scheme blocks, a
+  // contiguous run of them on each of the 8 XCDs that consecutive block ids go
+  // to in turn: groups of 64 lines start at any byte, so neighbours share
+  // cache lines at both ends, which then come from the XCD's own L2.
+  int blk, fld;
+  {
+    const int nf = gridDim.y, nsub = gridDim.x - b_full;
+    int bid = blockIdx.x + gridDim.x * blockIdx.y;
+    if (bid < nsub * nf) {
+      fld = bid % nf;
+      blk = b_full + bid / nf;
+    } else {
+      bid -= nsub * nf;
+      const int nb = b_full * nf, off = nsub * nf % 8;
+      // XCD of this block and its place among the XCD's full-scheme blocks
+      const int xc = (bid + off) % 8, first = (xc - off + 8) % 8, l = (bid - first) / 8;
+      int start = 0;
+      for (int q = 0; q < xc; ++q) start += (nb - (q - off + 8) % 8 + 7) / 8;
+      const int t = start + l;
+      blk = t % b_full;
+      fld = t / b_full;
+    }
+  }
+  const double *__restrict__ x = fs.x[fld];
+  double *__restrict__ out = fs.out[fld];
   int na, nb;
   long s, sa, sb;
   if (AXIS == 0) { na = ny; nb = nz; s = 1; sa = nx; sb = (long)nx * ny; }
   else if (AXIS == 1) { na = nx; nb = nz; s = nx; sa = 1; sb = (long)nx * ny; }
   else { na = nx; nb = ny; s = (long)nx * ny; sa = 1; sb = nx; }
   const int n = full.n;
-  int blk = blockIdx.x;
   SegLines L;
   L.sa = sa; L.sb = sb; L.s = s;
   // one call site of seg_solve: pick the scheme, the line family and the
@@ -298,7 +327,9 @@ __global__ void __launch_bounds__(64 * SEG_KMAX) der3d_seg_kernel(FieldSet fs, i
   SegTab T = full;
   long off = 0;
   bool solve = true;
+  L.groups = 0;
   if (blk < b_full) {
+    L.groups = groups;
     if (mode) { L.a0 = 1; L.na = na - 2; L.b0 = 1; L.nb = nb - 2; }
     else { L.a0 = 0; L.na = na; L.b0 = 0; L.nb = nb; }
   } else {
@@ -320,7 +351,7 @@ __global__ void __launch_bounds__(64 * SEG_KMAX) der3d_seg_kernel(FieldSet fs, i
   }
   if (solve) {
     L.nlines = L.na * L.nb;
-    seg_solve(x + off, out + off, T, L, blk, lds);
+    seg_solve<TRI, AXIS == 0>(x + off, out + off, T, L, blk, lds);
     return;
   }
   // zeros: the four two-boundary-plane lines and both ends of the sub lines
@@ -340,8 +371,23 @@ __global__ void __launch_bounds__(64 * SEG_KMAX) der3d_seg_kernel(FieldSet fs, i
   }
 }
 
-// batched lines: line l at x + l*ld, contiguous points (der/dder/der_s/dder_s);
-// surplus lanes walk the last line into the scratch line (as der3d_kernel)
+// batched lines on segmented line solves: line l at x + l*ld, contiguous
+// points (der/dder/der_s/dder_s)
+template <bool TRI>
+__global__ void __launch_bounds__(64 * SEG_KMAX)
+    der_lines_seg_kernel(const double *__restrict__ x, double *__restrict__ out, int nlines,
+                         long ld, SegTab T) {
+  extern __shared__ double lds[];
+  SegLines L;
+  L.sa = ld; L.sb = 0; L.s = 1;
+  L.a0 = 0; L.na = nlines; L.b0 = 0; L.nb = 1;
+  L.nlines = nlines;
+  L.groups = 0;
+  seg_solve<TRI, true>(x, out, T, L, blockIdx.x, lds);
+}
+
+// the same, one lane per line, for lines longer than the segmented solve
+// takes; surplus lanes walk the last line into the scratch line (as der3d_kernel)
 __global__ void __launch_bounds__(256) der_lines_kernel(const double *__restrict__ x,
                                                         double *__restrict__ out, int nlines,
                                                         long ld, LineTab T, int offset,
@@ -365,6 +411,8 @@ struct mf_der {
   double *dbuf = nullptr;      // device tables, then one scratch line of n
   double *scratch = nullptr;   // surplus lanes' output line
   mf::LineTab tab[2][2];       // [order-1][sub]
+  mf::SegTab seg[2][2];        // the segmented solve's tables (lines of up to 512 points)
+  bool tri[2] = {false, false};  // [order-1]: tridiagonal factors, full and sub scheme
   std::vector<double> host[2][2][2];  // [order-1][sub][0: dl_lu(n,5), 1: dr(n,7)]
 };
 
@@ -380,11 +428,12 @@ bool mf::der_host_tables(const mf_der *dc, int order, int sub, const double **dl
 
 namespace {
 // pack one scheme: dr row-major (7n) | p | f | d | e | c | 1/c, then the
-// segmented solve's tables (seg_tables): rows (SEG_ROW n) | ab (2n) | cd (2n)
-constexpr int kPackPerPoint = 13 + mf::SEG_ROW + 4;
-void pack_scheme(int n, const std::vector<double> &dl, const std::vector<double> &dr,
+// segmented solve's table (seg_tables) on lines it takes
+constexpr int kLinePack = 13;
+void pack_scheme(int n, const std::vector<double> &dl, const std::vector<double> &dr, bool tri,
                  std::vector<double> &dst) {
-  dst.assign((size_t)kPackPerPoint * n, 0.0);
+  const bool seg = mf::seg_count(n) <= mf::SEG_KMAX;
+  dst.assign((size_t)kLinePack * n + (seg ? mf::seg_table_doubles(n) : 0), 0.0);
   for (int i = 0; i < n; ++i)
     for (int m = 0; m < 7; ++m) dst[(size_t)7 * i + m] = dr[i + (size_t)n * m];
   double *p = &dst[(size_t)7 * n];
@@ -397,10 +446,17 @@ void pack_scheme(int n, const std::vector<double> &dl, const std::vector<double>
     p[5 * n + i] = 1.0 / dl[2 * (size_t)n + i];
   }
   // alpha = dl(1,1) and beta = dl(n,5) of the factored matrix
-  double *rows = p + 6 * n;
-  mf::seg_tables(n, dr.data(), p, p + n, p + 2 * n, p + 3 * n, p + 5 * n, dl[0],
-                 dl[4 * (size_t)n + n - 1], rows, rows + mf::SEG_ROW * n,
-                 rows + (mf::SEG_ROW + 2) * n);
+  if (seg)
+    mf::seg_tables(n, dr.data(), p, p + n, p + 2 * n, p + 3 * n, p + 5 * n, dl[0],
+                   dl[4 * (size_t)n + n - 1], tri, p + 6 * n);
+}
+
+// whether the factored matrix has two diagonals per sweep only: p and e zero
+// (and with them alpha = dl(1,1) and beta = dl(n,5))
+bool factors_tri(int n, const std::vector<double> &dl) {
+  for (int i = 0; i < n; ++i)
+    if (dl[i] != 0.0 || dl[4 * (size_t)n + i] != 0.0) return false;
+  return true;
 }
 #define HIPCHK(call)                                                             \
   do {                                                                           \
@@ -447,8 +503,15 @@ extern "C" int mf_der_create(const double *grid, int n, int solver_mode, int so,
         return mf::fail(MF_ERR_SETUP, "mf_der_create: singular Taylor system");
       }
       mf::pentalu(m, dl.data());
-      pack_scheme(m, dl, dr, packed[o][sub]);
     }
+  for (int o = 0; o < 2; ++o) {
+    h->tri[o] = true;
+    for (int sub = 0; sub < 1 + h->solver; ++sub)
+      h->tri[o] = h->tri[o] && factors_tri(sub ? n - 2 : n, h->host[o][sub][0]);
+    for (int sub = 0; sub < 1 + h->solver; ++sub)
+      pack_scheme(sub ? n - 2 : n, h->host[o][sub][0], h->host[o][sub][1], h->tri[o],
+                  packed[o][sub]);
+  }
   size_t total = 0;
   for (int o = 0; o < 2; ++o)
     for (int sub = 0; sub < 2; ++sub) total += packed[o][sub].size();
@@ -464,6 +527,7 @@ extern "C" int mf_der_create(const double *grid, int n, int solver_mode, int so,
       auto &pk = packed[o][sub];
       mf::LineTab &T = h->tab[o][sub];
       std::memset(&T, 0, sizeof(T));
+      h->seg[o][sub] = mf::SegTab{nullptr, 0, 0, 0};
       if (pk.empty()) continue;
       const int m = sub ? n - 2 : n;
       e = hipMemcpy(h->dbuf + off, pk.data(), pk.size() * sizeof(double), hipMemcpyHostToDevice);
@@ -483,6 +547,8 @@ extern "C" int mf_der_create(const double *grid, int n, int solver_mode, int so,
       T.alpha = h->host[o][sub][0][0];                       // dl(1,1)
       T.beta = h->host[o][sub][0][4 * (size_t)m + m - 1];    // dl(m,5) after pentalu
       T.n = m;
+      if (pk.size() > (size_t)kLinePack * m) 
+        h->seg[o][sub] = mf::SegTab{b + (size_t)kLinePack * m, m, mf::seg_count(m), mf::seg_len(m)};
       off += pk.size();
     }
   *out = h;
@@ -504,6 +570,20 @@ extern "C" int mf_der_lines(const mf_der *dc, int order, int sub, const double *
     return mf::fail(MF_ERR_ARG, "mf_der_lines: sub-line scheme needs a solver-mode handle");
   if (nlines == 0) return MF_OK;
   const mf::LineTab &T = dc->tab[order - 1][sub ? 1 : 0];
+  const mf::SegTab &S = dc->seg[order - 1][sub ? 1 : 0];
+  if (S.pack && mf::seg_fits(ld)) {
+    const dim3 grid((nlines + 63) / 64), block(64 * mf::seg_count(S.n));
+    const size_t lds = mf::seg_lds_doubles(S.n, true) * sizeof(double);
+    const int o = sub ? 1 : 0;
+    if (dc->tri[order - 1])
+      hipLaunchKernelGGL(mf::der_lines_seg_kernel<true>, grid, block, lds, (hipStream_t)stream,
+                         x + o, out + o, nlines, (long)ld, S);
+    else
+      hipLaunchKernelGGL(mf::der_lines_seg_kernel<false>, grid, block, lds, (hipStream_t)stream,
+                         x + o, out + o, nlines, (long)ld, S);
+    HIPCHK(hipGetLastError());
+    return MF_OK;
+  }
   const int blocks = (nlines + 255) / 256;
   hipLaunchKernelGGL(mf::der_lines_kernel, dim3(blocks), dim3(256), 13 * T.n * sizeof(double),
                      (hipStream_t)stream, x, out, nlines, (long)ld, T, sub ? 1 : 0, dc->scratch);
@@ -543,35 +623,35 @@ extern "C" int mf_der3d_batch(const mf_der *dc, int axis, int order, int nfields
     blocks = b_full + b_sub + 1;
   }
   hipStream_t st = (hipStream_t)stream;
-  if (mf::seg_count(F.n) <= mf::SEG_KMAX) {
-    // segmented solves: 64 lines per block, one wavefront per segment; the
-    // row tables follow the packed 1/c
-    auto seg_of = [](const mf::LineTab &t) {
-      if (!t.rc) return mf::SegTab{nullptr, nullptr, nullptr, 0.0, 0.0, 0};
-      const double *rows = t.rc + t.n;
-      return mf::SegTab{rows, rows + mf::SEG_ROW * t.n, rows + (mf::SEG_ROW + 2) * t.n,
-                        t.alpha, t.beta, t.n};
-    };
-    const mf::SegTab SF = seg_of(F), SS = seg_of(S);
+  const mf::SegTab &SF = dc->seg[order - 1][0], &SS = dc->seg[order - 1][1];
+  if (SF.pack && (axis != 0 || mf::seg_fits((long)nx * ny))) {
+    // segmented solves: 64 lines per block, one wavefront per segment
     int4 nb4 = make_int4(0, 0, 0, 0);
     int sb_full, sblocks;
+    const int groups = axis != 0 && mf::seg_aligned(nx) ? (nx + 63) / 64 : 0;
     if (!mode) {
-      sb_full = (int)(((long)na * nb + 63) / 64);
+      sb_full = groups ? groups * nb : (int)(((long)na * nb + 63) / 64);
       sblocks = sb_full;
     } else {
-      sb_full = (int)(((long)(na - 2) * (nb - 2) + 63) / 64);
+      sb_full = groups ? groups * (nb - 2) : (int)(((long)(na - 2) * (nb - 2) + 63) / 64);
       nb4.x = nb4.y = (na - 2 + 63) / 64;
       nb4.z = nb4.w = (nb - 2 + 63) / 64;
       sblocks = sb_full + nb4.x + nb4.y + nb4.z + nb4.w + 1;
     }
-    const size_t lds = mf::seg_lds_doubles(F.n) * sizeof(double);
+    const size_t lds = mf::seg_lds_doubles(F.n, axis == 0) * sizeof(double);
     const dim3 grid(sblocks, nfields), block(64 * mf::seg_count(F.n));
-    if (axis == 0)
-      hipLaunchKernelGGL(mf::der3d_seg_kernel<0>, grid, block, lds, st, fs, nx, ny, nz, SF, SS, mode, sb_full, nb4);
-    else if (axis == 1)
-      hipLaunchKernelGGL(mf::der3d_seg_kernel<1>, grid, block, lds, st, fs, nx, ny, nz, SF, SS, mode, sb_full, nb4);
-    else
-      hipLaunchKernelGGL(mf::der3d_seg_kernel<2>, grid, block, lds, st, fs, nx, ny, nz, SF, SS, mode, sb_full, nb4);
+    auto go = [&](auto ax, auto tri) {
+      hipLaunchKernelGGL((mf::der3d_seg_kernel<decltype(ax)::value, decltype(tri)::value>), grid,
+                         block, lds, st, fs, nx, ny, nz, SF, SS, mode, sb_full, nb4,
+                         groups);
+    };
+    auto pick = [&](auto ax) {
+      if (dc->tri[order - 1]) go(ax, std::true_type());
+      else go(ax, std::false_type());
+    };
+    if (axis == 0) pick(std::integral_constant<int, 0>());
+    else if (axis == 1) pick(std::integral_constant<int, 1>());
+    else pick(std::integral_constant<int, 2>());
     HIPCHK(hipGetLastError());
     return MF_OK;
   }

@@ -10,56 +10,102 @@
 // zero and A, B its homogeneous responses to unit incoming values, which
 // depend on the coefficients only and are tabulated at set-up (likewise
 // x_i = Q_i + C_i x_e + D_i x_{e+1} backward).  Each wave loads its
-// segment's inputs at once, runs P in registers, publishes its two boundary
-// values in LDS, chains the 2x2 maps of the segments before it to get its
-// incoming values, and fixes P up; then the same backward.  The result is the
-// sequential solve re-associated (rounding-level differences only), with K
-// times the wavefronts of one-lane-per-line and every load of a segment in
-// flight together.
+// segment's inputs at once, runs P in registers, publishes its boundary
+// values in LDS, chains the maps of the segments before it to get its
+// incoming values, and corrects P inside the backward sweep; then the same
+// backward, corrected as it is stored.  The result is the sequential solve
+// re-associated (rounding-level differences only), with K times the
+// wavefronts of one-lane-per-line and every load of a segment in flight
+// together.
 //
-// The coefficients are wave-uniform: they are read through the constant
-// address space, so they arrive by scalar loads into SGPRs (one 16-double
-// row per point) and cost neither LDS bandwidth nor vector registers.
+// What bounds it: HBM (16 B per point) when the chip is full, the chain of
+// the wave's own latencies when it is not.  The coefficients are the same for
+// every lane; they sit in the wave's vector registers, one per lane (a
+// segment's 14 x 32 doubles are 7 register pairs, loaded once, coalesced),
+// and reach the FMAs through v_readlane, which has no latency to wait for:
+// 28 lane reads and 15 FP64 operations per row.  (Scalar loads, four rows per wait on a
+// 24 KB table that the 16 KB scalar cache does not hold, kept a wave waiting.)
+// Where the factored matrix is tridiagonal (p = e = 0: the schemes of order 6
+// and below) a second instance drops p, e, A, D and one of the two exchanged
+// values: 20 lane reads and 11 operations.
+// Measured, before (scalar loads, contiguous lines read and written lane by
+// lane, blocks in launch order) and now: one derivative along x / y / z of
+// 201 x 256 x 187, in cache, 80 / 75 / 88 -> 45 / 49 / 43 us (154 MB; a copy
+// takes 31), all three from HBM 256 -> 186 us; six fields of 192 x 256 x 192
+// 400 / 413 / 404 -> 205 / 238 / 255 us (4.4-3.6 TB/s); 64^3 16 -> 12 us;
+// 49 152 contiguous lines of 192 points, one lane per line before, 130 -> 30 us.
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <type_traits>
+#include <vector>
+
 namespace mf {
 
-constexpr int SEG_LEN = 32;   // segment length (all segments but the last)
-constexpr int SEG_MAX = 38;   // longest last segment (it absorbs a short tail)
-constexpr int SEG_KMAX = 16;  // segments per line (wavefronts per block)
-constexpr int SEG_ROW = 16;   // coefficient doubles per point
+constexpr int SEG_LEN = 32;     // longest segment
+// Whether the lines along y or z of a field of nx columns go in groups of 64
+// aligned in memory: rows of whole cache lines (16 points), and few lanes lost
+// at the rows' ends.
+inline bool seg_aligned(int nx) { return nx % 16 == 0 && 16 * ((nx + 63) / 64 * 64 - nx) <= 2 * nx; }
 
-// Segmentation of a line of n points: K segments starting at 32 j, the last
-// running to n and at least 7 rows long (so that it holds the 7-point closure
-// inputs and row n-4).
-__host__ __device__ inline int seg_count(int n) {
-  int K = (n + SEG_LEN - 1) / SEG_LEN;
-  if (K > 1 && n - SEG_LEN * (K - 1) < 7) --K;
-  return K;
+// Contiguous lines: the wave shuffles 32-bit line offsets, so 64 lines that lie
+// `stride` points apart have to stay within 2^31 points.
+inline bool seg_fits(long stride) { return stride <= 0x7fffffffL / 64; }
+
+constexpr int SEG_KMAX = 16;    // segments per line (wavefronts per block)
+constexpr int SEG_PACK = 512;   // coefficient doubles per segment
+constexpr int SEG_CHAIN = 64;   // doubles per chain table (4 per segment)
+
+// Segmentation of a line of n points: K segments of seg_len(n) rows, the last
+// one the rest (for 33 <= n <= 512 at least 11 rows: it holds the 7-point
+// closure's inputs and row n-4).  Even segments, since a block takes as long
+// as its longest.
+__host__ __device__ inline int seg_count(int n) { return (n + SEG_LEN - 1) / SEG_LEN; }
+__host__ __device__ inline int seg_len(int n) { return (n + seg_count(n) - 1) / seg_count(n); }
+
+// LDS doubles per wave: the forward and backward exchange arrays, 2 x 64
+// each; on contiguous lines the wave's 64 x 16 transpose tile, whose start
+// doubles as the forward exchange (the tile is idle between the loads and the
+// last barrier), and the backward exchange
+constexpr int SEG_TP = 17;  // pitch of the transpose tile
+__host__ __device__ constexpr int seg_wave_doubles(bool xt) { return xt ? 64 * SEG_TP + 128 : 256; }
+// dynamic LDS doubles of a block running a scheme of n points
+__host__ __device__ inline int seg_lds_doubles(int n, bool xt) {
+  return seg_wave_doubles(xt) * seg_count(n);
 }
+// doubles of a scheme's table: the segments' packs, then the two chain tables
+inline size_t seg_table_doubles(int n) { return (size_t)SEG_PACK * seg_count(n) + 2 * SEG_CHAIN; }
 
-// dynamic LDS doubles of a block running a scheme of n points: the forward
-// and backward exchange arrays, [K][2][64] each
-__host__ __device__ inline int seg_lds_doubles(int n) { return 4 * 64 * seg_count(n); }
-
-// Row layout of the segment table (SEG_ROW doubles per point i, two 64-byte
-// halves: the forward sweep of an interior row reads the first, the backward
-// sweep the second):
-//   0..4 dr(i, 0..4) | 5 p | 6 f | 7 dr(i, 5) || 8 dr(i, 6) | 9 e | 10 d | 11 1/c | 12..15 0
-// The homogeneous responses sit in two arrays of their own, (A_i, B_i) and
-// (C_i, D_i) pairs: the compiler merges adjacent scalar loads, and a fix-up
-// coefficient merged into a load of the other sweep would be held in SGPRs
-// from one sweep to the next.
-enum { SR_P = 5, SR_F = 6, SR_E = 9, SR_D = 10, SR_RC = 11 };
-__host__ __device__ constexpr int sr_dr(int m) { return m < 5 ? m : m + 2; }
+// The right-hand side sum_m dr_m f_m of an interior row is formed on the
+// differences of its window,
+//   s f_2 + sum_j t_j (f_{j+1} - f_j),
+//   s = sum_m dr_m,  t_j = sum_{m > j} dr_m (j >= 2),  -sum_{m <= j} dr_m (j < 2),
+// the same sum (s is the rounding residue of a derivative's weights) without
+// the cancellation of the f_m themselves, for one subtraction per row.  The
+// 7-point rows at the ends, whose rounding the closure's small pivots
+// amplify, keep their weights as they are.
+//
+// A segment's pack, row k of the segment at seg_cw(tri) k:
+//   s, t(0..3) | dr(0..4), p, f, e, d, 1/c, A, B, C, D      (14 per row)
+//   s, t(0..3) | dr(0..4), f, d, 1/c, B, C                  (10 per row, tridiagonal)
+// and, from 496, what the line's ends need: dr(5..6) of rows 0 and 1, of
+// rows n-2 and n-1, alpha, beta.
+template <bool TRI>
+struct SegSlot {
+  static constexpr int P = 5, F = TRI ? 5 : 6, E = 7, D = TRI ? 6 : 8, RC = TRI ? 7 : 9,
+                       HA = 10, HB = TRI ? 8 : 11, HC = TRI ? 9 : 12, HD = 13;
+};
+__host__ __device__ constexpr int seg_cw(bool tri) { return tri ? 10 : 14; }
+constexpr int SEG_XHEAD = 496, SEG_XTAIL = 500, SEG_XALPHA = 504, SEG_XBETA = 505;
+static_assert(SEG_LEN * 14 <= SEG_XHEAD, "a segment's rows fit the pack");
+static_assert(4 * SEG_KMAX <= SEG_CHAIN, "the chain tables fit one register pair");
+// Chain tables, 4 doubles per segment j: forward A, B of its last row but one
+// and of its last row; backward C, D of its first and second row.
 
 struct SegTab {
-  const double *rows;  // n x SEG_ROW
-  const double *ab;    // n x 2: A, B
-  const double *cd;    // n x 2: C, D
-  double alpha, beta;
-  int n;
+  const double *pack;  // K x SEG_PACK, then the chain tables
+  int n, K, len;       // points, segments, segment length
 };
 
 struct SegLines {
@@ -68,167 +114,285 @@ struct SegLines {
   long sa, sb, s;
   int a0, na, b0, nb;
   int nlines;
+  // not 0: groups of 64 lines at a = 64 g .. 64 g + 63, this many for each b
+  // (lines outside a0 .. a0 + na - 1 are left out); 0: 64 lines in turn
+  int groups;
 };
 
-typedef const __attribute__((address_space(4))) double *seg_cptr;
+// lane `lane` (uniform) of v, in scalar registers
+__device__ __forceinline__ double seg_lane(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, lane);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// the wave's own LDS tile: its writes before its reads (no other wave uses it)
+__device__ __forceinline__ void seg_tile_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // One wavefront's segment [s0, s0 + len).  LEN rows are unrolled; DYN: the
 // length is the runtime len <= LEN (rows beyond it are skipped), else len =
 // LEN.  HEAD: segment 0 (7-point rows 0 and 1, the alpha term of row 0);
 // TAIL: the last segment (7-point rows n-2 and n-1, the beta term of row n-1).
-// Ef, Eb: the block's exchange arrays; w, K: this segment and the count.
-template <int LEN, bool HEAD, bool TAIL, bool DYN>
-__device__ __forceinline__ void seg_wave(const double *__restrict__ xl, double *__restrict__ ol,
-                                         long s, bool act, const SegTab &T, int w, int K,
-                                         int s0, int len, double *Ef, double *Eb) {
+// x0, out0: the block's first line; rel: this lane's line from there; lo, hi:
+// lanes lo .. hi - 1 have a line of their own (the others repeat one and
+// store nothing).  lds: the block's arrays; w, K: this segment
+// and the count.
+// XT: contiguous lines (s = 1).  A lane's line then lies in memory away from
+// the next lane's, so the wave moves 16 rows x 64 lines at a time through
+// its transpose tile: each load and store covers 128 contiguous bytes of four
+// lines (stored lane by lane, 8 bytes per line and instruction, HBM wrote
+// 1.56 x the field, and x took 85 us where y and z took 54-58 at
+// 201 x 256 x 187).
+template <int LEN, bool HEAD, bool TAIL, bool DYN, bool TRI, bool XT>
+__device__ __forceinline__ void seg_wave(const double *__restrict__ x0, double *__restrict__ out0,
+                                         long rel, int lo, int hi, long s, const SegTab &T, int w, int K,
+                                         int s0, int len, double *lds) {
   const int n = T.n;
   const int lane = threadIdx.x & 63;
-  // row s0 + k sits at a compile-time offset from Rs (scalar-load immediates)
-  const seg_cptr Rs = (seg_cptr)T.rows + (long)s0 * SEG_ROW;
-  const seg_cptr AB = (seg_cptr)T.ab, CD = (seg_cptr)T.cd;
-  const seg_cptr ABs = AB + 2L * s0, CDs = CD + 2L * s0;
+  typedef SegSlot<TRI> Slot;
+  constexpr int CW = seg_cw(TRI);
+  constexpr int NC = (LEN * CW + 63) / 64;  // register pairs of the rows
+  constexpr int WD = seg_wave_doubles(XT), WB = XT ? 64 * SEG_TP : 128;
+  const double *xl = x0 + rel;
+  // exchange slots of wave j: forward Ef[j WD ..], backward Eb[j WD ..]
+  double *Ef = lds + lane, *Eb = lds + WB + lane;
+  double *tile = lds + (long)WD * w;
+  // XT: this lane's place in a coalesced access, row tr of line 4 q + tl
+  const int tr = lane & 15, tl = lane >> 4;
   auto on = [&](int k) { return !DYN || k < len; };
   // tail rows: k = len - 2 (row n-2) and k = len - 1 (row n-1)
   auto is_n2 = [&](int k) { return TAIL && (DYN ? k == len - 2 : k == LEN - 2); };
   auto is_n1 = [&](int k) { return TAIL && (DYN ? k == len - 1 : k == LEN - 1); };
+  double cv[NC], cx = 0.0, cf = 0.0, cb = 0.0;
+  auto load_rows = [&]() {
+    const double *pk = T.pack + (long)SEG_PACK * w + lane;
+#pragma unroll
+    for (int j = 0; j < NC; ++j) cv[j] = pk[64 * j];
+    if (HEAD || TAIL) cx = pk[SEG_PACK - 64];
+  };
+  if (!XT) load_rows();
+  const double *ch = T.pack + (long)SEG_PACK * K + lane;  // loaded once V's registers free up
+  auto C = [&](int k, int m) { return seg_lane(cv[(k * CW + m) / 64], (k * CW + m) % 64); };
+  auto X = [&](int m) { return seg_lane(cx, m - (SEG_PACK - 64)); };
   // inputs V[k] = x[s0 - 2 + k]; the two before the line (segment 0) and the
   // two after it (last segment of exactly LEN rows) are never read; a
   // runtime-length segment clamps into the line
   double V[LEN + 4];
+  constexpr int NR = LEN / 16;  // 16-row tiles
+  if constexpr (XT) {
+    double R[NR][16];
 #pragma unroll
-  for (int k = 0; k < LEN + 4; ++k) {
-    if ((HEAD && k < 2) || (TAIL && !DYN && k >= LEN + 2)) {
-      V[k] = 0.0;
-      continue;
+    for (int t = 0; t < NR; ++t)
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        int r = s0 + 16 * t + tr;
+        if (DYN) r = r > n - 1 ? n - 1 : r;
+        R[t][q] = x0[__shfl((int)rel, 4 * q + tl, 64) + r];
+      }
+    // the rows next to the segment (the rows of a DYN segment's tile that lie
+    // beyond its len are its successor's: nothing more to fetch)
+    V[0] = HEAD ? 0.0 : xl[s0 - 2];
+    V[1] = HEAD ? 0.0 : xl[s0 - 1];
+    V[LEN + 2] = TAIL ? 0.0 : xl[s0 + LEN > n - 1 ? n - 1 : s0 + LEN];
+    V[LEN + 3] = TAIL ? 0.0 : xl[s0 + LEN + 1 > n - 1 ? n - 1 : s0 + LEN + 1];
+#pragma unroll
+    for (int t = 0; t < NR; ++t) {
+#pragma unroll
+      for (int q = 0; q < 16; ++q) tile[(4 * q + tl) * SEG_TP + tr] = R[t][q];
+      seg_tile_sync();
+#pragma unroll
+      for (int r = 0; r < 16; ++r) V[2 + 16 * t + r] = tile[lane * SEG_TP + r];
+      seg_tile_sync();
+      if (t == 0) load_rows();
+      __builtin_amdgcn_sched_barrier(0);
     }
-    int q = s0 - 2 + k;
-    if (DYN) q = q > n - 1 ? n - 1 : q;
-    V[k] = xl[(long)q * s];
+  } else {
+#pragma unroll
+    for (int k = 0; k < LEN + 4; ++k) {
+      if ((HEAD && k < 2) || (TAIL && !DYN && k >= LEN + 2)) {
+        V[k] = 0.0;
+        continue;
+      }
+      int q = s0 - 2 + k;
+      if (DYN) q = q > n - 1 ? n - 1 : q;
+      V[k] = xl[(long)q * s];
+    }
   }
   // forward particular solution from zero incoming values (segment 0 starts
-  // at the true start)
+  // at the true start); df[j]: the differences of the row's window
   double Y[LEN];
   double ym1 = 0.0, ym2 = 0.0, ym3 = 0.0, yl0 = 0.0, yl1 = 0.0;
+  double df[4] = {0.0, V[1] - V[0], V[2] - V[1], V[3] - V[2]};
+  // a 7-point row on x[0..6] = V[v0..v0+6]; its last two weights at X(m)
+  auto row7 = [&](int k, int v0, int m) {
+    double r = C(k, 0) * V[v0];
+#pragma unroll
+    for (int j = 1; j < 7; ++j) r = fma(j < 5 ? C(k, j) : X(m + j - 5), V[v0 + j], r);
+    return r;
+  };
 #pragma unroll
   for (int k = 0; k < LEN; ++k) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) df[j] = df[j + 1];
+    df[3] = V[k + 4] - V[k + 3];
     if (on(k)) {
-      const seg_cptr c = Rs + k * SEG_ROW;
-      double rr = 0.0, yi;
-      if (HEAD && k < 2) {  // 7-point head rows on x[0..6] = V[2..8]
-#pragma unroll
-        for (int m = 0; m < 7; ++m) rr = fma(c[sr_dr(m)], V[2 + m], rr);
-        yi = (k == 0) ? rr : rr - c[SR_F] * ym1;
-      } else if (k >= 4 && (is_n2(k) || is_n1(k))) {
-        // 7-point tail rows on x[n-7..n-1] = V[k-3..k+3] (row n-2) or V[k-4..k+2] (row n-1)
-        if (is_n2(k)) {
-#pragma unroll
-          for (int m = 0; m < 7; ++m) rr = fma(c[sr_dr(m)], V[k - 3 + m], rr);
-        } else {
-#pragma unroll
-          for (int m = 0; m < 7; ++m) rr = fma(c[sr_dr(m)], V[k - 4 + m], rr);
-        }
-        yi = rr - c[SR_P] * ym2 - c[SR_F] * ym1;
-        if (is_n1(k)) yi -= T.beta * ym3;
+      double yi;
+      // the row's window: V[k..k+4] inside, x[0..6] on the 7-point rows 0 and 1,
+      // x[n-7..n-1] on rows n-2 (V[k-3..k+3]) and n-1 (V[k-4..k+2])
+      if (HEAD && k < 2) {
+        yi = row7(k, 2, SEG_XHEAD + 2 * k);
+      } else if (k >= 4 && is_n2(k)) {
+        yi = row7(k, k >= 4 ? k - 3 : 0, SEG_XTAIL);
+      } else if (k >= 4 && is_n1(k)) {
+        yi = row7(k, k >= 4 ? k - 4 : 0, SEG_XTAIL + 2);
       } else {
-        rr = c[0] * V[k] + c[1] * V[k + 1] + c[2] * V[k + 2] + c[3] * V[k + 3] + c[4] * V[k + 4];
-        yi = rr - c[SR_P] * ym2 - c[SR_F] * ym1;
+        yi = C(k, 0) * V[k + 2];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) yi = fma(C(k, 1 + j), df[j], yi);
       }
+      // what the sweep waits for comes last
+      if (!TRI && is_n1(k)) yi = fma(-X(SEG_XBETA), ym3, yi);
+      if (!TRI && !(HEAD && k < 2)) yi = fma(-C(k, Slot::P), ym2, yi);
+      if (!(HEAD && k == 0)) yi = fma(-C(k, Slot::F), ym1, yi);
       Y[k] = yi;
       ym3 = ym2; ym2 = ym1; ym1 = yi;
       if (DYN ? k == len - 2 : k == LEN - 2) yl0 = yi;
       if (DYN ? k == len - 1 : k == LEN - 1) yl1 = yi;
     }
-    // keep the scalar coefficient loads near their rows (hoisting them all
-    // to the top exhausts the SGPRs)
-    if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    if (k == LEN / 2 && !HEAD) cf = ch[0];
+    if (k == LEN / 2 && !TAIL) cb = ch[SEG_CHAIN];
+    // keep the lane reads near their rows (hoisting them exhausts the SGPRs)
+    if (k % 2 == 1) __builtin_amdgcn_sched_barrier(0);
   }
-  // publish the segment's last two particular values
-  Ef[(w * 2 + 0) * 64 + lane] = yl0;
-  Ef[(w * 2 + 1) * 64 + lane] = yl1;
+  // publish the segment's last particular values
+  if (!TRI) Ef[w * WD] = yl0;
+  Ef[w * WD + 64] = yl1;
   __syncthreads();
+  double v0 = 0.0, v1 = 0.0;
   if (!HEAD) {
     // incoming (y_{s0-2}, y_{s0-1}): segment 0 ends on its own values, later
     // segments map theirs through their homogeneous responses
-    double v0 = Ef[lane], v1 = Ef[64 + lane];
+    if (!TRI) v0 = Ef[0];
+    v1 = Ef[64];
     for (int j = 1; j < w; ++j) {
-      const seg_cptr c = AB + 2L * (SEG_LEN * (j + 1) - 2);  // rows e_j-2, e_j-1
-      const double p0 = Ef[(j * 2 + 0) * 64 + lane], p1 = Ef[(j * 2 + 1) * 64 + lane];
-      const double n0 = p0 + c[0] * v0 + c[1] * v1;
-      const double n1 = p1 + c[2] * v0 + c[3] * v1;
-      v0 = n0; v1 = n1;
-    }
-#pragma unroll
-    for (int k = 0; k < LEN; ++k) {
-      const seg_cptr c = ABs + 2 * k;
-      if (on(k)) Y[k] = Y[k] + c[0] * v0 + c[1] * v1;
-      if (k % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+      const double p1 = Ef[j * WD + 64];
+      if (TRI) {
+        v1 = fma(seg_lane(cf, 4 * j + 3), v1, p1);
+      } else {
+        const double p0 = Ef[j * WD];
+        const double n0 = fma(seg_lane(cf, 4 * j + 1), v1, fma(seg_lane(cf, 4 * j + 0), v0, p0));
+        v1 = fma(seg_lane(cf, 4 * j + 3), v1, fma(seg_lane(cf, 4 * j + 2), v0, p1));
+        v0 = n0;
+      }
     }
   }
   // backward particular solution from zero incoming values (the last segment
-  // ends at the true end), in place in Y
-  double xp1 = 0.0, xp2 = 0.0, x1 = 0.0, x2 = 0.0, x3 = 0.0;
+  // ends at the true end), in place in Y, on the corrected forward values
+  double xp1 = 0.0, xp2 = 0.0, x3 = 0.0;
 #pragma unroll
   for (int k = LEN - 1; k >= 0; --k) {
     if (on(k)) {
-      const seg_cptr c = Rs + k * SEG_ROW;
-      double xi;
-      if (is_n1(k)) {
-        xi = Y[k] * c[SR_RC];
-      } else if (HEAD && k == 0) {
-        xi = (Y[0] - c[SR_E] * x2 - c[SR_D] * x1 - T.alpha * x3) * c[SR_RC];
-      } else {
-        xi = (Y[k] - c[SR_E] * xp2 - c[SR_D] * xp1) * c[SR_RC];
+      double xi = Y[k];
+      if (!HEAD) {
+        if (!TRI) xi = fma(C(k, Slot::HA), v0, xi);
+        xi = fma(C(k, Slot::HB), v1, xi);
       }
+      if (!is_n1(k)) {
+        if (HEAD && k == 0 && !TRI) xi = fma(-X(SEG_XALPHA), x3, xi);
+        if (!TRI) xi = fma(-C(k, Slot::E), xp2, xi);
+        xi = fma(-C(k, Slot::D), xp1, xi);
+      }
+      xi *= C(k, Slot::RC);
       Y[k] = xi;
       xp2 = xp1; xp1 = xi;
       if (HEAD && k == 3) x3 = xi;
-      if (HEAD && k == 2) x2 = xi;
-      if (HEAD && k == 1) x1 = xi;
     }
-    if (k % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+    if (k % 2 == 0) __builtin_amdgcn_sched_barrier(0);
   }
-  Eb[(w * 2 + 0) * 64 + lane] = Y[0];
-  Eb[(w * 2 + 1) * 64 + lane] = Y[1];
+  Eb[w * WD] = Y[0];
+  if (!TRI) Eb[w * WD + 64] = Y[1];
   __syncthreads();
+  v0 = v1 = 0.0;
   if (!TAIL) {
     // incoming (x_{e0}, x_{e0+1}) from the segments after this one
-    double v0 = Eb[((K - 1) * 2 + 0) * 64 + lane], v1 = Eb[((K - 1) * 2 + 1) * 64 + lane];
+    v0 = Eb[(K - 1) * WD];
+    if (!TRI) v1 = Eb[(K - 1) * WD + 64];
     for (int j = K - 2; j > w; --j) {
-      const seg_cptr c = CD + 2L * SEG_LEN * j;  // rows s_j, s_j+1
-      const double q0 = Eb[(j * 2 + 0) * 64 + lane], q1 = Eb[(j * 2 + 1) * 64 + lane];
-      const double n0 = q0 + c[0] * v0 + c[1] * v1;
-      const double n1 = q1 + c[2] * v0 + c[3] * v1;
-      v0 = n0; v1 = n1;
-    }
-#pragma unroll
-    for (int k = 0; k < LEN; ++k) {
-      const seg_cptr c = CDs + 2 * k;
-      if (on(k)) Y[k] = Y[k] + c[0] * v0 + c[1] * v1;
-      if (k % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+      const double q0 = Eb[j * WD];
+      if (TRI) {
+        v0 = fma(seg_lane(cb, 4 * j + 0), v0, q0);
+      } else {
+        const double q1 = Eb[j * WD + 64];
+        const double n0 = fma(seg_lane(cb, 4 * j + 1), v1, fma(seg_lane(cb, 4 * j + 0), v0, q0));
+        v1 = fma(seg_lane(cb, 4 * j + 3), v1, fma(seg_lane(cb, 4 * j + 2), v0, q1));
+        v0 = n0;
+      }
     }
   }
-  if (act) {
+  auto fixed = [&](int k) {
+    double xi = Y[k];
+    if (!TAIL) {
+      xi = fma(C(k, Slot::HC), v0, xi);
+      if (!TRI) xi = fma(C(k, Slot::HD), v1, xi);
+    }
+    return xi;
+  };
+  if constexpr (XT) {
+    int relo = (int)rel;  // opaque: the offsets are formed here, not kept from the loads
+    asm volatile("" : "+v"(relo));
+#pragma unroll
+    for (int t = 0; t < NR; ++t) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        if (on(16 * t + r)) tile[lane * SEG_TP + r] = fixed(16 * t + r);
+        if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+      seg_tile_sync();
+      const bool rok = 16 * t + tr < (DYN ? len : LEN);
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        const int l = 4 * q + tl;
+        const int o = __shfl(relo, l, 64) + s0 + 16 * t + tr;
+        const double v = tile[l * SEG_TP + tr];
+        if (rok && l < hi) out0[o] = v;
+        if (q % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+      seg_tile_sync();
+    }
+  } else {
     // a fresh copy of the stride, opaque to the compiler, so that the store
     // offsets are computed here rather than shared with the load offsets and
     // held in SGPRs through the whole segment
     long so = s;
     asm volatile("" : "+s"(so));
-    double *po = ol + (long)s0 * so;
+    double *po = out0 + rel + (long)s0 * so;
+    const bool act = lane >= lo && lane < hi;
 #pragma unroll
-    for (int k = 0; k < LEN; ++k)
-      if (on(k)) po[(long)k * so] = Y[k];
+    for (int k = 0; k < LEN; ++k) {
+      if (on(k)) {
+        const double xi = fixed(k);
+        if (act) po[(long)k * so] = xi;
+      }
+      if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
   }
 }
 
 // Solve the scheme on 64 lines per block, wave w = segment w.
 // x, out: the field and result; lines per SegLines (one family of lines).
-// lds: forward exchange [K][2][64] | backward [K][2][64].
+// lds: seg_lds_doubles(n, XT) (of the longest scheme of the launch).
 // Every wave of the block passes the same two barriers.
+template <bool TRI, bool XT>
 __device__ __forceinline__ void seg_solve(const double *__restrict__ x, double *__restrict__ out,
                                           const SegTab &T, const SegLines &L, int lblock,
                                           double *lds) {
   const int n = T.n;
-  const int K = seg_count(n);
+  const int K = T.K;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (w >= K) {
     // waves beyond K (blocks sized for a longer scheme) only join the barriers
@@ -236,81 +400,121 @@ __device__ __forceinline__ void seg_solve(const double *__restrict__ x, double *
     __syncthreads();
     return;
   }
-  double *Ef = lds;
-  double *Eb = Ef + 128 * K;
-  // this lane's line
-  int l = lblock * 64 + (int)(threadIdx.x & 63);
-  const bool act = l < L.nlines;
-  l = act ? l : L.nlines - 1;
-  const long base = (long)(L.a0 + l % L.na) * L.sa + (long)(L.b0 + l / L.na) * L.sb;
-  const double *xl = x + base;
-  double *ol = out + base;
-  const int s0 = SEG_LEN * w;
-  const int len = (w == K - 1) ? n - s0 : SEG_LEN;
-  if (K == 1)
-    seg_wave<SEG_MAX, true, true, true>(xl, ol, L.s, act, T, w, K, s0, len, Ef, Eb);
-  else if (w == 0)
-    seg_wave<SEG_LEN, true, false, false>(xl, ol, L.s, act, T, w, K, s0, len, Ef, Eb);
-  else if (w < K - 1)
-    seg_wave<SEG_LEN, false, false, false>(xl, ol, L.s, act, T, w, K, s0, len, Ef, Eb);
-  else if (len == SEG_LEN)
-    seg_wave<SEG_LEN, false, true, false>(xl, ol, L.s, act, T, w, K, s0, len, Ef, Eb);
-  else
-    seg_wave<SEG_MAX, false, true, true>(xl, ol, L.s, act, T, w, K, s0, len, Ef, Eb);
+  // the block's first line, and this lane's from there
+  const int lane = threadIdx.x & 63;
+  int lo = 0, hi;
+  long base, rel;
+  if (!XT && L.groups) {
+    const int ag = 64 * (lblock % L.groups), b = lblock / L.groups;
+    lo = max(0, L.a0 - ag);
+    hi = min(64, L.a0 + L.na - ag);
+    base = (long)ag * L.sa + (long)(L.b0 + b) * L.sb;
+    rel = min(max(lane, lo), hi - 1) * L.sa;
+  } else {
+    const int l0 = lblock * 64;
+    hi = min(64, L.nlines - l0);
+    const int l = l0 + min(lane, hi - 1);
+    const int a0 = l0 % L.na, b0 = l0 / L.na;
+    base = (long)(L.a0 + a0) * L.sa + (long)(L.b0 + b0) * L.sb;
+    rel = (long)(l % L.na - a0) * L.sa + (long)(l / L.na - b0) * L.sb;
+  }
+  const double *x0 = x + base;
+  double *o0 = out + base;
+  const int s0 = T.len * w;
+  const int len = (w == K - 1) ? n - s0 : T.len;
+  auto go = [&](auto head, auto tail, auto dyn) {
+    seg_wave<SEG_LEN, decltype(head)::value, decltype(tail)::value, decltype(dyn)::value, TRI, XT>(
+        x0, o0, rel, lo, hi, L.s, T, w, K, s0, len, lds);
+  };
+  typedef std::true_type yes;
+  typedef std::false_type no;
+  if (K == 1) {
+    go(yes(), yes(), yes());
+  } else if (len == SEG_LEN) {
+    if (w == 0) go(yes(), no(), no());
+    else if (w < K - 1) go(no(), no(), no());
+    else go(no(), yes(), no());
+  } else {
+    if (w == 0) go(yes(), no(), yes());
+    else if (w < K - 1) go(no(), no(), yes());
+    else go(no(), yes(), yes());
+  }
 }
 
-// Segment tables of a scheme of n points (host side) from its dr (n,7)
-// column-major and packed p, f, d, e, 1/c: rows[i*SEG_ROW + ...] as SR_*, and
-// the homogeneous responses ab = (A_i, B_i) (forward, zero on segment 0) and
-// cd = (C_i, D_i) (backward, zero on the last segment).
+// Table of a scheme of n points (host side) from its dr (n,7) column-major
+// and packed p, f, d, e, 1/c: the segments' packs and the chain tables, formed
+// in extended precision and rounded once.  The homogeneous responses are zero
+// on segment 0 (forward) and on the last one (backward).
 inline void seg_tables(int n, const double *dr, const double *p, const double *f,
                        const double *d, const double *e, const double *rc, double alpha,
-                       double beta, double *rows, double *ab, double *cd) {
-  const int K = seg_count(n);
-  for (int i = 0; i < n; ++i) {
-    double *r = rows + (size_t)i * SEG_ROW;
-    for (int m = 0; m < 7; ++m) r[sr_dr(m)] = dr[i + (size_t)n * m];
-    r[SR_P] = p[i];
-    r[SR_F] = f[i];
-    r[SR_E] = e[i];
-    r[SR_D] = d[i];
-    r[SR_RC] = rc[i];
-    for (int m = 12; m < SEG_ROW; ++m) r[m] = 0.0;
-    ab[2 * (size_t)i] = ab[2 * (size_t)i + 1] = cd[2 * (size_t)i] = cd[2 * (size_t)i + 1] = 0.0;
-  }
-  // slot 0..3: A, B, C, D
-  auto at = [&](int i, int slot) -> double & {
-    return (slot < 2 ? ab : cd)[2 * (size_t)i + (slot & 1)];
-  };
+                       double beta, bool tri, double *out) {
+  typedef long double real;
+  const int K = seg_count(n), CW = seg_cw(tri);
+  double *fch = out + (size_t)SEG_PACK * K, *bch = fch + SEG_CHAIN;
+  std::fill(out, out + seg_table_doubles(n), 0.0);
+  std::vector<real> R[4];  // A, B, C, D
+  for (int u = 0; u < 4; ++u) R[u].assign(n, 0);
   for (int w = 0; w < K; ++w) {
-    const int s0 = SEG_LEN * w, e0 = (w == K - 1) ? n : s0 + SEG_LEN;
-    if (w > 0) {
-      for (int u = 0; u < 2; ++u) {
-        const int slot = u;  // A or B
-        double m2 = u ? 0.0 : 1.0, m1 = u ? 1.0 : 0.0;  // y_{s0-2}, y_{s0-1}
-        for (int i = s0; i < e0; ++i) {
-          double yi = -p[i] * m2 - f[i] * m1;
-          if (i == n - 1) yi -= beta * at(n - 4, slot);
-          at(i, slot) = yi;
-          m2 = m1;
-          m1 = yi;
-        }
+    const int s0 = seg_len(n) * w, e0 = (w == K - 1) ? n : s0 + seg_len(n);
+    for (int u = 0; u < 2 && w > 0; ++u) {
+      real m2 = u ? 0 : 1, m1 = u ? 1 : 0;  // y_{s0-2}, y_{s0-1}
+      for (int i = s0; i < e0; ++i) {
+        real yi = -(real)p[i] * m2 - (real)f[i] * m1;
+        if (i == n - 1) yi -= beta * R[u][n - 4];
+        R[u][i] = yi;
+        m2 = m1;
+        m1 = yi;
       }
     }
-    if (w < K - 1) {
-      for (int u = 0; u < 2; ++u) {
-        const int slot = 2 + u;  // C or D
-        double p1 = u ? 0.0 : 1.0, p2 = u ? 1.0 : 0.0;  // x_{e0}, x_{e0+1}
-        for (int i = e0 - 1; i >= s0; --i) {
-          double xi = -e[i] * p2 - d[i] * p1;
-          if (i == 0) xi -= alpha * at(3, slot);
-          xi *= rc[i];
-          at(i, slot) = xi;
-          p2 = p1;
-          p1 = xi;
-        }
+    for (int u = 2; u < 4 && w < K - 1; ++u) {
+      real p1 = u == 2 ? 1 : 0, p2 = u == 2 ? 0 : 1;  // x_{e0}, x_{e0+1}
+      for (int i = e0 - 1; i >= s0; --i) {
+        real xi = -(real)e[i] * p2 - (real)d[i] * p1;
+        if (i == 0) xi -= alpha * R[u][3];
+        xi *= rc[i];
+        R[u][i] = xi;
+        p2 = p1;
+        p1 = xi;
       }
     }
+    double *pk = out + (size_t)SEG_PACK * w;
+    for (int i = s0; i < e0; ++i) {
+      double *r = pk + (size_t)CW * (i - s0);
+      auto w = [&](int m) { return (real)dr[i + (size_t)n * m]; };
+      if (i < 2 || i >= n - 2) {
+        for (int m = 0; m < 5; ++m) r[m] = (double)w(m);
+        const int x = i < 2 ? SEG_XHEAD + 2 * i : SEG_XTAIL + 2 * (i - (n - 2));
+        pk[x] = (double)w(5);
+        pk[x + 1] = (double)w(6);
+      } else {
+        r[0] = (double)(w(0) + w(1) + w(2) + w(3) + w(4));
+        r[1] = (double)-w(0);
+        r[2] = (double)(-w(0) - w(1));
+        r[3] = (double)(w(3) + w(4));
+        r[4] = (double)w(4);
+      }
+      auto put = [&](auto slot) {
+        typedef decltype(slot) S;
+        r[S::F] = f[i]; r[S::D] = d[i]; r[S::RC] = rc[i];
+        r[S::HB] = (double)R[1][i]; r[S::HC] = (double)R[2][i];
+        if (!tri) {
+          r[S::P] = p[i]; r[S::E] = e[i];
+          r[S::HA] = (double)R[0][i]; r[S::HD] = (double)R[3][i];
+        }
+      };
+      if (tri) put(SegSlot<true>());
+      else put(SegSlot<false>());
+    }
+    pk[SEG_XALPHA] = alpha;
+    pk[SEG_XBETA] = beta;
+    fch[4 * w + 0] = (double)R[0][e0 - 2];
+    fch[4 * w + 1] = (double)R[1][e0 - 2];
+    fch[4 * w + 2] = (double)R[0][e0 - 1];
+    fch[4 * w + 3] = (double)R[1][e0 - 1];
+    bch[4 * w + 0] = (double)R[2][s0];
+    bch[4 * w + 1] = (double)R[3][s0];
+    bch[4 * w + 2] = (double)R[2][s0 + 1];
+    bch[4 * w + 3] = (double)R[3][s0 + 1];
   }
 }
 

@@ -83,10 +83,8 @@ def test_derivatives_c1():
     _der_case(mf, (gx, gy, gz), u, 6, label="c1")
 
 
-# line lengths cover one to four 32-row segments (9 .. 130, a 38-row last
-# segment at 70, sub-lines with fewer segments than the full lines at 39) and
-# a 340-point line, longer than the segmented solve's LDS tables allow, which
-# takes the one-lane-per-line kernel
+# line lengths cover one to eleven segments of up to 32 rows, and sub-lines
+# with fewer segments than the full lines (33, 65, 130)
 @pytest.mark.parametrize("shape", [(9, 10, 11), (33, 17, 40), (70, 65, 10), (130, 12, 9),
                                    (39, 340, 38)])
 @pytest.mark.parametrize("so", [4, 6, 8])
@@ -129,6 +127,67 @@ def test_der_lines():
         ora = getattr(odc, name)(x)
         ex = getattr(odc, name)(x.astype(np.longdouble))
         _check("lines " + name, got, ex, ora)
+
+
+# one segment, even and uneven segments, 16 full ones, and the one-lane kernel
+# beyond; groups of 64 lines full, short by one and just begun; lines apart by
+# more than their length
+@pytest.mark.parametrize("n", [10, 32, 33, 64, 66, 321, 481, 512, 513])
+@pytest.mark.parametrize("so", [6, 8])
+def test_der_lines_segments(n, so):
+    mf, torch = _mf()
+    g = o.grid_tanh(n, 0, 1, 1.3)
+    dc = mf.DerivativeCoefficients(g, solver=True, so=so)
+    odc = o.DerCoeffs(g, solver=True, so=so)
+    rng = np.random.default_rng(n)
+    for nl, gap in ((1, 0), (63, 0), (65, 3), (128, 1)):
+        x = np.asfortranarray(rng.standard_normal((n + gap, nl)))
+        xd = mf.to_device(x)
+        for name in ("der", "dder", "der_s", "dder_s"):
+            print("run lines n=%d so=%d nl=%d gap=%d %s" % (n, so, nl, gap, name), flush=True)
+            out = mf.fortran_zeros((n + gap, nl))
+            out.fill_(7.0)
+            getattr(dc, name)(xd[:n], out[:n])
+            got = mf.to_host(out)
+            ends = slice(1, n - 1) if name.endswith("_s") else slice(0, n)
+            ora = getattr(odc, name)(x[:n])[ends]
+            ex = getattr(odc, name)(x[:n].astype(np.longdouble))[ends]
+            _check("lines n=%d so=%d %s" % (n, so, name), got[ends], ex, ora)
+            got[ends] = 7.0
+            assert (got == 7.0).all()  # nothing else is written
+
+
+# rows of whole cache lines: groups of 64 lines aligned in memory (64, 240 and
+# 192 columns; 48 and 80 lose too many lanes and keep the groups in turn)
+@pytest.mark.parametrize("shape", [(64, 11, 34), (240, 10, 12), (192, 33, 9), (48, 12, 10),
+                                   (80, 9, 33)])
+def test_derivatives_aligned_groups(shape):
+    mf, torch = _mf()
+    rng = np.random.default_rng(sum(shape))
+    gs = [o.grid_uniform(shape[0], 0, 1), o.grid_tanh(shape[1], 0, 2, 1.8),
+          o.grid_asin(shape[2], -0.5, 0.5)]
+    f = np.asfortranarray(rng.standard_normal(shape))
+    for so in (6, 8):
+        _der_case(mf, gs, f, so, label=str(shape))
+
+
+def test_derivatives_batch_fields():
+    """Eight fields in one launch equal eight launches, bit for bit."""
+    import ctypes as C
+    mf, torch = _mf()
+    shape = (70, 41, 36)
+    gs = [o.grid_uniform(shape[0]), o.grid_tanh(shape[1], 0, 1, 1.5), o.grid_uniform(shape[2])]
+    rng = np.random.default_rng(8)
+    x = [mf.to_device(np.asfortranarray(rng.standard_normal(shape))) for _ in range(8)]
+    for axis in range(3):
+        print("run batch axis %d" % axis, flush=True)
+        dc = mf.DerivativeCoefficients(gs[axis], solver=True, so=6)
+        out = [mf.fortran_zeros(shape) for _ in range(8)]
+        arr = C.c_void_p * 8
+        assert mf.load().mf_der3d_batch(dc.handle, axis, 1, 8, arr(*[t.data_ptr() for t in x]),
+                                        arr(*[t.data_ptr() for t in out]), *shape, None) == 0
+        for a, b in zip(x, out):
+            assert bool((mf.derivative(dc, a, axis, 1) == b).all())
 
 
 @pytest.mark.parametrize("n,so", [(64, 6), (192, 6), (33, 4)])
