@@ -167,7 +167,9 @@ class DerivativeCoefficients:
             raise ValueError("line length %d != handle size %d" % (x2.shape[0], self.n))
         nl = x2.shape[1]
         if out is None:
-            out = torch.zeros_like(x) if x.dim() == 1 else fortran_zeros(tuple(x2.shape), x.device)
+            out = torch.empty_like(x) if x.dim() == 1 else fortran_empty(tuple(x2.shape), x.device)
+            if sub:  # the sub-line scheme leaves the end points as they are
+                out[::self.n - 1] = 0.0
         o2 = out.reshape(self.n, 1) if out.dim() == 1 else out
         ld = x2.stride(1) if nl > 1 else self.n
         if x2.stride(0) != 1 or (nl > 1 and (o2.stride(0) != 1 or o2.stride(1) != ld)):
