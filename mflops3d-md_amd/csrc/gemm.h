@@ -5,16 +5,29 @@
 //   x-transform:  C(n1, n2 n3) = W(n1,n1) . F(n1, n2 n3)          (W left)
 //   y-transform:  C_k(n1, n2)  = F_k(n1,n2) . Wt(n2,n2), k = 1..n3 (W right, batched)
 //   z-transform:  C(n1 n2, n3) = F(n1 n2, n3) . Wt(n3,n3)         (W right)
-// In all three A is M-contiguous and B is K-contiguous, so one kernel serves
-// them.  The block tile spans the whole eigenvector dimension (256 >= n), so
-// each field element is read from HBM exactly once per transform and the
-// eigenvector matrix streams from L2.
+// In all three A is M-contiguous.  B is K-contiguous where it is the field
+// (x) and N-contiguous where it is the matrix (y and z: W itself, whose
+// columns are Wt's rows).
+//
+// One wave forms one (16 MI) x (16 NI) tile of C on its own: the MFMA
+// operands come straight from global memory into registers, D k-steps ahead,
+// with no LDS and no barrier.  A 16 x 16 x 4 FP64 MFMA occupies its SIMD for
+// 64 cycles, so a 64 x 64 tile spends 1024 cycles on a k-step's 8 loads of
+// 512 bytes; the waves of a block take the tiles that share the field's
+// values, which then come from L1, and the matrix streams from L2.  What bounds
+// it is the matrix rate on large problems and, on small ones, the latency of
+// one pass of loads: there the tiles shrink until every SIMD has a wave
+// (gemm_tile_of), and with 16 k-steps ahead a 62-point axis is one pass.
 //
 // MFMA operand order is swapped (D = B^T-fragment x A-fragment) so that the
 // 16 lanes holding one D row are 16 consecutive m: stores of the
 // column-major C are 128-byte contiguous segments.
 #pragma once
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
 
 namespace mf {
 
@@ -57,35 +70,25 @@ struct EpiArgs {
   int nx, ny;
 };
 
-// Block tile BM x BN on 4 waves.  A side of 64/128/256 is split into 64-wide
-// wave tiles (4 x 4 MFMA blocks of 16); a side of 192 into 4 wave tiles of 48
-// (3 MFMA blocks), for eigenvector dimensions of 129..192 points.
-template <typename T, typename TA, typename TB, typename TC, int BM, int BN, int EPI>
-__global__ void __launch_bounds__(256)
-    gemm_mode_kernel(const TA *__restrict__ A, long lda, long sA, const TB *__restrict__ B,
-                     long ldb, TC *__restrict__ C, long ldc, long sC, int M, int N, int K,
-                     EpiArgs ep) {
-  constexpr int BK = 16;
-  constexpr int NA = BM * BK / 256;
-  constexpr int NB = BN * BK / 256;
-  // wave grid WM x WN, each wave MI x NI MFMA blocks of 16 x 16
-  constexpr int MI = BM == 192 ? 3 : 4, NI = BN == 192 ? 3 : 4;
-  constexpr int WM = BM / (16 * MI), WN = BN / (16 * NI);
-  static_assert(WM * WN == 4 && WM * 16 * MI == BM && WN * 16 * NI == BN, "4 wave tiles");
+// A: M-contiguous; B: K-contiguous (KB) or N-contiguous.  tm x tn x batch
+// tiles, one per wave: the M tiles of a column group in turn when the field is
+// B, the N tiles of a row group when it is A.
+template <typename T, typename TC, int MI, int NI, int D, bool KB, int EPI>
+__global__ void __launch_bounds__(256, 2)
+    gemm_mode_kernel(const T *__restrict__ A, long lda, long sA, const T *__restrict__ B, long ldb,
+                     TC *__restrict__ C, long ldc, long sC, int M, int N, int K, int tm, int tn,
+                     long waves, EpiArgs ep) {
   typedef typename Mfma<T>::acc_t acc_t;
-  __shared__ T As[BK][BM];
-  __shared__ T Bs[BN][BK + 1];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const long m0 = (long)blockIdx.x * BM;
-  const long n0 = (long)blockIdx.y * BN;
-  A += (long)blockIdx.z * sA;
-  if (EPI == EPI_STORE || EPI == EPI_DIVIDE) C += (long)blockIdx.z * sC;
-  // four wave tiles arranged WM x WN
-  const int wm = (wave % WM) * 16 * MI;
-  const int wn = (wave / WM) * 16 * NI;
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const int wv = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (wv >= waves) return;
+  int im, in, ib;
+  if (KB) { im = wv % tm; in = (wv / tm) % tn; }
+  else { in = wv % tn; im = (wv / tn) % tm; }
+  ib = wv / (tm * tn);
+  const int m0 = im * 16 * MI, n0 = in * 16 * NI;
+  A += (long)ib * sA;
+  if (EPI == EPI_STORE || EPI == EPI_DIVIDE) C += (long)ib * sC;
 
   acc_t acc[MI][NI];
 #pragma unroll
@@ -93,63 +96,83 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int b = 0; b < NI; ++b) acc[a][b] = (acc_t){0, 0, 0, 0};
 
-  T ra[NA], rb[NB];
-  auto load = [&](int kt) {
+  // Operand pointers at k = 4 s + g of step s.  Rows and columns past the
+  // edge repeat the last one (their results are not stored); in the last step
+  // lanes past K repeat k = K - 1 and their operands are set to zero.
+  const int KS = (K + 3) / 4;
+  const int over = max(0, 4 * (KS - 1) + g - (K - 1));
+  const long sb = KB ? 1 : ldb;
+  const long a4 = 4 * lda, b4 = 4 * sb, aL = (4 - over) * lda, bL = (4 - over) * sb;
+  const T *pa[MI], *pb[NI];
 #pragma unroll
-    for (int q = 0; q < NA; ++q) {
-      const int e = tid + 256 * q;
-      const long m = m0 + (e % BM);
-      const int k = kt + e / BM;
-      ra[q] = (m < M && k < K) ? (T)A[m + lda * k] : (T)0;
-    }
+  for (int i = 0; i < MI; ++i)
+    pa[i] = A + min(m0 + 16 * i + c, M - 1) + lda * (KS == 1 ? g - over : g);
 #pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int e = tid + 256 * q;
-      const int k = kt + e % BK;
-      const long n = n0 + e / BK;
-      rb[q] = (n < N && k < K) ? (T)B[k + ldb * n] : (T)0;
-    }
+  for (int i = 0; i < NI; ++i)
+    pb[i] = B + (long)min(n0 + 16 * i + c, N - 1) * (KB ? ldb : 1) + sb * (KS == 1 ? g - over : g);
+  T af[D][MI], bf[D][NI];
+  // fetch step s into slot d and move the pointers to step s + 1
+  auto fetch = [&](int d, int s) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) af[d][i] = *pa[i];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) bf[d][i] = *pb[i];
+    const bool last = s + 2 == KS, end = s + 2 > KS;
+    const long da = end ? 0 : (last ? aL : a4), db = end ? 0 : (last ? bL : b4);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) pa[i] += da;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) pb[i] += db;
   };
-  load(0);
-  for (int kt = 0; kt < K; kt += BK) {
-    __syncthreads();
+  auto mma = [&](int d) {
 #pragma unroll
-    for (int q = 0; q < NA; ++q) {
-      const int e = tid + 256 * q;
-      As[e / BM][e % BM] = ra[q];
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < NI; ++ni)
+        acc[mi][ni] = Mfma<T>::op(bf[d][ni], af[d][mi], acc[mi][ni]);
+  };
+  auto mma_end = [&](int d, int s) {  // a step that may be the last
+    if (s + 1 == KS && over > 0) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i) af[d][i] = (T)0;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) bf[d][i] = (T)0;
     }
+    mma(d);
+  };
 #pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int e = tid + 256 * q;
-      Bs[e / BK][e % BK] = rb[q];
-    }
-    __syncthreads();
-    if (kt + BK < K) load(kt + BK);
+  for (int d = 0; d < D; ++d)
+    if (d < KS) fetch(d, d);
+  int s = 0;
+  for (; s + 2 * D <= KS; s += D) {
 #pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      T af[MI], bf[NI];
-#pragma unroll
-      for (int i = 0; i < MI; ++i) af[i] = As[kk + (lane >> 4)][wm + i * 16 + (lane & 15)];
-#pragma unroll
-      for (int i = 0; i < NI; ++i) bf[i] = Bs[wn + i * 16 + (lane & 15)][kk + (lane >> 4)];
-#pragma unroll
-      for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = Mfma<T>::op(bf[ni], af[mi], acc[mi][ni]);
+    for (int d = 0; d < D; ++d) {
+      mma(d);
+      fetch(d, s + d + D);
     }
   }
-  // epilogue: lane holds C(m0+wm+16mi+lane%16, n0+wn+16ni+row(lane,r)).
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (s + d < KS) {
+      mma_end(d, s + d);
+      if (s + d + D < KS) fetch(d, s + d + D);
+    }
+  s += D;
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (s + d < KS) mma_end(d, s + d);
+  // epilogue: lane holds C(m0+16mi+lane%16, n0+16ni+row(lane,r)).
   // Index splits (m -> i1,i2; n -> j,k) take one 32-bit division per lane and
   // then advance with wrap-around.
   int i1 = 0, i2 = 0;
   if (EPI == EPI_DIVIDE) {
-    const int mb = (int)(m0 + wm + (lane & 15));
+    const int mb = m0 + c;
     i1 = mb % ep.n1;
     i2 = mb / ep.n1;
   }
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi) {
-    const long m = m0 + wm + mi * 16 + (lane & 15);
+    const int m = m0 + mi * 16 + c;
     if (mi > 0 && EPI == EPI_DIVIDE) {
       i1 += 16;
       while (i1 >= ep.n1) { i1 -= ep.n1; ++i2; }
@@ -164,7 +187,7 @@ __global__ void __launch_bounds__(256)
     int jb = 0, kb = 0;
     if (EPI == EPI_SCATTER || EPI == EPI_SCATTER_ADD) {
       ubase = m + 1;
-      const int nb = (int)(n0 + wn);
+      const int nb = n0;
       jb = nb % ep.n2;
       kb = nb / ep.n2;
     }
@@ -173,7 +196,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int dn = ni * 16 + Mfma<T>::row(lane, r);
-        const long n = n0 + wn + dn;
+        const int n = n0 + dn;
         if (n >= N) continue;
         const double v = (double)acc[mi][ni][r];
         if (EPI == EPI_STORE) {
@@ -196,6 +219,69 @@ __global__ void __launch_bounds__(256)
             *p += v;
         }
       }
+  }
+}
+
+// Tile of a product, in MFMA blocks: the one whose waves take the least time
+// on the busiest SIMD, a k-step of a wave costing its MFMAs (64 cycles each)
+// or its loads (512 B each, a CU's L1 delivering 64 B a cycle to 4 SIMDs),
+// whichever is more, and each wave the latency of its first loads.  At 254
+// points 64 x 64 tiles (4 waves per SIMD); 48 wide where that pads less (130
+// columns in three); a 62^3 field 16 x 16 tiles, since 64-wide ones would leave
+// fifteen SIMDs of sixteen empty.  Measured against block tiles staged through
+// LDS (one barrier pair per 16-deep step, two blocks per CU), bit for bit the
+// same results: a 256^3 FP64 solve 1.397 -> 1.051 ms, a 64^3 one 121 -> 38 us,
+// training targets 256^3 -> 64^3 1.90 -> 1.33 ms.
+struct GemmTile {
+  int mi, ni;
+};
+inline GemmTile gemm_tile_of(int M, int N, int K, int batch, int ncu) {
+  static const GemmTile all[] = {{4, 4}, {4, 3}, {3, 4}, {3, 3}, {4, 2}, {2, 4}, {2, 2}, {1, 1}};
+  GemmTile best = all[0];
+  double least = 0.0;
+  for (const GemmTile &t : all) {
+    const double w = (double)((M + 16 * t.mi - 1) / (16 * t.mi)) *
+                     ((N + 16 * t.ni - 1) / (16 * t.ni)) * batch;
+    const double per = std::ceil(w / (4.0 * ncu));
+    const double step = std::max(64.0 * t.mi * t.ni, 32.0 * (t.mi + t.ni));
+    const double cost = per * ((K + 3) / 4) * step + 2000.0 * std::ceil(per / 2.0);
+    if (least == 0.0 || cost < least) {
+      least = cost;
+      best = t;
+    }
+  }
+  return best;
+}
+
+// C = A B (per batch) with the epilogue EPI, enqueued on st.
+template <typename T, typename TC, bool KB, int EPI>
+void gemm_launch(const T *A, long lda, long sA, const T *B, long ldb, TC *C, long ldc, long sC,
+                 int M, int N, int K, int batch, const EpiArgs &ep, int ncu, hipStream_t st) {
+  const GemmTile t = gemm_tile_of(M, N, K, batch, ncu);
+  const int tm = (M + 16 * t.mi - 1) / (16 * t.mi), tn = (N + 16 * t.ni - 1) / (16 * t.ni);
+  const long waves = (long)tm * tn * batch;
+  const dim3 grid((unsigned)((waves + 3) / 4));
+  auto go = [&](auto mi, auto ni, auto d) {
+    hipLaunchKernelGGL((gemm_mode_kernel<T, TC, decltype(mi)::value, decltype(ni)::value,
+                                         decltype(d)::value, KB, EPI>),
+                       grid, dim3(256), 0, st, A, lda, sA, B, ldb, C, ldc, sC, M, N, K, tm, tn,
+                       waves, ep);
+  };
+  typedef std::integral_constant<int, 1> I1;
+  typedef std::integral_constant<int, 2> I2;
+  typedef std::integral_constant<int, 3> I3;
+  typedef std::integral_constant<int, 4> I4;
+  typedef std::integral_constant<int, 8> I8;
+  typedef std::integral_constant<int, 16> I16;
+  switch (10 * t.mi + t.ni) {
+    case 44: go(I4(), I4(), I4()); break;
+    case 43: go(I4(), I3(), I4()); break;
+    case 34: go(I3(), I4(), I4()); break;
+    case 33: go(I3(), I3(), I4()); break;
+    case 42: go(I4(), I2(), I4()); break;
+    case 24: go(I2(), I4(), I4()); break;
+    case 22: go(I2(), I2(), I8()); break;
+    default: go(I1(), I1(), I16()); break;
   }
 }
 

@@ -298,7 +298,7 @@ struct mf_filter {
   int nin = 0, nout = 0;
   std::vector<double> F;   // nout x nin, column-major
   double *dF = nullptr;    // F (nout x nin) column-major
-  double *dFt = nullptr;   // F^T (nin x nout) column-major
+  int ncu = 256;           // compute units of the device the handle was created on
 };
 
 namespace {
@@ -426,16 +426,16 @@ extern "C" int mf_filter_create(const double *xi, const double *wi, int nin, con
       h->F[o + (size_t)nout * r] = (double)v;
     }
   }
-  std::vector<double> Ft((size_t)nin * nout);
-  for (int o = 0; o < nout; ++o)
-    for (int r = 0; r < nin; ++r) Ft[r + (size_t)nin * o] = h->F[o + (size_t)nout * r];
+  {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
+      h->ncu = cus;
+  }
   hipError_t e = hipMalloc(&h->dF, h->F.size() * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&h->dFt, Ft.size() * sizeof(double));
   if (e == hipSuccess) e = hipMemcpy(h->dF, h->F.data(), h->F.size() * sizeof(double), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(h->dFt, Ft.data(), Ft.size() * sizeof(double), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     if (h->dF) (void)hipFree(h->dF);
-    if (h->dFt) (void)hipFree(h->dFt);
     delete h;
     return mf::fail(MF_ERR_DEVICE, std::string("mf_filter_create: ") + hipGetErrorString(e));
   }
@@ -446,7 +446,6 @@ extern "C" int mf_filter_create(const double *xi, const double *wi, int nin, con
 extern "C" int mf_filter_destroy(mf_filter *h) {
   if (!h) return MF_OK;
   if (h->dF) (void)hipFree(h->dF);
-  if (h->dFt) (void)hipFree(h->dFt);
   delete h;
   return MF_OK;
 }
@@ -458,31 +457,15 @@ extern "C" int mf_filter_matrix(const mf_filter *h, double *F) {
 }
 
 namespace {
+// C = A B: the filter matrix left (WLEFT) of the field, or right of it (B the
+// matrix F itself, whose columns are F^T's rows)
 template <bool WLEFT>
 void launch_fgemm(const double *A, long lda, long sA, const double *B, long ldb, double *C, long ldc,
-                  long sC, int M, int N, int K, int batch, hipStream_t st) {
+                  long sC, int M, int N, int K, int batch, int ncu, hipStream_t st) {
   mf::EpiArgs ep;
   std::memset(&ep, 0, sizeof(ep));
-  const int d = WLEFT ? M : N;
-  const int t = d <= 64 ? 64 : (d <= 128 ? 128 : 256);
-  auto go = [&](auto bm, auto bn) {
-    constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value;
-    dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN, batch);
-    hipLaunchKernelGGL((mf::gemm_mode_kernel<double, double, double, double, BM, BN, mf::EPI_STORE>),
-                       grid, dim3(256), 0, st, A, lda, sA, B, ldb, C, ldc, sC, M, N, K, ep);
-  };
-  using I64 = std::integral_constant<int, 64>;
-  using I128 = std::integral_constant<int, 128>;
-  using I256 = std::integral_constant<int, 256>;
-  if (WLEFT) {
-    if (t == 64) go(I64(), I256());
-    else if (t == 128) go(I128(), I128());
-    else go(I256(), I64());
-  } else {
-    if (t == 64) go(I256(), I64());
-    else if (t == 128) go(I128(), I128());
-    else go(I64(), I256());
-  }
+  mf::gemm_launch<double, double, WLEFT, mf::EPI_STORE>(A, lda, sA, B, ldb, C, ldc, sC, M, N, K, batch,
+                                                       ep, ncu, st);
 }
 }  // namespace
 
@@ -494,13 +477,13 @@ extern "C" int mf_filter3d(const mf_filter *fx, const mf_filter *fy, const mf_fi
   hipStream_t st = (hipStream_t)stream;
   double *w1 = work, *w2 = work + (size_t)nxo * nyi * nzi;
   // x: w1 (nxo, nyi nzi) = Fx in
-  launch_fgemm<true>(fx->dF, nxo, 0, in, nxi, w1, nxo, 0, nxo, nyi * nzi, nxi, 1, st);
+  launch_fgemm<true>(fx->dF, nxo, 0, in, nxi, w1, nxo, 0, nxo, nyi * nzi, nxi, 1, fx->ncu, st);
   // y: w2_k (nxo, nyo) = w1_k Fy^T, batched over z
-  launch_fgemm<false>(w1, nxo, (long)nxo * nyi, fy->dFt, nyi, w2, nxo, (long)nxo * nyo, nxo, nyo, nyi,
-                      nzi, st);
+  launch_fgemm<false>(w1, nxo, (long)nxo * nyi, fy->dF, nyo, w2, nxo, (long)nxo * nyo, nxo, nyo, nyi,
+                      nzi, fx->ncu, st);
   // z: out (nxo nyo, nzo) = w2 Fz^T
-  launch_fgemm<false>(w2, (long)nxo * nyo, 0, fz->dFt, nzi, out, (long)nxo * nyo, 0, nxo * nyo, nzo,
-                      nzi, 1, st);
+  launch_fgemm<false>(w2, (long)nxo * nyo, 0, fz->dF, nzo, out, (long)nxo * nyo, 0, nxo * nyo, nzo,
+                      nzi, 1, fx->ncu, st);
   LESCHK(hipGetLastError());
   return MF_OK;
 }

@@ -210,10 +210,12 @@ struct mf_solver3d {
   mf::Solver1D ax[3];
   // device memory
   void *dmem = nullptr;
-  // FP64 eigen transforms: Wx = inv_vect_x, Vx = vect_x; Wy_t = inv_vect_y^T ...
-  double *Wx = nullptr, *Vx = nullptr, *Wyt = nullptr, *Vyt = nullptr, *Wzt = nullptr, *Vzt = nullptr;
-  float *Wx32 = nullptr, *Vx32 = nullptr, *Wyt32 = nullptr, *Vyt32 = nullptr, *Wzt32 = nullptr,
-        *Vzt32 = nullptr;  // mixed: W' = inv(V) inv(lhs)
+  // FP64 eigen transforms: W = inv_vect, V = vect of each axis; Wyt, Wzt the
+  // transposes the unit-impulse spectra read
+  double *Wx = nullptr, *Vx = nullptr, *Wy = nullptr, *Vy = nullptr, *Wz = nullptr, *Vz = nullptr;
+  double *Wyt = nullptr, *Wzt = nullptr;
+  float *Wx32 = nullptr, *Vx32 = nullptr, *Wy32 = nullptr, *Vy32 = nullptr, *Wz32 = nullptr,
+        *Vz32 = nullptr;  // mixed: W' = inv(V) inv(lhs)
   // the same six matrices split into three bf16 parts, [part][k/8][row][k%8]
   // (row = the eigenvector-dimension index, zero-padded to wrows[axis] rows
   // and kp[axis] columns)
@@ -471,7 +473,7 @@ extern "C" int mf_solver3d_create(const double *gx, int nx, const double *gy, in
   }
   const int n[3] = {h->n1, h->n2, h->n3};
   // host images of the device tables
-  std::vector<double> W[3], V[3], Wp[3];
+  std::vector<double> W[3], V[3], Wp[3], wp0[3];  // wp0: W' untransposed
   for (int a = 0; a < 3; ++a) {
     const mf::Solver1D &s = h->ax[a];
     const int m = n[a];
@@ -483,6 +485,7 @@ extern "C" int mf_solver3d_create(const double *gx, int nx, const double *gy, in
         if (b == 0.0) continue;
         for (int i = 0; i < m; ++i) wp[i + (size_t)m * j] += s.inv_vect[i + (size_t)m * k] * b;
       }
+    wp0[a] = wp;
     if (a == 0) {
       W[a] = s.inv_vect;
       V[a] = s.vect;
@@ -604,6 +607,8 @@ extern "C" int mf_solver3d_create(const double *gx, int nx, const double *gy, in
       return r;
     };
     for (int a = 0; a < 3; ++a) { dW[a] = take((size_t)n[a] * n[a]); dV[a] = take((size_t)n[a] * n[a]); }
+    h->Wyt = take((size_t)n[1] * n[1]);
+    h->Wzt = take((size_t)n[2] * n[2]);
     for (int a = 0; a < 3; ++a) {
       fW[a] = (float *)take(((size_t)n[a] * n[a] + 1) / 2);
       fV[a] = (float *)take(((size_t)n[a] * n[a] + 1) / 2);
@@ -650,8 +655,8 @@ extern "C" int mf_solver3d_create(const double *gx, int nx, const double *gy, in
     return mf::fail(MF_ERR_DEVICE, std::string("mf_solver3d_create: hipMalloc: ") + hipGetErrorString(e));
   }
   carve((double *)h->dmem);
-  h->Wx = dW[0]; h->Vx = dV[0]; h->Wyt = dW[1]; h->Vyt = dV[1]; h->Wzt = dW[2]; h->Vzt = dV[2];
-  h->Wx32 = fW[0]; h->Vx32 = fV[0]; h->Wyt32 = fW[1]; h->Vyt32 = fV[1]; h->Wzt32 = fW[2]; h->Vzt32 = fV[2];
+  h->Wx = dW[0]; h->Vx = dV[0]; h->Wy = dW[1]; h->Vy = dV[1]; h->Wz = dW[2]; h->Vz = dV[2];
+  h->Wx32 = fW[0]; h->Vx32 = fV[0]; h->Wy32 = fW[1]; h->Vy32 = fV[1]; h->Wz32 = fW[2]; h->Vz32 = fV[2];
   auto up = [&](void *dst, const void *src, size_t bytes) {
     return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
   };
@@ -662,10 +667,13 @@ extern "C" int mf_solver3d_create(const double *gx, int nx, const double *gy, in
   };
   e = hipSuccess;
   for (int a = 0; a < 3 && e == hipSuccess; ++a) {
-    e = up(dW[a], W[a].data(), W[a].size() * sizeof(double));
-    if (e == hipSuccess) e = up(dV[a], V[a].data(), V[a].size() * sizeof(double));
-    if (e == hipSuccess) e = upf(fW[a], Wp[a]);
-    if (e == hipSuccess) e = upf(fV[a], V[a]);
+    const std::vector<double> &iv = h->ax[a].inv_vect, &v = h->ax[a].vect;
+    e = up(dW[a], iv.data(), iv.size() * sizeof(double));
+    if (e == hipSuccess) e = up(dV[a], v.data(), v.size() * sizeof(double));
+    if (e == hipSuccess && a > 0)
+      e = up(a == 1 ? h->Wyt : h->Wzt, W[a].data(), W[a].size() * sizeof(double));
+    if (e == hipSuccess) e = upf(fW[a], wp0[a]);
+    if (e == hipSuccess) e = upf(fV[a], v);
   }
   // three-part bf16 splits: [part][k/8][row][k%8]; the x matrices are the left
   // operand (row = m of W(m,k)), the stored y/z transposes the right one
@@ -775,63 +783,21 @@ extern "C" int mf_solver3d_create(const double *gx, int nx, const double *gy, in
 namespace {
 using mf::EpiArgs;
 
-template <typename T, typename TA, typename TB, typename TC, int BM, int BN, int EPI>
-void launch_tile(mf_solver3d *h, const TA *A, long lda, long sA, const TB *B, long ldb, TC *C,
+// One transform (or batch of transforms) on the FP64 or FP32 matrix cores.
+// WLEFT: the matrix is A and the field B (K-contiguous); else the field is A
+// and the matrix B, N-contiguous.
+template <typename T, typename TC, bool WLEFT, int EPI>
+void launch_gemm(mf_solver3d *h, const T *A, long lda, long sA, const T *B, long ldb, TC *C,
                  long ldc, long sC, int M, int N, int K, int batch, const EpiArgs &ep,
                  hipStream_t st) {
-  dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN, batch);
   ProfScope ps(h, sizeof(T) == 8 ? P_T64 : P_T32, 2.0 * M * N * K * batch, st);
-  hipLaunchKernelGGL((mf::gemm_mode_kernel<T, TA, TB, TC, BM, BN, EPI>), grid, dim3(256), 0, st, A,
-                     lda, sA, B, ldb, C, ldc, sC, M, N, K, ep);
+  mf::gemm_launch<T, TC, WLEFT, EPI>(A, lda, sA, B, ldb, C, ldc, sC, M, N, K, batch, ep, h->ncu, st);
 }
 
-// Block tile by the eigenvector dimension n (M for the x-transform, whose
-// eigenvector matrix is the left operand; N for y/z): the tile side along n
-// is the smallest of 64/128/192/256 covering it, so every field element is
-// read once and few MFMA rows are padding.  WLEFT selects the orientation.
-inline int gemm_mode_tile(int n) { return n > 128 && n <= 192 ? 192 : gemm_tile(n); }
-
-template <typename T, typename TA, typename TB, typename TC, bool WLEFT, int EPI>
-void launch_gemm(mf_solver3d *h, const TA *A, long lda, long sA, const TB *B, long ldb, TC *C,
-                 long ldc, long sC, int M, int N, int K, int batch, const EpiArgs &ep,
-                 hipStream_t st) {
-  const int t = gemm_mode_tile(WLEFT ? M : N);
-  // the batched y-transform with a 256-wide N tile and 129..192 rows: one
-  // 192-row M tile and four 64-wide N tiles (the field slice re-read from L2)
-  // give 4 blocks per slice where 64-row M tiles give 3, which at 190 slices
-  // leaves the last round of blocks a quarter full
-  if (!WLEFT && t == 256 && M > 128 && M <= 192 && batch > 1) {
-    launch_tile<T, TA, TB, TC, 192, 64, EPI>(h, A, lda, sA, B, ldb, C, ldc, sC, M, N, K, batch, ep, st);
-    return;
-  }
-  if (t == 192) {
-    if (WLEFT)
-      launch_tile<T, TA, TB, TC, 192, 64, EPI>(h, A, lda, sA, B, ldb, C, ldc, sC, M, N, K, batch, ep, st);
-    else
-      launch_tile<T, TA, TB, TC, 64, 192, EPI>(h, A, lda, sA, B, ldb, C, ldc, sC, M, N, K, batch, ep, st);
-    return;
-  }
-  if (WLEFT) {
-    if (t == 64)
-      launch_tile<T, TA, TB, TC, 64, 256, EPI>(h, A, lda, sA, B, ldb, C, ldc, sC, M, N, K, batch, ep, st);
-    else if (t == 128)
-      launch_tile<T, TA, TB, TC, 128, 128, EPI>(h, A, lda, sA, B, ldb, C, ldc, sC, M, N, K, batch, ep, st);
-    else
-      launch_tile<T, TA, TB, TC, 256, 64, EPI>(h, A, lda, sA, B, ldb, C, ldc, sC, M, N, K, batch, ep, st);
-  } else {
-    if (t == 64)
-      launch_tile<T, TA, TB, TC, 256, 64, EPI>(h, A, lda, sA, B, ldb, C, ldc, sC, M, N, K, batch, ep, st);
-    else if (t == 128)
-      launch_tile<T, TA, TB, TC, 128, 128, EPI>(h, A, lda, sA, B, ldb, C, ldc, sC, M, N, K, batch, ep, st);
-    else
-      launch_tile<T, TA, TB, TC, 64, 256, EPI>(h, A, lda, sA, B, ldb, C, ldc, sC, M, N, K, batch, ep, st);
-  }
-}
-
-// Six transforms: in (interior, type TIn) -> u interior (scatter or add).
-template <typename T, typename TIn>
-void transforms(mf_solver3d *h, const TIn *in, T *w1, T *w2, const T *Wx, const T *Wyt,
-                const T *Wzt, const T *Vx, const T *Vyt, const T *Vzt, double sigma, double *u,
+// Six transforms: in (interior) -> u interior (scatter or add).
+template <typename T>
+void transforms(mf_solver3d *h, const T *in, T *w1, T *w2, const T *Wx, const T *Wy,
+                const T *Wz, const T *Vx, const T *Vy, const T *Vz, double sigma, double *u,
                 bool accumulate, hipStream_t st, bool last = true) {
   const int n1 = h->n1, n2 = h->n2, n3 = h->n3;
   const long n12 = (long)n1 * n2;
@@ -847,21 +813,21 @@ void transforms(mf_solver3d *h, const TIn *in, T *w1, T *w2, const T *Wx, const 
   ep.nx = h->nx;
   ep.ny = h->ny;
   // forward X: w1 = Wx . in
-  launch_gemm<T, T, TIn, T, true, mf::EPI_STORE>(h, Wx, n1, 0, in, n1, w1, n1, 0, n1, n2 * n3, n1, 1, ep, st);
-  // forward Y: w2_k = w1_k . Wyt
-  launch_gemm<T, T, T, T, false, mf::EPI_STORE>(h, w1, n1, n12, Wyt, n2, w2, n1, n12, n1, n2, n2, n3, ep, st);
-  // forward Z with the eigenvalue divide: w1 = (w2 . Wzt) / lambda
-  launch_gemm<T, T, T, T, false, mf::EPI_DIVIDE>(h, w2, n12, 0, Wzt, n3, w1, n12, 0, (int)n12, n3, n3, 1, ep, st);
-  // backward Z: w2 = w1 . Vzt
-  launch_gemm<T, T, T, T, false, mf::EPI_STORE>(h, w1, n12, 0, Vzt, n3, w2, n12, 0, (int)n12, n3, n3, 1, ep, st);
-  // backward Y: w1_k = w2_k . Vyt
-  launch_gemm<T, T, T, T, false, mf::EPI_STORE>(h, w2, n1, n12, Vyt, n2, w1, n1, n12, n1, n2, n2, n3, ep, st);
+  launch_gemm<T, T, true, mf::EPI_STORE>(h, Wx, n1, 0, in, n1, w1, n1, 0, n1, n2 * n3, n1, 1, ep, st);
+  // forward Y: w2_k = w1_k . Wy
+  launch_gemm<T, T, false, mf::EPI_STORE>(h, w1, n1, n12, Wy, n2, w2, n1, n12, n1, n2, n2, n3, ep, st);
+  // forward Z with the eigenvalue divide: w1 = (w2 . Wz) / lambda
+  launch_gemm<T, T, false, mf::EPI_DIVIDE>(h, w2, n12, 0, Wz, n3, w1, n12, 0, (int)n12, n3, n3, 1, ep, st);
+  // backward Z: w2 = w1 . Vz
+  launch_gemm<T, T, false, mf::EPI_STORE>(h, w1, n12, 0, Vz, n3, w2, n12, 0, (int)n12, n3, n3, 1, ep, st);
+  // backward Y: w1_k = w2_k . Vy
+  launch_gemm<T, T, false, mf::EPI_STORE>(h, w2, n1, n12, Vy, n2, w1, n1, n12, n1, n2, n2, n3, ep, st);
   // backward X into u's interior
   if (!last) return;
   if (accumulate)
-    launch_gemm<T, T, T, double, true, mf::EPI_SCATTER_ADD>(h, Vx, n1, 0, w1, n1, (double *)nullptr, 0, 0, n1, n2 * n3, n1, 1, ep, st);
+    launch_gemm<T, double, true, mf::EPI_SCATTER_ADD>(h, Vx, n1, 0, w1, n1, (double *)nullptr, 0, 0, n1, n2 * n3, n1, 1, ep, st);
   else
-    launch_gemm<T, T, T, double, true, mf::EPI_SCATTER>(h, Vx, n1, 0, w1, n1, (double *)nullptr, 0, 0, n1, n2 * n3, n1, 1, ep, st);
+    launch_gemm<T, double, true, mf::EPI_SCATTER>(h, Vx, n1, 0, w1, n1, (double *)nullptr, 0, 0, n1, n2 * n3, n1, 1, ep, st);
 }
 
 // ---- split-bf16 transforms (MF_MIXED_BF16X3)
@@ -899,7 +865,7 @@ void launch_bf3(mf_solver3d *h, const TF *F, long ldf, long sF, const __bf16 *W,
   }
 }
 
-// The six transforms of transforms<float, double> with the pre-split
+// The six transforms of transforms<float> with the pre-split
 // matrices W' = inv(V) inv(lhs) and V.
 void transforms_bf3(mf_solver3d *h, const float *in, float *w1, float *w2, double sigma,
                     double *u, bool accumulate, hipStream_t st, bool last = true) {
@@ -1165,11 +1131,11 @@ extern "C" int mf_solver3d_time_transforms(mf_solver3d *h, int precision, int re
   HIPCHK(hipEventCreate(&e1));
   auto five = [&] {
     if (precision == MF_FP64)
-      transforms<double, double>(h, h->T2, h->T1, h->T2, h->Wx, h->Wyt, h->Wzt, h->Vx, h->Vyt,
-                                 h->Vzt, 0.0, nullptr, false, st, false);
+      transforms<double>(h, h->T2, h->T1, h->T2, h->Wx, h->Wy, h->Wz, h->Vx, h->Vy,
+                                 h->Vz, 0.0, nullptr, false, st, false);
     else if (precision == MF_MIXED)
-      transforms<float, float>(h, h->R32, h->F1, h->F2, h->Wx32, h->Wyt32, h->Wzt32, h->Vx32,
-                               h->Vyt32, h->Vzt32, 0.0, nullptr, false, st, false);
+      transforms<float>(h, h->R32, h->F1, h->F2, h->Wx32, h->Wy32, h->Wz32, h->Vx32,
+                               h->Vy32, h->Vz32, 0.0, nullptr, false, st, false);
     else if (precision == MF_MIXED_BF16X3)
       transforms_bf3(h, h->R32, h->F1, h->F2, 0.0, nullptr, false, st, false);
     else
@@ -1315,8 +1281,8 @@ void inner_solve(mf_solver3d *h, int precision, double sigma, double *u, bool ac
   else if (precision == MF_MIXED_FP16X2)
     transforms_h2(h, h->R32, h->F1, h->F2, sigma, u, accumulate, st);
   else
-    transforms<float, float>(h, h->R32, h->F1, h->F2, h->Wx32, h->Wyt32, h->Wzt32, h->Vx32,
-                             h->Vyt32, h->Vzt32, sigma, u, accumulate, st);
+    transforms<float>(h, h->R32, h->F1, h->F2, h->Wx32, h->Wy32, h->Wz32, h->Vx32,
+                             h->Vy32, h->Vz32, sigma, u, accumulate, st);
 }
 
 // u's faces from the latest sweep's interior and the norms of its residuals
@@ -1363,8 +1329,8 @@ int mf::solver3d_solve_begin(mf_solver3d *h, const double *g, double sigma, doub
       hipLaunchKernelGGL(mf::null_sub_kernel, dim3((unsigned)nb), dim3(256), 0, st, h->T2, N,
                          (const double *)h->npart, h->n3 * mf::NULL_SLICES, h->inv_wsum);
     }
-    transforms<double, double>(h, h->T2, h->T1, h->T2, h->Wx, h->Wyt, h->Wzt, h->Vx, h->Vyt,
-                               h->Vzt, sigma, u, false, st);
+    transforms<double>(h, h->T2, h->T1, h->T2, h->Wx, h->Wy, h->Wz, h->Vx, h->Vy,
+                               h->Vz, sigma, u, false, st);
     HIPCHK(hipGetLastError());
     return launch_faces(h, u, bcx, bcy, bcz, st);
   }
@@ -1569,11 +1535,11 @@ extern "C" int mf_influence_impulses(mf_solver3d *h, const mf_der *dx, const mf_
                          dim3((unsigned)(((long)n1 * n2 + 255) / 256), 1, nb), dim3(256), 0, st, W1, ia);
     }
     // backward transforms, batched over the impulses
-    launch_gemm<double, double, double, double, false, mf::EPI_STORE>(
-        h, W1, n12, N, h->Vzt, n3, W2, n12, N, (int)n12, n3, n3, nb, ep, st);
-    launch_gemm<double, double, double, double, false, mf::EPI_STORE>(
-        h, W2, n1, n12, h->Vyt, n2, W1, n1, n12, n1, n2, n2, n3 * nb, ep, st);
-    launch_gemm<double, double, double, double, true, mf::EPI_STORE>(
+    launch_gemm<double, double, false, mf::EPI_STORE>(
+        h, W1, n12, N, h->Vz, n3, W2, n12, N, (int)n12, n3, n3, nb, ep, st);
+    launch_gemm<double, double, false, mf::EPI_STORE>(
+        h, W2, n1, n12, h->Vy, n2, W1, n1, n12, n1, n2, n2, n3 * nb, ep, st);
+    launch_gemm<double, double, true, mf::EPI_STORE>(
         h, h->Vx, n1, 0, W1, n1, W2, n1, 0, n1, (int)((long)n2 * n3 * nb), n1, 1, ep, st);
     mf::FaceDerArgs fa;
     fa.n1 = n1; fa.n2 = n2; fa.n3 = n3; fa.face = face; fa.first = first + b0;
@@ -1994,7 +1960,7 @@ int mf::influence_assemble(const std::vector<InflSub> &subs, double sigma, bool 
                                tb + tt.ahat[pp.fi], b1);
             // Z = G_side TT_c
             const double *G = b1 + (long)(pp.fo % 2) * n[b] * n[c];
-            launch_gemm<double, double, double, double, true, mf::EPI_STORE>(
+            launch_gemm<double, double, true, mf::EPI_STORE>(
                 h, G, n[b], 0, W + ttoff[c], n[c], b2, n[b], 0, n[b], n[c] * n[c], n[c], 1, ep, st);
           } else {
             const int u = 3 - s - t;
@@ -2003,11 +1969,11 @@ int mf::influence_assemble(const std::vector<InflSub> &subs, double sigma, bool 
             hipLaunchKernelGGL(mf::infl_h_kernel, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, st,
                                ea, s, t, u, n[s], n[t], n[u], layout, tb + tt.Om[t][pp.fo % 2], b1);
             if (layout == 0)  // Y = (Vs diag(ahat)) H
-              launch_gemm<double, double, double, double, true, mf::EPI_STORE>(
+              launch_gemm<double, double, true, mf::EPI_STORE>(
                   h, tb + tt.VsA[pp.fi], n[s], 0, b1, n[s], b2, n[s], 0, n[s], n[t] * n[u], n[s], 1,
                   ep, st);
             else  // Y'_ct = H'_ct (Vs diag(ahat))^T, batched over ct
-              launch_gemm<double, double, double, double, true, mf::EPI_STORE>(
+              launch_gemm<double, double, true, mf::EPI_STORE>(
                   h, b1, n[u], (long)n[u] * n[s], tb + tt.VsT[pp.fi], n[s], b2, n[u],
                   (long)n[u] * n[s], n[u], n[s], n[s], n[t], ep, st);
           }
