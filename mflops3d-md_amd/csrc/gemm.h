@@ -57,6 +57,13 @@ struct Mfma<float> {
   static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
 };
 
+// R = 1 / (lx + ly + lz + sigma), 0 where max(|sigma|, |l|) < 1e-11 (the
+// eigen-divide's null-mode guard, class_solver_3d.f90:202-225)
+__device__ __forceinline__ double inv_eig(double lx, double ly, double lz, double sigma) {
+  const double big = fmax(fmax(fabs(sigma), fmax(fabs(lx), fabs(ly))), fabs(lz));
+  return big < 1e-11 ? 0.0 : 1.0 / (((lx + ly) + lz) + sigma);
+}
+
 enum EpiMode { EPI_STORE = 0, EPI_DIVIDE = 1, EPI_SCATTER = 2, EPI_SCATTER_ADD = 3 };
 
 struct EpiArgs {
@@ -70,27 +77,15 @@ struct EpiArgs {
   int nx, ny;
 };
 
-// A: M-contiguous; B: K-contiguous (KB) or N-contiguous.  tm x tn x batch
-// tiles, one per wave: the M tiles of a column group in turn when the field is
-// B, the N tiles of a row group when it is A.
-template <typename T, typename TC, int MI, int NI, int D, bool KB, int EPI>
-__global__ void __launch_bounds__(256, 2)
-    gemm_mode_kernel(const T *__restrict__ A, long lda, long sA, const T *__restrict__ B, long ldb,
-                     TC *__restrict__ C, long ldc, long sC, int M, int N, int K, int tm, int tn,
-                     long waves, EpiArgs ep) {
+// The products of one tile of C = A B, rows from m0 and columns from n0, by one
+// wave: lane l ends with C(m0 + 16 mi + l%16, n0 + 16 ni + row(l, r)) in
+// acc[mi][ni][r].  A: M-contiguous; B: K-contiguous (KB) or N-contiguous.
+template <typename T, int MI, int NI, int D, bool KB>
+__device__ __forceinline__ void gemm_tile(const T *__restrict__ A, long lda,
+                                          const T *__restrict__ B, long ldb, int M, int N, int K,
+                                          int m0, int n0, typename Mfma<T>::acc_t (&acc)[MI][NI]) {
   typedef typename Mfma<T>::acc_t acc_t;
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  const int wv = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (wv >= waves) return;
-  int im, in, ib;
-  if (KB) { im = wv % tm; in = (wv / tm) % tn; }
-  else { in = wv % tn; im = (wv / tn) % tm; }
-  ib = wv / (tm * tn);
-  const int m0 = im * 16 * MI, n0 = in * 16 * NI;
-  A += (long)ib * sA;
-  if (EPI == EPI_STORE || EPI == EPI_DIVIDE) C += (long)ib * sC;
-
-  acc_t acc[MI][NI];
 #pragma unroll
   for (int a = 0; a < MI; ++a)
 #pragma unroll
@@ -140,9 +135,10 @@ __global__ void __launch_bounds__(256, 2)
     }
     mma(d);
   };
+  // every fetch is unconditional (past the last step it repeats it), so that the
+  // compiler waits for exactly the loads each step needs
 #pragma unroll
-  for (int d = 0; d < D; ++d)
-    if (d < KS) fetch(d, d);
+  for (int d = 0; d < D; ++d) fetch(d, d);
   int s = 0;
   for (; s + 2 * D <= KS; s += D) {
 #pragma unroll
@@ -151,16 +147,41 @@ __global__ void __launch_bounds__(256, 2)
       fetch(d, s + d + D);
     }
   }
+  if (s + D < KS) {
 #pragma unroll
-  for (int d = 0; d < D; ++d)
-    if (s + d < KS) {
-      mma_end(d, s + d);
-      if (s + d + D < KS) fetch(d, s + d + D);
+    for (int d = 0; d < D; ++d) {
+      mma(d);
+      fetch(d, s + d + D);
     }
-  s += D;
+    s += D;
+  }
 #pragma unroll
   for (int d = 0; d < D; ++d)
     if (s + d < KS) mma_end(d, s + d);
+}
+
+// A: M-contiguous; B: K-contiguous (KB) or N-contiguous.  tm x tn x batch
+// tiles, one per wave: the M tiles of a column group in turn when the field is
+// B, the N tiles of a row group when it is A.
+template <typename T, typename TC, int MI, int NI, int D, bool KB, int EPI>
+__global__ void __launch_bounds__(256, 2)
+    gemm_mode_kernel(const T *__restrict__ A, long lda, long sA, const T *__restrict__ B, long ldb,
+                     TC *__restrict__ C, long ldc, long sC, int M, int N, int K, int tm, int tn,
+                     long waves, EpiArgs ep) {
+  typedef typename Mfma<T>::acc_t acc_t;
+  const int lane = threadIdx.x & 63, c = lane & 15;
+  const int wv = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (wv >= waves) return;
+  int im, in, ib;
+  if (KB) { im = wv % tm; in = (wv / tm) % tn; }
+  else { in = wv % tn; im = (wv / tn) % tm; }
+  ib = wv / (tm * tn);
+  const int m0 = im * 16 * MI, n0 = in * 16 * NI;
+  A += (long)ib * sA;
+  if (EPI == EPI_STORE || EPI == EPI_DIVIDE) C += (long)ib * sC;
+
+  acc_t acc[MI][NI];
+  gemm_tile<T, MI, NI, D, KB>(A, lda, B, ldb, M, N, K, m0, n0, acc);
   // epilogue: lane holds C(m0+16mi+lane%16, n0+16ni+row(lane,r)).
   // Index splits (m -> i1,i2; n -> j,k) take one 32-bit division per lane and
   // then advance with wrap-around.
@@ -230,7 +251,7 @@ __global__ void __launch_bounds__(256, 2)
 // columns in three); a 62^3 field 16 x 16 tiles, since 64-wide ones would leave
 // fifteen SIMDs of sixteen empty.  Measured against block tiles staged through
 // LDS (one barrier pair per 16-deep step, two blocks per CU), bit for bit the
-// same results: a 256^3 FP64 solve 1.397 -> 1.051 ms, a 64^3 one 121 -> 38 us,
+// same results: a 256^3 FP64 solve 1.397 -> 1.051 ms, a 64^3 one 121 -> 37 us,
 // training targets 256^3 -> 64^3 1.90 -> 1.33 ms.
 struct GemmTile {
   int mi, ni;

@@ -31,13 +31,6 @@
 
 namespace mf {
 
-// R = 1 / (lx + ly + lz + sigma), 0 where max(|sigma|, |l|) < 1e-11 (the
-// eigen-divide's null-mode guard, class_solver_3d.f90:202-225)
-__device__ __forceinline__ double inv_eig(double lx, double ly, double lz, double sigma) {
-  const double big = fmax(fmax(fabs(sigma), fmax(fabs(lx), fabs(ly))), fabs(lz));
-  return big < 1e-11 ? 0.0 : 1.0 / (((lx + ly) + lz) + sigma);
-}
-
 // T[(o + n c) + n^2 a] = V(o,a) W(a,c) and TT[a + n (o + n c)] = the same
 // (V, W column-major n x n); one thread per element
 __global__ void __launch_bounds__(256) infl_t_kernel(const double *__restrict__ V,

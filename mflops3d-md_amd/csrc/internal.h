@@ -67,6 +67,21 @@ struct InflStats {
 int influence_assemble(const std::vector<InflSub> &subs, double sigma, bool graph, void *stream,
                        InflStats *stats = nullptr);
 
+// What the influence operator of a subdomain is made of, one axis at a time
+// (solve.hip): the device eigenvector matrices W = inv(V), V (column-major) and
+// eigenvalues of a solver handle ...
+struct SpectralAxes {
+  const double *W[3], *V[3], *lam[3];
+  int n[3];
+};
+SpectralAxes solver3d_axes(const struct ::mf_solver3d *sc);
+// ... ahat = W(-fold) of a unit value on face f (0..5), and per axis and side
+// the boundary-derivative row of the face in spectral space (what) and its
+// weights of the line's two end values (dcoef[output side][value side]).
+std::vector<double> influence_ahat(const struct ::mf_solver3d *sc, int face);
+bool influence_rows(const struct ::mf_solver3d *sc, const struct ::mf_der *d, int axis,
+                    std::vector<double> what[2], double dcoef[2][2]);
+
 // host copies of a derivative handle's tables (order 1|2, sub 0|1)
 bool der_host_tables(const struct ::mf_der *dc, int order, int sub, const double **dl_lu,
                      const double **dr, int *n);

@@ -53,29 +53,58 @@ struct Band {
 // BC fold: R(i,j,k) = g(i+1,j+1,k+1) - sum over the 6 faces of
 // fold_a(idx)*bc_a  with fold vectors fx1(i) = inv_lhs(i,1) ddr(1,1) +
 // inv_lhs(i,2) ddr(2,1), fx2(i) = inv_lhs(i,n-1) ddr(n-1,8) + inv_lhs(i,n) ddr(n,7).
+// One wave takes 64 columns i, FOLD_J rows j and kc planes: of the twelve
+// factors of a point only the two y-face values change with both i and k, and
+// they serve FOLD_J rows; the z-face values stay in registers over the planes
+// and the rest is wave-uniform.  HBM-bound, 16 B per point (one point per
+// thread with twelve loads beside its own: 133 us at 254^3, where a copy of
+// the field takes 53).
+constexpr int FOLD_J = 4;
 __global__ void __launch_bounds__(256)
     fold_kernel(const double *__restrict__ g, double *__restrict__ R, int n1, int n2, int n3,
                 const double *__restrict__ fold,  // fx1 fx2 fy1 fy2 fz1 fz2
                 const double *__restrict__ bcx, const double *__restrict__ bcy,
-                const double *__restrict__ bcz) {
-  // launch: block (64,4), grid (ceil(n1/64), ceil(n2/4), n3)
+                const double *__restrict__ bcz, int kc) {
+  // launch: block (64,4), grid (ceil(n1/64), ceil(n2/(4 FOLD_J)), ceil(n3/kc))
   const int i = blockIdx.x * 64 + threadIdx.x;
-  const int j = blockIdx.y * 4 + threadIdx.y;
-  const int k = blockIdx.z;
-  if (i >= n1 || j >= n2) return;
-  const long p = i + (long)n1 * (j + (long)n2 * k);
+  const int j0 = (blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.y)) * FOLD_J;
+  const int k0 = blockIdx.z * kc, k1 = min(n3, k0 + kc);
+  if (i >= n1 || j0 >= n2) return;
   const int nx = n1 + 2, ny = n2 + 2;
   const double *fx1 = fold, *fx2 = fx1 + n1, *fy1 = fx2 + n1, *fy2 = fy1 + n2;
   const double *fz1 = fy2 + n2, *fz2 = fz1 + n3;
-  double v = g[(i + 1) + (long)nx * ((j + 1) + (long)ny * (k + 1))];
   const long sx = (long)n2 * n3, sy = (long)n1 * n3, sz = (long)n1 * n2;
-  v -= fx1[i] * bcx[j + (long)n2 * k];
-  v -= fx2[i] * bcx[sx + j + (long)n2 * k];
-  v -= fy1[j] * bcy[i + (long)n1 * k];
-  v -= fy2[j] * bcy[sy + i + (long)n1 * k];
-  v -= fz1[k] * bcz[i + (long)n1 * j];
-  v -= fz2[k] * bcz[sz + i + (long)n1 * j];
-  R[p] = v;
+  const double a1 = fx1[i], a2 = fx2[i];
+  double z1[FOLD_J], z2[FOLD_J], b1[FOLD_J], b2[FOLD_J];
+#pragma unroll
+  for (int q = 0; q < FOLD_J; ++q) {
+    const int j = min(j0 + q, n2 - 1);
+    z1[q] = bcz[i + (long)n1 * j];
+    z2[q] = bcz[sz + i + (long)n1 * j];
+    b1[q] = fy1[j];
+    b2[q] = fy2[j];
+  }
+  for (int k = k0; k < k1; ++k) {
+    const double y1 = bcy[i + (long)n1 * k], y2 = bcy[sy + i + (long)n1 * k];
+    const double c1 = fz1[k], c2 = fz2[k];
+    double v[FOLD_J];
+#pragma unroll
+    for (int q = 0; q < FOLD_J; ++q) {
+      const int j = min(j0 + q, n2 - 1);
+      v[q] = g[(i + 1) + (long)nx * ((j + 1) + (long)ny * (k + 1))];
+    }
+#pragma unroll
+    for (int q = 0; q < FOLD_J; ++q) {
+      const int j = min(j0 + q, n2 - 1);
+      v[q] -= a1 * bcx[j + (long)n2 * k];
+      v[q] -= a2 * bcx[sx + j + (long)n2 * k];
+      v[q] -= b1[q] * y1;
+      v[q] -= b2[q] * y2;
+      v[q] -= c1 * z1[q];
+      v[q] -= c2 * z2[q];
+      if (j0 + q < n2) R[i + (long)n1 * (j + (long)n2 * k)] = v[q];
+    }
+  }
 }
 
 // Null component of a singular problem (sigma = 0 and a zero eigenvalue on
@@ -1317,8 +1346,13 @@ int mf::solver3d_solve_begin(mf_solver3d *h, const double *g, double sigma, doub
   if (precision == MF_FP64) {
     {
       ProfScope ps(h, P_FOLD, 16.0 * N, st);
-      hipLaunchKernelGGL(mf::fold_kernel, dim3((h->n1 + 63) / 64, (h->n2 + 3) / 4, h->n3), dim3(64, 4), 0, st, g, h->T2, h->n1, h->n2,
-                         h->n3, (const double *)h->fold, bcx, bcy, bcz);
+      // eight planes per wave on fields that fill the chip with them
+      const int kc = N >= (1L << 22) ? 8 : 1;
+      hipLaunchKernelGGL(mf::fold_kernel,
+                         dim3((h->n1 + 63) / 64, (h->n2 + 4 * mf::FOLD_J - 1) / (4 * mf::FOLD_J),
+                              (h->n3 + kc - 1) / kc),
+                         dim3(64, 4), 0, st, g, h->T2, h->n1, h->n2, h->n3, (const double *)h->fold,
+                         bcx, bcy, bcz, kc);
     }
     if (h->null_mode && sigma == 0.0) {
       ProfScope ps(h, P_FOLD, 16.0 * N, st);
@@ -1669,6 +1703,36 @@ void launch_infl_tile(int tile, const mf::InflProblem *probs, int nprob, long ti
 }
 
 }  // namespace
+
+mf::SpectralAxes mf::solver3d_axes(const mf_solver3d *h) {
+  SpectralAxes a;
+  const double *W[3] = {h->Wx, h->Wy, h->Wz}, *V[3] = {h->Vx, h->Vy, h->Vz};
+  const double *lam = h->lam;
+  const int n[3] = {h->n1, h->n2, h->n3};
+  for (int q = 0; q < 3; ++q) {
+    a.W[q] = W[q];
+    a.V[q] = V[q];
+    a.lam[q] = lam;
+    a.n[q] = n[q];
+    lam += n[q];
+  }
+  return a;
+}
+
+std::vector<double> mf::influence_ahat(const mf_solver3d *sc, int face) {
+  return impulse_ahat(sc, face / 2, face % 2);
+}
+
+bool mf::influence_rows(const mf_solver3d *sc, const mf_der *d, int axis,
+                        std::vector<double> what[2], double dcoef[2][2]) {
+  AxisTabs t;
+  if (!axis_tabs(sc, d, axis, t)) return false;
+  for (int s = 0; s < 2; ++s) {
+    what[s] = t.what[s];
+    for (int q = 0; q < 2; ++q) dcoef[s][q] = t.dcoef[s][q];
+  }
+  return true;
+}
 
 int mf::influence_assemble(const std::vector<InflSub> &subs, double sigma, bool graph, void *stream,
                            InflStats *stats) {
