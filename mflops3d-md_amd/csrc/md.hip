@@ -14,9 +14,12 @@
 // own interfaces (u_s x u_s, column-major in HBM): M = sum_s E_s D_s E_s^T,
 // with E_s the injection of s's interface unknowns.  D_s is filled from the
 // batched unit-impulse responses (mf_influence_impulses) by a scatter kernel.
-// A matrix-vector product is then one gather, one memory-bound GEMV per
-// subdomain (column chunks, fixed-order partial sums) and one combine of the
-// two sides of every interface unknown, so M x is deterministic.  The system
+// A product with the stored blocks (mf_md_matvec) is then one gather, one
+// memory-bound GEMV per subdomain (column chunks, fixed-order partial sums)
+// and one combine of the two sides of every interface unknown, so M x is
+// deterministic.  The solve applies the same operator from its one-axis
+// factors (infl_apply.h), which reads none of the blocks; with blocks from
+// unit-impulse solves (MF_INFL_IMPULSES=1) it multiplies by those.  The system
 // is solved by restarted GMRES on the device (classical Gram-Schmidt applied
 // twice, fixed-order dot products; the small Hessenberg least-squares
 // problem on the host).  Interface numbering and unknown order follow
@@ -30,6 +33,7 @@
 // the mean of its start; 2 zeroes the first right-hand-side entry.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstdio>
@@ -37,6 +41,7 @@
 #include <string>
 #include <vector>
 
+#include "infl_apply.h"
 #include "internal.h"
 #include "mflops/mf.h"
 
@@ -284,6 +289,14 @@ struct mf_md {
   size_t D_doubles = 0;
   long *map = nullptr;     // concatenated local -> global
   long *pa = nullptr, *pb = nullptr;
+  // the operator from its factors (infl_apply.h): four grouped transforms and
+  // the spectral sum between them; null: the solve multiplies by the blocks
+  void *apply = nullptr;   // one allocation: tables, problems, tile lists, roles
+  mf::ApplyProblem *ap[4] = {nullptr, nullptr, nullptr, nullptr};
+  int2 *atile[4] = {nullptr, nullptr, nullptr, nullptr};
+  int atiles[4] = {0, 0, 0, 0};
+  mf::ApplyRole *arole = nullptr;
+  int aroles = 0, ablocks = 0;
   double *ws = nullptr;    // GMRES and GEMV workspace
   size_t ws_doubles = 0;
   int restart = 30;
@@ -309,6 +322,7 @@ struct mf_md {
     if (map) (void)hipFree(map);
     if (pa) (void)hipFree(pa);
     if (pb) (void)hipFree(pb);
+    if (apply) (void)hipFree(apply);
     if (ws) (void)hipFree(ws);
     if (hist) (void)hipFree(hist);
     if (ones) (void)hipFree(ones);
@@ -332,7 +346,7 @@ namespace {
 // workspace layout (doubles): xs / ys (nloc each), GEMV partials, the Krylov
 // basis (ninf x (m+1)), w, x, r, dot partials, small vectors
 struct Ws {
-  double *xs, *ys, *part, *V, *w, *x, *r, *dpart, *hcol;
+  double *xs, *ys, *part, *V, *w, *x, *r, *dpart, *hcol, *t1, *xh;
   long nchunk_max;
 };
 
@@ -351,6 +365,8 @@ Ws carve(mf_md *h) {
   w.r = p; p += h->ninf;
   w.dpart = p; p += 256 * m1;
   w.hcol = p; p += 2 * m1;
+  w.t1 = p; p += h->nloc;
+  w.xh = p; p += h->nloc;
   w.nchunk_max = 0;
   return w;
 }
@@ -359,7 +375,7 @@ size_t ws_size(const mf_md *h) {
   const long m1 = h->restart + 1;
   long pmax = 0;
   for (auto &s : h->subs) pmax = std::max(pmax, ((s.u + 511) / 512) * s.u);
-  return 2 * (size_t)h->nloc + pmax + (size_t)h->ninf * m1 + 3 * (size_t)h->ninf + 256 * m1 + 2 * m1;
+  return 4 * (size_t)h->nloc + pmax + (size_t)h->ninf * m1 + 3 * (size_t)h->ninf + 256 * m1 + 2 * m1;
 }
 
 // y = M x (device vectors of ninf)
@@ -379,6 +395,149 @@ int matvec(mf_md *h, const Ws &w, const double *x, double *y, hipStream_t st) {
   hipLaunchKernelGGL(mf::md::combine_kernel, dim3(mf::md::nblk(h->ninf)), dim3(256), 0, st,
                      (const double *)w.ys, (const long *)h->pa, (const long *)h->pb, h->ninf, y);
   MDCHK(hipGetLastError());
+  return MF_OK;
+}
+
+// y = M x from the operator's factors, or by the blocks where the handle has
+// none (apply_setup)
+int apply_op(mf_md *h, const Ws &w, const double *x, double *y, hipStream_t st) {
+  if (!h->apply) return matvec(h, w, x, y, st);
+  const double *none = nullptr;
+  auto grid = [&](int q) { return dim3((unsigned)((h->atiles[q] + 3) / 4)); };
+  hipLaunchKernelGGL((mf::apply_gemm_kernel<true, false>), grid(0), dim3(256), 0, st,
+                     (const mf::ApplyProblem *)h->ap[0], (const int2 *)h->atile[0], h->atiles[0],
+                     none, x, w.t1, none);
+  hipLaunchKernelGGL((mf::apply_gemm_kernel<false, false>), grid(1), dim3(256), 0, st,
+                     (const mf::ApplyProblem *)h->ap[1], (const int2 *)h->atile[1], h->atiles[1],
+                     (const double *)w.t1, none, w.xh, none);
+  hipLaunchKernelGGL(mf::apply_sum_kernel, dim3(h->ablocks, h->aroles), dim3(64, mf::APPLY_SPLIT), 0,
+                     st, (const mf::ApplyRole *)h->arole, (const double *)w.xh, w.t1, h->sigma);
+  hipLaunchKernelGGL((mf::apply_gemm_kernel<true, false>), grid(2), dim3(256), 0, st,
+                     (const mf::ApplyProblem *)h->ap[2], (const int2 *)h->atile[2], h->atiles[2],
+                     none, (const double *)w.t1, w.xh, none);
+  hipLaunchKernelGGL((mf::apply_gemm_kernel<false, true>), grid(3), dim3(256), 0, st,
+                     (const mf::ApplyProblem *)h->ap[3], (const int2 *)h->atile[3], h->atiles[3],
+                     (const double *)w.xh, none, w.ys, x);
+  hipLaunchKernelGGL(mf::md::combine_kernel, dim3(mf::md::nblk(h->ninf)), dim3(256), 0, st,
+                     (const double *)w.ys, (const long *)h->pa, (const long *)h->pb, h->ninf, y);
+  MDCHK(hipGetLastError());
+  return MF_OK;
+}
+
+// Tables and launch lists of apply_op.  Per face (in the order of the
+// concatenated local unknowns): offset ys_off + loc_off in every face vector,
+// its unknowns contiguous in x from ioff (both column-major over the face).
+int apply_setup(mf_md *h) {
+  if (!h->ninf) return MF_OK;
+  std::vector<double> tab;
+  std::vector<mf::ApplyProblem> pr[4];
+  std::vector<int2> tl[4];
+  std::vector<mf::ApplyRole> roles;
+  auto put = [&](const std::vector<double> &v) {
+    const size_t o = tab.size();
+    tab.insert(tab.end(), v.begin(), v.end());
+    return (const double *)(o * sizeof(double));  // an offset until the upload
+  };
+  int maxpts = 0;
+  for (auto &s : h->subs) {
+    if (!s.u) continue;
+    const mf::SpectralAxes A = mf::solver3d_axes(s.sc);
+    std::vector<double> what[3][2];
+    double dco[3][2][2];
+    for (int q = 0; q < 3; ++q)
+      if (!mf::influence_rows(s.sc, s.d[q], q, what[q], dco[q]))
+        return mf::fail(MF_ERR_SETUP, "mf_md_create: derivative tables");
+    mf::ApplyRole base;
+    std::memset(&base, 0, sizeof(base));
+    for (int q = 0; q < 3; ++q) { base.n[q] = A.n[q]; base.lam[q] = A.lam[q]; }
+    base.nf = s.nf;
+    long xof[6];  // each face's unknowns in x
+    for (int f = 0; f < s.nf; ++f) {
+      base.fax[f] = s.face[f] / 2;
+      base.ahat[f] = put(mf::influence_ahat(s.sc, s.face[f]));
+      base.xoff[f] = s.ys_off + s.loc_off[f];
+      xof[f] = h->ioff[s.iface[f]];
+    }
+    for (int f = 0; f < s.nf; ++f) {
+      const int a = s.face[f] / 2, b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
+      const int nb = A.n[b], nc = A.n[c];
+      const long off = base.xoff[f];
+      for (int q = 0; q < 4; ++q) {
+        mf::ApplyProblem p;
+        std::memset(&p, 0, sizeof(p));
+        const bool left = q % 2 == 0;
+        p.M = nb; p.N = nc; p.K = left ? nb : nc;
+        p.lda = nb; p.ldc = nb;
+        p.ldb = left ? nb : nc;
+        if (left) p.A = q == 0 ? A.W[b] : A.V[b];
+        else p.B = q == 1 ? A.W[c] : A.V[c];
+        p.a = off;
+        p.b = q == 0 ? xof[f] : off;
+        p.c = off;
+        p.x0 = p.x1 = -1;
+        if (q == 3)
+          for (int e = 0; e < s.nf; ++e)
+            if (s.face[e] / 2 == a) {
+              const double w = dco[a][s.face[f] % 2][s.face[e] % 2];
+              if (p.x0 < 0) { p.x0 = xof[e]; p.c0 = w; }
+              else { p.x1 = xof[e]; p.c1 = w; }
+            }
+        const int tm = (nb + 15) / 16;
+        p.tn = (nc + 15) / 16;
+        for (int t = 0; t < tm * p.tn; ++t) tl[q].push_back(make_int2((int)pr[q].size(), t));
+        pr[q].push_back(p);
+      }
+    }
+    for (int a = 0; a < 3; ++a) {
+      mf::ApplyRole r = base;
+      r.a = a;
+      for (int f = 0; f < s.nf; ++f)
+        if (s.face[f] / 2 == a) {
+          r.what[r.no] = put(what[a][s.face[f] % 2]);
+          r.goff[r.no] = s.ys_off + s.loc_off[f];
+          ++r.no;
+        }
+      if (!r.no) continue;
+      if (r.no == 1) r.what[1] = r.what[0];
+      const int b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
+      maxpts = std::max(maxpts, A.n[b] * A.n[c]);
+      roles.push_back(r);
+    }
+  }
+  // one allocation: tables, then each launch's problems and tiles, then roles
+  size_t bytes = 0;
+  auto take = [&](size_t n) {
+    const size_t o = bytes;
+    bytes += (n + 255) / 256 * 256;
+    return o;
+  };
+  const size_t o_tab = take(tab.size() * sizeof(double));
+  size_t o_pr[4], o_tl[4];
+  for (int q = 0; q < 4; ++q) {
+    o_pr[q] = take(pr[q].size() * sizeof(mf::ApplyProblem));
+    o_tl[q] = take(tl[q].size() * sizeof(int2));
+  }
+  const size_t o_ro = take(roles.size() * sizeof(mf::ApplyRole));
+  MDCHK(hipMalloc(&h->apply, bytes));
+  char *d = (char *)h->apply;
+  for (auto &r : roles) {
+    for (int f = 0; f < r.nf; ++f) r.ahat[f] = (const double *)(d + o_tab + (size_t)r.ahat[f]);
+    for (int q = 0; q < 2; ++q) r.what[q] = (const double *)(d + o_tab + (size_t)r.what[q]);
+  }
+  std::vector<char> img(bytes, 0);
+  std::memcpy(&img[o_tab], tab.data(), tab.size() * sizeof(double));
+  for (int q = 0; q < 4; ++q) {
+    std::memcpy(&img[o_pr[q]], pr[q].data(), pr[q].size() * sizeof(mf::ApplyProblem));
+    std::memcpy(&img[o_tl[q]], tl[q].data(), tl[q].size() * sizeof(int2));
+    h->ap[q] = (mf::ApplyProblem *)(d + o_pr[q]);
+    h->atile[q] = (int2 *)(d + o_tl[q]);
+    h->atiles[q] = (int)tl[q].size();
+  }
+  std::memcpy(&img[o_ro], roles.data(), roles.size() * sizeof(mf::ApplyRole));
+  h->arole = (mf::ApplyRole *)(d + o_ro);
+  h->aroles = (int)roles.size();
+  h->ablocks = (maxpts + 63) / 64;
+  MDCHK(hipMemcpy(h->apply, img.data(), bytes, hipMemcpyHostToDevice));
   return MF_OK;
 }
 
@@ -589,6 +748,13 @@ int md_create(const int nd[3], const int *npts, const double *grids, const int b
   if (e == hipSuccess && h->ninf) e = hipMalloc(&h->hist, 3 * (size_t)h->ninf * sizeof(double));
   if (e == hipSuccess && h->ninf) e = hipMemset(h->hist, 0, 3 * (size_t)h->ninf * sizeof(double));
   if (e != hipSuccess) return bail(mf::fail(MF_ERR_DEVICE, std::string("mf_md_create: ") + hipGetErrorString(e)));
+  // blocks from unit-impulse solves: the solve multiplies by them
+  const char *imp_env = std::getenv("MF_INFL_IMPULSES");
+  const bool impulses = imp_env && imp_env[0] == '1';
+  if (!impulses) {
+    const int rc = apply_setup(h);
+    if (rc != MF_OK) return bail(rc);
+  }
   if (!assemble) {  // the caller fills the blocks (matrix cache)
     *out = h;
     return MF_OK;
@@ -596,8 +762,7 @@ int md_create(const int nd[3], const int *npts, const double *grids, const int b
   // influence blocks by spectral contraction (one persistent grouped launch,
   // captured in a HIP graph), or, with MF_INFL_IMPULSES=1, from batched
   // unit-impulse solves as the reference forms them
-  const char *imp_env = std::getenv("MF_INFL_IMPULSES");
-  if (!(imp_env && imp_env[0] == '1')) {
+  if (!impulses) {
     std::vector<mf::InflSub> is;
     for (auto &s : h->subs) {
       if (!s.u) continue;
@@ -780,7 +945,7 @@ extern "C" int mf_md_solve(mf_md *h, const double *const *g, double *const *u,
   bool done = bnorm == 0.0;
   while (!done && iters < max_iter) {
     // r0 = b - M x -> V[:,0]
-    MDRC(matvec(h, w, w.x, V, st));
+    MDRC(apply_op(h, w, w.x, V, st));
     hipLaunchKernelGGL(mf::md::axpby_kernel, dim3(mf::md::nblk(n)), dim3(256), 0, st, 1.0,
                        (const double *)b, -1.0, V, n);
     // with the constant null space every Krylov vector is kept orthogonal
@@ -799,7 +964,7 @@ extern "C" int mf_md_solve(mf_md *h, const double *const *g, double *const *u,
     int k = 0;
     for (; k < m && iters < max_iter; ++k) {
       double *vk1 = V + (long)(k + 1) * n;
-      MDRC(matvec(h, w, V + (long)k * n, vk1, st));
+      MDRC(apply_op(h, w, V + (long)k * n, vk1, st));
       if (nullsp) MDRC(remove_constant(h, w, vk1, st));
       // classical Gram-Schmidt, applied twice
       for (int pass = 0; pass < 2; ++pass) {
@@ -850,7 +1015,7 @@ extern "C" int mf_md_solve(mf_md *h, const double *const *g, double *const *u,
     if (rel <= tol) done = true;
   }
   // true residual of the final x
-  MDRC(matvec(h, w, w.x, w.w, st));
+  MDRC(apply_op(h, w, w.x, w.w, st));
   hipLaunchKernelGGL(mf::md::axpby_kernel, dim3(mf::md::nblk(n)), dim3(256), 0, st, 1.0,
                      (const double *)b, -1.0, w.w, n);
   if (nullsp) MDRC(remove_constant(h, w, w.w, st));

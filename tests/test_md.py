@@ -411,6 +411,52 @@ def test_gpu_md_spectral_assembly(lay, bct, per):
     assert torch.equal(ys[0], ys[1]) and torch.equal(ys[1], ys[2])
 
 
+def layout_uneven():
+    return [[o.grid_asin(12, 0.0, 0.5), o.grid_asin(19, 0.5, 1.0)],
+            [o.grid_asin(35, 0.0, 0.4), o.grid_asin(10, 0.4, 0.7), o.grid_asin(17, 0.7, 1.0)],
+            [o.grid_asin(18, 0.0, 1.0)]]
+
+
+# faces smaller and larger than a 16 x 16 tile, up to four faces on a
+# subdomain, Neumann outer faces, and a single subdomain along a periodic axis
+# (both its faces carry the same unknowns)
+@pytest.mark.gpu
+@pytest.mark.parametrize("lay,bct,per", [(layout_uneven, (1,) * 6, (False, False, False)),
+                                         (layout_3d, (1, 2, 1, 1, 2, 1), (False, False, False)),
+                                         (lambda: layout_periodic(12), (2, 2, 1, 2, 2, 2),
+                                          (True, False, True))])
+def test_gpu_md_factored_operator(lay, bct, per):
+    """The solve's operator, applied from its one-axis factors, against the
+    blocks: at a GMRES tolerance of 1e-13 the interface values of the two agree
+    to the conditioning of the system times rounding (bar 1e-10), and the
+    block product at the factored solution equals the one at the block
+    solution."""
+    mf, torch = _mf()
+    grids = lay()
+    sigma = -7.0
+    print("run md factored operator %s periods %s" % ([len(v) for v in grids], per), flush=True)
+    mk = lambda: mf.Multidomain(grids, sigma, bct=bct, periods=per)
+    h, hd = mk(), _with_env("MF_INFL_IMPULSES", "1", mk)
+    rng = np.random.default_rng(11)
+    g = [mf.to_device(np.asfortranarray(rng.standard_normal(s))) for s in h.shapes]
+    bc = [torch.tensor(rng.standard_normal(2 * ((s[1] - 2) * (s[2] - 2) + (s[0] - 2) * (s[2] - 2)
+                                               + (s[0] - 2) * (s[1] - 2))), device="cuda")
+          for s in h.shapes]
+    xs, reps = [], []
+    for q in (h, hd):
+        x = torch.zeros(q.ninf, dtype=torch.float64, device="cuda")
+        u, rep = q.solve(g, bc, tol=1e-13, max_iter=200, x_iface=x)
+        xs.append(x)
+        reps.append(rep)
+    err = ((xs[0] - xs[1]).abs().max() / xs[1].abs().max()).item()
+    y0, y1 = hd.matvec(xs[0]), hd.matvec(xs[1])
+    ey = ((y0 - y1).abs().max() / y1.abs().max()).item()
+    print("  x %.2e  M x %.2e  its %d / %d" % (err, ey, reps[0].iterations, reps[1].iterations),
+          flush=True)
+    assert err < 1e-10 and ey < 1e-11
+    assert abs(reps[0].iterations - reps[1].iterations) <= 1
+
+
 @pytest.mark.gpu
 def test_gpu_md_rejects_bad_layout():
     mf, torch = _mf()
