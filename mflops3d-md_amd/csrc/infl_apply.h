@@ -81,6 +81,11 @@ struct ApplyRole {
 
 constexpr int APPLY_SPLIT = 4;  // waves per 64 face points, each a part of the summed axis
 
+// NF: the most faces of any subdomain (a role with fewer adds zero times a
+// finite value for the rest, so that the line's loads need no branch and four
+// points' loads are in flight together: 33 us a product with one point at a
+// time, at the sizes above)
+template <int NF>
 __global__ void __launch_bounds__(64 * APPLY_SPLIT)
     apply_sum_kernel(const ApplyRole *__restrict__ roles, const double *__restrict__ xhat,
                      double *__restrict__ ghat, double sigma) {
@@ -94,13 +99,13 @@ __global__ void __launch_bounds__(64 * APPLY_SPLIT)
   const int ib = pt % nb, ic = pt / nb;
   // per face, its term along the line: k q[st al], Xhat times ahat(al) on the
   // line's own axis, ahat of the line times Xhat along it otherwise
-  double k[6];
-  const double *q[6];
-  long st[6];
+  double k[NF];
+  const double *q[NF];
+  int st[NF];
 #pragma unroll
-  for (int f = 0; f < 6; ++f) {
+  for (int f = 0; f < NF; ++f) {
     k[f] = 0.0;
-    q[f] = xhat;
+    q[f] = r.ahat[0];
     st[f] = 0;
     if (f < r.nf) {
       const double *xh = xhat + r.xoff[f];
@@ -120,20 +125,19 @@ __global__ void __launch_bounds__(64 * APPLY_SPLIT)
       }
     }
   }
-  double l3[3];
-  l3[b] = r.lam[b][ib];
-  l3[c] = r.lam[c][ic];
+  const double *la = r.lam[a], *w0 = r.what[0], *w1 = r.what[1];
+  const double lb = r.lam[b][ib], lc = r.lam[c][ic];
   const int per = (na + APPLY_SPLIT - 1) / APPLY_SPLIT, a0 = w * per, a1 = min(na, a0 + per);
   double s0 = 0.0, s1 = 0.0;
+#pragma unroll 4
   for (int al = a0; al < a1; ++al) {
     double v = 0.0;
 #pragma unroll
-    for (int f = 0; f < 6; ++f)
-      if (f < r.nf) v = fma(k[f], q[f][st[f] * al], v);
-    l3[a] = r.lam[a][al];
-    v *= inv_eig(l3[0], l3[1], l3[2], sigma);
-    s0 = fma(r.what[0][al], v, s0);
-    if (r.no > 1) s1 = fma(r.what[1][al], v, s1);
+    for (int f = 0; f < NF; ++f) v = fma(k[f], q[f][(long)st[f] * al], v);
+    v *= a == 0 ? inv_eig(la[al], lb, lc, sigma)
+                : (a == 1 ? inv_eig(lb, la[al], lc, sigma) : inv_eig(lb, lc, la[al], sigma));
+    s0 = fma(w0[al], v, s0);
+    s1 = fma(w1[al], v, s1);
   }
   red[0][w][lane] = s0;
   red[1][w][lane] = s1;

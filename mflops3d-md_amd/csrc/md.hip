@@ -171,6 +171,14 @@ __global__ void __launch_bounds__(256) axpby_kernel(double a, const double *x, d
   if (t < n) y[t] = fma(a, x[t], b * y[t]);
 }
 
+// v /= sqrt(n2) unless it is zero (n2: device scalar)
+__global__ void __launch_bounds__(256) normalise_kernel(double *v, long n,
+                                                        const double *__restrict__ n2) {
+  const long t = (long)blockIdx.x * 256 + threadIdx.x;
+  const double hn = sqrt(n2[0]);
+  if (t < n && hn > 0.0) v[t] *= 1.0 / hn;
+}
+
 // x += sum_j V[:, j] c[j]
 __global__ void __launch_bounds__(256) update_kernel(const double *__restrict__ V, long n, int k,
                                                      const double *__restrict__ c,
@@ -296,9 +304,10 @@ struct mf_md {
   int2 *atile[4] = {nullptr, nullptr, nullptr, nullptr};
   int atiles[4] = {0, 0, 0, 0};
   mf::ApplyRole *arole = nullptr;
-  int aroles = 0, ablocks = 0;
+  int aroles = 0, ablocks = 0, anf = 0;  // anf: the most interface faces of a subdomain
   double *ws = nullptr;    // GMRES and GEMV workspace
   size_t ws_doubles = 0;
+  double *hpin = nullptr;  // pinned: the scalars a GMRES iteration reads back
   int restart = 30;
   // initial-guess history (md_solve with inf_sol, class_md.f90:389-400,
   // 419-424): the last three interface solutions, oldest first
@@ -324,6 +333,7 @@ struct mf_md {
     if (pb) (void)hipFree(pb);
     if (apply) (void)hipFree(apply);
     if (ws) (void)hipFree(ws);
+    if (hpin) (void)hipHostFree(hpin);
     if (hist) (void)hipFree(hist);
     if (ones) (void)hipFree(ones);
   }
@@ -364,7 +374,7 @@ Ws carve(mf_md *h) {
   w.x = p; p += h->ninf;
   w.r = p; p += h->ninf;
   w.dpart = p; p += 256 * m1;
-  w.hcol = p; p += 2 * m1;
+  w.hcol = p; p += 2 * m1 + 2;
   w.t1 = p; p += h->nloc;
   w.xh = p; p += h->nloc;
   w.nchunk_max = 0;
@@ -375,7 +385,7 @@ size_t ws_size(const mf_md *h) {
   const long m1 = h->restart + 1;
   long pmax = 0;
   for (auto &s : h->subs) pmax = std::max(pmax, ((s.u + 511) / 512) * s.u);
-  return 4 * (size_t)h->nloc + pmax + (size_t)h->ninf * m1 + 3 * (size_t)h->ninf + 256 * m1 + 2 * m1;
+  return 4 * (size_t)h->nloc + pmax + (size_t)h->ninf * m1 + 3 * (size_t)h->ninf + 256 * m1 + 2 * m1 + 2;
 }
 
 // y = M x (device vectors of ninf)
@@ -410,8 +420,14 @@ int apply_op(mf_md *h, const Ws &w, const double *x, double *y, hipStream_t st) 
   hipLaunchKernelGGL((mf::apply_gemm_kernel<false, false>), grid(1), dim3(256), 0, st,
                      (const mf::ApplyProblem *)h->ap[1], (const int2 *)h->atile[1], h->atiles[1],
                      (const double *)w.t1, none, w.xh, none);
-  hipLaunchKernelGGL(mf::apply_sum_kernel, dim3(h->ablocks, h->aroles), dim3(64, mf::APPLY_SPLIT), 0,
-                     st, (const mf::ApplyRole *)h->arole, (const double *)w.xh, w.t1, h->sigma);
+  auto sum = [&](auto nf) {
+    hipLaunchKernelGGL((mf::apply_sum_kernel<decltype(nf)::value>), dim3(h->ablocks, h->aroles),
+                       dim3(64, mf::APPLY_SPLIT), 0, st, (const mf::ApplyRole *)h->arole,
+                       (const double *)w.xh, w.t1, h->sigma);
+  };
+  if (h->anf <= 2) sum(std::integral_constant<int, 2>());
+  else if (h->anf <= 4) sum(std::integral_constant<int, 4>());
+  else sum(std::integral_constant<int, 6>());
   hipLaunchKernelGGL((mf::apply_gemm_kernel<true, false>), grid(2), dim3(256), 0, st,
                      (const mf::ApplyProblem *)h->ap[2], (const int2 *)h->atile[2], h->atiles[2],
                      none, (const double *)w.t1, w.xh, none);
@@ -451,6 +467,7 @@ int apply_setup(mf_md *h) {
     std::memset(&base, 0, sizeof(base));
     for (int q = 0; q < 3; ++q) { base.n[q] = A.n[q]; base.lam[q] = A.lam[q]; }
     base.nf = s.nf;
+    h->anf = std::max(h->anf, s.nf);
     long xof[6];  // each face's unknowns in x
     for (int f = 0; f < s.nf; ++f) {
       base.fax[f] = s.face[f] / 2;
@@ -549,8 +566,20 @@ int dots(mf_md *h, const Ws &w, const double *V, int k, const double *v, double 
   hipLaunchKernelGGL(mf::md::dots_sum_kernel, dim3(k), dim3(256), 0, st, (const double *)w.dpart, nb,
                      w.hcol);
   MDCHK(hipGetLastError());
-  MDCHK(hipMemcpyAsync(out, w.hcol, k * sizeof(double), hipMemcpyDeviceToHost, st));
+  MDCHK(hipMemcpyAsync(h->hpin, w.hcol, k * sizeof(double), hipMemcpyDeviceToHost, st));
   MDCHK(hipStreamSynchronize(st));
+  std::memcpy(out, h->hpin, k * sizeof(double));
+  return MF_OK;
+}
+
+// the same, left on the device in out (k doubles)
+int dots_dev(mf_md *h, const Ws &w, const double *V, int k, const double *v, double *out,
+             hipStream_t st) {
+  const int nb = 256;
+  hipLaunchKernelGGL(mf::md::dots_part_kernel, dim3(nb, k), dim3(256), 0, st, V, h->ninf, v, w.dpart);
+  hipLaunchKernelGGL(mf::md::dots_sum_kernel, dim3(k), dim3(256), 0, st, (const double *)w.dpart, nb,
+                     out);
+  MDCHK(hipGetLastError());
   return MF_OK;
 }
 
@@ -724,6 +753,9 @@ int md_create(const int nd[3], const int *npts, const double *grids, const int b
   if (e == hipSuccess && h->ninf) e = hipMalloc(&h->pb, h->ninf * sizeof(long));
   h->ws_doubles = ws_size(h);
   if (e == hipSuccess) e = hipMalloc(&h->ws, h->ws_doubles * sizeof(double));
+  if (e == hipSuccess)
+    e = hipHostMalloc((void **)&h->hpin, (2 * (size_t)h->restart + 4) * sizeof(double),
+                      hipHostMallocDefault);
   if (e == hipSuccess && h->nloc) e = hipMemcpy(h->map, hmap.data(), h->nloc * sizeof(long), hipMemcpyHostToDevice);
   if (e == hipSuccess && h->ninf) e = hipMemcpy(h->pa, hpa.data(), h->ninf * sizeof(long), hipMemcpyHostToDevice);
   if (e == hipSuccess && h->ninf) e = hipMemcpy(h->pb, hpb.data(), h->ninf * sizeof(long), hipMemcpyHostToDevice);
@@ -939,7 +971,7 @@ extern "C" int mf_md_solve(mf_md *h, const double *const *g, double *const *u,
   const int m = h->restart;
   double *b = w.r;  // the right-hand side, kept
   double *V = w.V;
-  std::vector<double> H((m + 1) * m), cs(m), sn(m), gv(m + 1), hc(m + 1), hc2(m + 1);
+  std::vector<double> H((m + 1) * m), cs(m), sn(m), gv(m + 1), hc(m + 1);
   int iters = 0;
   double rel = bnorm > 0.0 ? 1.0 : 0.0;
   bool done = bnorm == 0.0;
@@ -966,18 +998,25 @@ extern "C" int mf_md_solve(mf_md *h, const double *const *g, double *const *u,
       double *vk1 = V + (long)(k + 1) * n;
       MDRC(apply_op(h, w, V + (long)k * n, vk1, st));
       if (nullsp) MDRC(remove_constant(h, w, vk1, st));
-      // classical Gram-Schmidt, applied twice
+      // classical Gram-Schmidt, applied twice, then the norm and the scaling,
+      // all on the device: the coefficients of both passes and the squared
+      // norm come to the host together, one wait per iteration
       for (int pass = 0; pass < 2; ++pass) {
-        double *hh = pass ? hc2.data() : hc.data();
-        MDRC(dots(h, w, V, k + 1, vk1, hh, st));
-        MDCHK(hipMemcpyAsync(w.hcol, hh, (k + 1) * sizeof(double), hipMemcpyHostToDevice, st));
+        double *hd = w.hcol + pass * (k + 1);
+        MDRC(dots_dev(h, w, V, k + 1, vk1, hd, st));
         hipLaunchKernelGGL(mf::md::orth_kernel, dim3(mf::md::nblk(n)), dim3(256), 0, st,
-                           (const double *)V, n, k + 1, (const double *)w.hcol, vk1);
+                           (const double *)V, n, k + 1, (const double *)hd, vk1);
       }
-      for (int j = 0; j <= k; ++j) hc[j] += hc2[j];
-      double hn2 = 0.0;
-      MDRC(dots(h, w, vk1, 1, vk1, &hn2, st));
-      const double hn = std::sqrt(hn2);
+      double *hn2d = w.hcol + 2 * (k + 1);
+      MDRC(dots_dev(h, w, vk1, 1, vk1, hn2d, st));
+      hipLaunchKernelGGL(mf::md::normalise_kernel, dim3(mf::md::nblk(n)), dim3(256), 0, st, vk1, n,
+                         (const double *)hn2d);
+      MDCHK(hipGetLastError());
+      MDCHK(hipMemcpyAsync(h->hpin, w.hcol, (2 * (k + 1) + 1) * sizeof(double), hipMemcpyDeviceToHost,
+                           st));
+      MDCHK(hipStreamSynchronize(st));
+      for (int j = 0; j <= k; ++j) hc[j] = h->hpin[j] + h->hpin[k + 1 + j];
+      const double hn = std::sqrt(h->hpin[2 * (k + 1)]);
       ++iters;
       // Givens rotations on column k
       for (int j = 0; j < k; ++j) {
@@ -994,9 +1033,6 @@ extern "C" int mf_md_solve(mf_md *h, const double *const *g, double *const *u,
       gv[k] = cs[k] * gv[k];
       for (int j = 0; j <= k; ++j) H[j + (size_t)(m + 1) * k] = hc[j];
       rel = std::fabs(gv[k + 1]) / bnorm;
-      if (hn > 0.0)
-        hipLaunchKernelGGL(mf::md::axpby_kernel, dim3(mf::md::nblk(n)), dim3(256), 0, st, 0.0,
-                           (const double *)vk1, 1.0 / hn, vk1, n);
       if (rel <= tol || hn == 0.0) { ++k; break; }
     }
     // x += V y, H y = g (upper triangular k x k)
