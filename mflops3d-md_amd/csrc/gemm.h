@@ -64,7 +64,9 @@ __device__ __forceinline__ double inv_eig(double lx, double ly, double lz, doubl
   return big < 1e-11 ? 0.0 : 1.0 / (((lx + ly) + lz) + sigma);
 }
 
-enum EpiMode { EPI_STORE = 0, EPI_DIVIDE = 1, EPI_SCATTER = 2, EPI_SCATTER_ADD = 3 };
+enum EpiMode {
+  EPI_STORE = 0, EPI_DIVIDE = 1, EPI_SCATTER = 2, EPI_SCATTER_ADD = 3, EPI_FIELDS = 4, EPI_TAU = 5
+};
 
 struct EpiArgs {
   // EPI_DIVIDE: m = i1 + n1*i2, n = i3 -> value / (lx[i1]+ly[i2]+lz[i3]+sigma),
@@ -75,6 +77,14 @@ struct EpiArgs {
   // EPI_SCATTER(_ADD): m = i, n = j + n2*k -> u[(i+1) + nx((j+1) + ny(k+1))]
   double *u;
   int nx, ny;
+  // EPI_FIELDS: batch b -> out[b] instead of C + sC b.  EPI_TAU: batch b is the
+  // filtered product of fields p and q, point t = m + ldc n:
+  // tau[6 t + col[b]] = (value - p[b][t] q[b][t]) inv
+  double *out[3];
+  const double *p[3], *q[3];
+  float *tau;
+  int col[3];
+  double inv;
 };
 
 // The products of one tile of C = A B, rows from m0 and columns from n0, by one
@@ -179,6 +189,7 @@ __global__ void __launch_bounds__(256, 2)
   const int m0 = im * 16 * MI, n0 = in * 16 * NI;
   A += (long)ib * sA;
   if (EPI == EPI_STORE || EPI == EPI_DIVIDE) C += (long)ib * sC;
+  if (EPI == EPI_FIELDS) C = (TC *)ep.out[ib];
 
   acc_t acc[MI][NI];
   gemm_tile<T, MI, NI, D, KB>(A, lda, B, ldb, M, N, K, m0, n0, acc);
@@ -220,8 +231,11 @@ __global__ void __launch_bounds__(256, 2)
         const int n = n0 + dn;
         if (n >= N) continue;
         const double v = (double)acc[mi][ni][r];
-        if (EPI == EPI_STORE) {
+        if (EPI == EPI_STORE || EPI == EPI_FIELDS) {
           C[m + ldc * n] = (TC)v;
+        } else if (EPI == EPI_TAU) {
+          const long t = m + ldc * n;
+          ep.tau[6 * t + ep.col[ib]] = (float)((v - ep.p[ib][t] * ep.q[ib][t]) * ep.inv);
         } else if (EPI == EPI_DIVIDE) {
           const double lzn = ep.lz[n];
           const double big = fmax(fmax(fabs(ep.sigma), big_xy), fabs(lzn));

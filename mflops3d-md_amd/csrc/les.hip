@@ -141,20 +141,95 @@ __global__ void __launch_bounds__(256) les_nu_kernel(NuArgs a) {
 inline unsigned nblk(long n) { return (unsigned)((n + 255) / 256); }
 
 // ---- learned-closure data path ----
-__global__ void __launch_bounds__(256) prod_kernel(const double *__restrict__ a,
-                                                   const double *__restrict__ b,
-                                                   double *__restrict__ o, long N) {
-  const long t = (long)blockIdx.x * 256 + threadIdx.x;
-  if (t < N) o[t] = a[t] * b[t];
-}
-
-// T[t][col] = (F(u_i u_j) - F(u_i) F(u_j)) / tscale
-__global__ void __launch_bounds__(256) tau_kernel(const double *__restrict__ uu,
-                                                  const double *__restrict__ ui,
-                                                  const double *__restrict__ uj,
-                                                  float *__restrict__ T, int col, double inv, long N) {
-  const long t = (long)blockIdx.x * 256 + threadIdx.x;
-  if (t < N) T[t * O + col] = (float)((uu[t] - ui[t] * uj[t]) * inv);
+// The x pass of three filtered fields at once: w1_f = F B_f for the fields
+// (G = 0) u, v, w, (1) uu, uv, uw or (2) vv, vw, ww, formed from u, v, w as
+// they are loaded; or of one field, (3) u or (4) uv.  One wave takes 16 MI filtered points of 16 columns, three
+// accumulators deep: the matrix's operands serve all three fields, and no
+// product field is written.  Bounded by the FP64 matrix rate (24 MFMAs of 64
+// cycles on 10 loads per step at 64 points); 256^3 -> 64^3 with its y and z
+// passes 1.26 -> 0.62 ms for all nine fields (a pass over memory per product,
+// and a GEMM of its own for each field and axis, before).
+constexpr int FX_D = 4;  // k-steps in flight
+template <int G, int MI>
+__global__ void __launch_bounds__(256, 2)
+    filter_x_kernel(const double *__restrict__ F, int M, const double *__restrict__ u,
+                    const double *__restrict__ v, const double *__restrict__ w, long N, int K,
+                    double *__restrict__ out, int tm, long waves) {
+  typedef Mfma<double>::acc_t acc_t;
+  constexpr int NL = G < 2 ? 3 : (G == 3 ? 1 : 2), NF = G < 3 ? 3 : 1;
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const long wv = (long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (wv >= waves) return;
+  const int m0 = (int)(wv % tm) * 16 * MI;
+  const long n0 = (wv / tm) * 16, nc = min(n0 + c, N - 1);
+  // operands at k = 4 s + g of step s; lanes past K in the last step repeat
+  // k = K - 1 and are zeroed (as gemm_tile)
+  const int KS = (K + 3) / 4;
+  const int over = max(0, 4 * (KS - 1) + g - (K - 1));
+  const int g0 = KS == 1 ? g - over : g;
+  const double *pa[MI], *pb[NL];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) pa[i] = F + min(m0 + 16 * i + c, M - 1) + (long)M * g0;
+  pb[0] = (G == 2 ? v : u) + (long)K * nc + g0;
+  if (NL > 1) pb[NL > 1 ? 1 : 0] = (G == 2 ? w : v) + (long)K * nc + g0;
+  if (NL > 2) pb[NL - 1] = w + (long)K * nc + g0;
+  double af[FX_D][MI], q[FX_D][NL];
+  auto fetch = [&](int d, int s) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) af[d][i] = *pa[i];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) q[d][i] = *pb[i];
+    const int st = s + 2 > KS ? 0 : (s + 2 == KS ? 4 - over : 4);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) pa[i] += (long)st * M;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) pb[i] += st;
+  };
+  acc_t acc[NF][MI];
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int i = 0; i < MI; ++i) acc[f][i] = (acc_t){0, 0, 0, 0};
+  auto mma = [&](int d, int s) {
+    if (s + 1 == KS && over > 0) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i) af[d][i] = 0.0;
+#pragma unroll
+      for (int i = 0; i < NL; ++i) q[d][i] = 0.0;
+    }
+    const double x = q[d][0], y = q[d][NL > 1 ? 1 : 0], z = q[d][NL - 1];
+    const double b[3] = {G == 0 || G == 3 ? x : (G == 4 ? x * y : x * x),
+                         G == 0 ? y : x * y, G == 0 ? z : (G == 1 ? x * z : y * y)};
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int i = 0; i < MI; ++i) acc[f][i] = Mfma<double>::op(b[f], af[d][i], acc[f][i]);
+  };
+#pragma unroll
+  for (int d = 0; d < FX_D; ++d) fetch(d, d);
+  int s = 0;
+  for (; s + FX_D < KS; s += FX_D) {
+#pragma unroll
+    for (int d = 0; d < FX_D; ++d) {
+      mma(d, s + d);
+      fetch(d, s + d + FX_D);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < FX_D; ++d)
+    if (s + d < KS) mma(d, s + d);
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int m = m0 + 16 * i + c;
+    if (m >= M) continue;
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const long n = n0 + Mfma<double>::row(lane, r);
+        if (n < N) out[(long)M * N * f + m + (long)M * n] = acc[f][i][r];
+      }
+  }
 }
 
 struct FeatArgs {
@@ -729,24 +804,82 @@ extern "C" int mf_sgs_targets(const mf_filter *fx, const mf_filter *fy, const mf
     return mf::fail(MF_ERR_ARG, "mf_sgs_targets: null pointer");
   if (!(tscale > 0.0)) return mf::fail(MF_ERR_ARG, "mf_sgs_targets: tscale must be positive");
   hipStream_t st = (hipStream_t)stream;
-  const long Nf = (long)fx->nin * fy->nin * fz->nin;
-  const long Nc = (long)fx->nout * fy->nout * fz->nout;
-  double *prod = work, *fb = work + Nf;
-  double *fw = fb + Nc;  // filter work
+  const int nxi = fx->nin, nyi = fy->nin, nzi = fz->nin;
+  const int nxo = fx->nout, nyo = fy->nout, nzo = fz->nout;
+  const long Nf = (long)nxi * nyi * nzi, Nc = (long)nxo * nyo * nzo;
+  const long n1 = (long)nxo * nyi * nzi, n2 = (long)nxo * nyo * nzi;
+  // Three groups of three fields: u v w (the filtered velocity), uu uv uw and
+  // vv vw ww (the stresses xx xy xz and yy yz zz).  The x pass leaves a group's
+  // fields one after the other, so that y and z take each as a batch; work
+  // holds them where 3 (n1 + n2) fits it (filters to about 2/5 of the points and
+  // fewer); else they are taken one at a time.
+  const int pi[9] = {0, 1, 2, 0, 0, 0, 1, 1, 2}, pj[9] = {-1, -1, -1, 0, 1, 2, 1, 2, 2};
+  const int cols[6] = {0, 3, 4, 1, 5, 2};
   const double *q[3] = {u, v, w};
   double *qb[3] = {ubar, vbar, wbar};
-  for (int c = 0; c < 3; ++c) {
-    int rc = mf_filter3d(fx, fy, fz, q[c], qb[c], fw, st);
-    if (rc != MF_OK) return rc;
-  }
-  const int pi[6] = {0, 1, 2, 0, 0, 1}, pj[6] = {0, 1, 2, 1, 2, 2};
-  for (int col = 0; col < 6; ++col) {
-    hipLaunchKernelGGL(prod_kernel, dim3(nblk(Nf)), dim3(256), 0, st, q[pi[col]], q[pj[col]], prod, Nf);
-    int rc = mf_filter3d(fx, fy, fz, prod, fb, fw, st);
-    if (rc != MF_OK) return rc;
-    hipLaunchKernelGGL(tau_kernel, dim3(nblk(Nc)), dim3(256), 0, st, (const double *)fb,
-                       (const double *)qb[pi[col]], (const double *)qb[pj[col]], tau, col,
-                       1.0 / tscale, Nc);
+  mf::EpiArgs ep;
+  std::memset(&ep, 0, sizeof(ep));
+  ep.tau = tau;
+  ep.inv = 1.0 / tscale;
+  for (int c = 0; c < 3; ++c) ep.out[c] = qb[c];
+  const long N = (long)nyi * nzi;
+  const bool grouped = 3 * (n1 + n2) <= Nf + Nc + n1 + n2;
+  double *w1 = work, *w2 = work + (grouped ? 3 : 1) * n1;
+  auto yz = [&](int first, int nf) {
+    // y: w2_k (nxo, nyo) = w1_k Fy^T over z and the fields
+    mf::gemm_launch<double, double, false, mf::EPI_STORE>(
+        (const double *)w1, nxo, (long)nxo * nyi, (const double *)fy->dF, nyo, w2, nxo,
+        (long)nxo * nyo, nxo, nyo, nyi, nzi * nf, ep, fx->ncu, st);
+    for (int b = 0; b < nf; ++b) {
+      const int f = first + b;
+      ep.out[b] = f < 3 ? qb[f] : nullptr;
+      if (f >= 3) {
+        ep.p[b] = qb[pi[f]];
+        ep.q[b] = qb[pj[f]];
+        ep.col[b] = cols[f - 3];
+      }
+    }
+    // z: (nxo nyo, nzo) = w2 Fz^T over the fields, into the filtered velocity
+    // or, with its products taken off, the stresses
+    const long m = (long)nxo * nyo;
+    if (first < 3)
+      mf::gemm_launch<double, double, false, mf::EPI_FIELDS>(
+          (const double *)w2, m, n2, (const double *)fz->dF, nzo, (double *)nullptr, m, 0, (int)m, nzo,
+          nzi, nf, ep, fx->ncu, st);
+    else
+      mf::gemm_launch<double, double, false, mf::EPI_TAU>(
+          (const double *)w2, m, n2, (const double *)fz->dF, nzo, (double *)nullptr, m, 0, (int)m, nzo,
+          nzi, nf, ep, fx->ncu, st);
+  };
+  // rows of the x pass's tiles: the widest that pads the filtered points least
+  int mi = 4;
+  for (int t = 3; t >= 1; --t)
+    if ((nxo + 16 * t - 1) / (16 * t) * t < (nxo + 16 * mi - 1) / (16 * mi) * mi) mi = t;
+  const int tm = (nxo + 16 * mi - 1) / (16 * mi);
+  const long waves = (N + 15) / 16 * tm;
+  const double *a0 = nullptr, *a1 = nullptr, *a2 = nullptr;
+  auto xpass = [&](auto gg, auto mm) {
+    hipLaunchKernelGGL((filter_x_kernel<decltype(gg)::value, decltype(mm)::value>),
+                       dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, (const double *)fx->dF, nxo,
+                       a0, a1, a2, N, nxi, w1, tm, waves);
+  };
+  auto group = [&](auto gg, const double *f0, const double *f1, const double *f2, int first, int nf) {
+    a0 = f0; a1 = f1; a2 = f2;
+    if (mi == 4) xpass(gg, std::integral_constant<int, 4>());
+    else if (mi == 3) xpass(gg, std::integral_constant<int, 3>());
+    else if (mi == 2) xpass(gg, std::integral_constant<int, 2>());
+    else xpass(gg, std::integral_constant<int, 1>());
+    yz(first, nf);
+  };
+  if (grouped) {
+    group(std::integral_constant<int, 0>(), u, v, w, 0, 3);
+    group(std::integral_constant<int, 1>(), u, v, w, 3, 3);
+    group(std::integral_constant<int, 2>(), u, v, w, 6, 3);
+  } else {
+    for (int f = 0; f < 3; ++f)
+      group(std::integral_constant<int, 3>(), q[f], nullptr, nullptr, f, 1);
+    for (int f = 3; f < 9; ++f)
+      group(std::integral_constant<int, 4>(), q[pi[f]], q[pj[f]], nullptr, f, 1);
   }
   LESCHK(hipGetLastError());
   return MF_OK;

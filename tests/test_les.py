@@ -494,6 +494,27 @@ def test_oracle_eddy_targets_project_to_smagorinsky():
     assert np.abs(nu0).max() == 0.0
 
 
+# three fields per pass (64- and 16-row tiles, with a remainder) and, where the
+# workspace does not hold three, one field at a time (48- and 16-row tiles)
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape_in,shape_out", [((200, 24, 18), (64, 9, 8)), ((61, 22, 19), (17, 8, 6)),
+                                                ((70, 40, 33), (33, 15, 12)), ((30, 20, 22), (14, 9, 10))])
+def test_gpu_sgs_targets_groups(shape_in, shape_out):
+    mf, torch = _mf()
+    Fs, axes = _filters(shape_in, shape_out, tuple(max(5, n - 2) for n in shape_out))
+    fs = [mf.SplineFilter(*a, 3) for a in axes]
+    rng = np.random.default_rng(sum(shape_in))
+    q = [rng.standard_normal(shape_in) for _ in range(3)]
+    print("run sgs targets %s -> %s" % (shape_in, shape_out), flush=True)
+    bars, tau = mf.sgs_targets(*fs, *[mf.to_device(a) for a in q], tscale=0.5)
+    qb, tref = L.sgs_targets(*Fs, *q, tscale=0.5)
+    for a, b in zip(bars, qb):
+        assert np.abs(mf.to_host(a) - b).max() < 1e-12 * np.abs(b).max()
+    tau = tau.cpu().numpy()
+    for c in range(6):
+        assert np.abs(tau[:, c] - tref[:, c]).max() < 1e-6 * np.abs(tref).max(), c
+
+
 @pytest.mark.gpu
 def test_gpu_eddy_targets_match_oracle():
     mf, torch = _mf()
