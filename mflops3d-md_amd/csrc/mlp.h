@@ -14,7 +14,7 @@
 // cycles per 16 samples with the padding), 15 000 with the gradient (268), on
 // 154 TFLOP/s of measured FP32 matrix rate, beside 128 tanhf per sample on
 // the vector units; the input and output rows are 64 B per sample.  Measured
-// at 1 045 568 samples: loss and gradient 0.47 ms (9.96 ms with one sample per
+// at 1 045 568 samples: loss and gradient 0.44 ms (9.96 ms with one sample per
 // lane on vector FMAs, 64-sample partials in memory and a serial sum of them).
 #pragma once
 #include <hip/hip_runtime.h>
@@ -144,7 +144,9 @@ __global__ void __launch_bounds__(64 * MLP_WAVES, 2)
 // gradient (24 FP32 accumulators per lane), and each tile's FP32 sums are
 // added into FP64 ones, as many samples per FP32 sum as the tile has.  Three
 // LDS buffers (dh1 reuses h2's) let two blocks share a CU: one's tanhf and
-// barriers run beside the other's MFMAs.
+// barriers run beside the other's MFMAs.  W2 lies in LDS once, widened: as two
+// bf16 copies (one transposed) every operand had to be widened in each tile,
+// which took 0.03 of 0.47 ms.
 constexpr int MLP_PITCH = MLP_TILE + 4;
 constexpr int MLP_WP = H + 8;  // bf16 pitch of the weight matrices in LDS
 
@@ -155,15 +157,12 @@ __global__ void __launch_bounds__(64 * MLP_WAVES, 2)
   __shared__ float S[3][H][MLP_PITCH];             // h2 then dh1 | dh2 | h1
   __shared__ float SX[I0 + 1][MLP_PITCH];          // inputs and a row of ones
   __shared__ float SD[O][MLP_PITCH];               // dY
-  __shared__ unsigned short W2[H][MLP_WP], W2t[H][MLP_WP], W3[O][MLP_WP], W3t[H][8];
+  __shared__ float W2[H][MLP_PITCH];               // widened; rows forward, columns backward
+  __shared__ unsigned short W3[O][MLP_WP], W3t[H][8];
   __shared__ float B2[H];
   const int tid = threadIdx.x, l = tid & 63, c = l & 15, g = l >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  for (int t = tid; t < NW2; t += 64 * MLP_WAVES) {
-    const unsigned short v = wb[NW1 + t];
-    W2[t / H][t % H] = v;
-    W2t[t % H][t / H] = v;
-  }
+  for (int t = tid; t < NW2; t += 64 * MLP_WAVES) W2[t / H][t % H] = bf2f(wb[NW1 + t]);
   for (int t = tid; t < NW3; t += 64 * MLP_WAVES) W3[t / H][t % H] = wb[NW1 + NW2 + t];
   for (int t = tid; t < 8 * H; t += 64 * MLP_WAVES)
     W3t[t / 8][t % 8] = t % 8 < O ? wb[NW1 + NW2 + (t % 8) * H + t / 8] : (unsigned short)0;
@@ -206,7 +205,7 @@ __global__ void __launch_bounds__(64 * MLP_WAVES, 2)
     for (int kb = 0; kb < 4; ++kb) {
       mlp_f4 a[4];
 #pragma unroll
-      for (int ib = 0; ib < 4; ++ib) a[ib] = mlp_widen4(&W2[16 * ib + c][16 * kb + 4 * g]);
+      for (int ib = 0; ib < 4; ++ib) a[ib] = *(const mlp_f4 *)&W2[16 * ib + c][16 * kb + 4 * g];
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -271,7 +270,9 @@ __global__ void __launch_bounds__(64 * MLP_WAVES, 2)
     for (int kb = 0; kb < 4; ++kb) {
       mlp_f4 a[4];
 #pragma unroll
-      for (int ib = 0; ib < 4; ++ib) a[ib] = mlp_widen4(&W2t[16 * ib + c][16 * kb + 4 * g]);
+      for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) a[ib][r] = W2[16 * kb + 4 * g + r][16 * ib + c];
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
