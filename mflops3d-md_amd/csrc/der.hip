@@ -22,6 +22,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "conv.h"
 #include "der_seg.h"
 #include "internal.h"
 #include "stage.h"
@@ -281,59 +282,63 @@ __global__ void __launch_bounds__(256) der3d_kernel(FieldSet fs, int nx, int ny,
 // (full scheme), the next nb4.x .. nb4.w blocks the four families of
 // one-boundary-plane lines (sub-line scheme on points 1..n-2), and the last
 // block writes the zeros (two-boundary-plane lines, sub-line end points).
-template <int AXIS, bool TRI>
-__global__ void __launch_bounds__(64 * SEG_KMAX) der3d_seg_kernel(FieldSet fs, int nx, int ny,
-                                                                  int nz, SegTab full,
-                                                                  SegTab sub, int mode,
-                                                                  int b_full, int4 nb4,
-                                                                  int groups) {
-  extern __shared__ double lds[];
-  // The boundary-plane blocks come first: at y and z half of them read one
-  // point per cache line and take longest.  Then the full-scheme blocks, a
-  // contiguous run of them on each of the 8 XCDs that consecutive block ids go
-  // to in turn: groups of 64 lines start at any byte, so neighbours share
-  // cache lines at both ends, which then come from the XCD's own L2.
-  int blk, fld;
-  {
-    const int nf = gridDim.y, nsub = gridDim.x - b_full;
-    int bid = blockIdx.x + gridDim.x * blockIdx.y;
-    if (bid < nsub * nf) {
-      fld = bid % nf;
-      blk = b_full + bid / nf;
-    } else {
-      bid -= nsub * nf;
-      const int nb = b_full * nf, off = nsub * nf % 8;
-      // XCD of this block and its place among the XCD's full-scheme blocks
-      const int xc = (bid + off) % 8, first = (xc - off + 8) % 8, l = (bid - first) / 8;
-      int start = 0;
-      for (int q = 0; q < xc; ++q) start += (nb - (q - off + 8) % 8 + 7) / 8;
-      const int t = start + l;
-      blk = t % b_full;
-      fld = t / b_full;
-    }
+struct SegGrid {
+  int nx, ny, nz;
+  SegTab full, sub;
+  int mode, b_full;
+  int4 nb4;
+  int groups;
+};
+
+// Block and field of this block: the boundary-plane blocks come first (at y
+// and z half of them read one point per cache line and take longest), then
+// the full-scheme blocks, a contiguous run of them on each of the 8 XCDs that
+// consecutive block ids go to in turn: groups of lines start at any byte, so
+// neighbours share cache lines at both ends, which then come from the XCD's
+// own L2.  inner: fields next to each other rather than one after the other.
+__device__ __forceinline__ void seg_place(const SegGrid &G, bool inner, int &blk, int &fld) {
+  const int nf = gridDim.y, nsub = gridDim.x - G.b_full;
+  int bid = blockIdx.x + gridDim.x * blockIdx.y;
+  if (bid < nsub * nf) {
+    fld = bid % nf;
+    blk = G.b_full + bid / nf;
+    return;
   }
-  const double *__restrict__ x = fs.x[fld];
-  double *__restrict__ out = fs.out[fld];
+  bid -= nsub * nf;
+  const int nb = G.b_full * nf, off = nsub * nf % 8;
+  // XCD of this block and its place among the XCD's full-scheme blocks
+  const int xc = (bid + off) % 8, first = (xc - off + 8) % 8, l = (bid - first) / 8;
+  int start = 0;
+  for (int q = 0; q < xc; ++q) start += (nb - (q - off + 8) % 8 + 7) / 8;
+  const int t = start + l;
+  blk = inner ? t / nf : t % G.b_full;
+  fld = inner ? t % nf : t / G.b_full;
+}
+
+template <int AXIS, bool TRI, class Job>
+__device__ __forceinline__ void seg_block(const Job &job, const SegGrid &G, int blk, double *lds) {
+  const int nx = G.nx, ny = G.ny, nz = G.nz;
+  const int4 nb4 = G.nb4;
   int na, nb;
   long s, sa, sb;
   if (AXIS == 0) { na = ny; nb = nz; s = 1; sa = nx; sb = (long)nx * ny; }
   else if (AXIS == 1) { na = nx; nb = nz; s = nx; sa = 1; sb = (long)nx * ny; }
   else { na = nx; nb = ny; s = (long)nx * ny; sa = 1; sb = nx; }
-  const int n = full.n;
+  const int n = G.full.n;
   SegLines L;
   L.sa = sa; L.sb = sb; L.s = s;
   // one call site of seg_solve: pick the scheme, the line family and the
   // field offset of this block, then solve
-  SegTab T = full;
+  SegTab T = G.full;
   long off = 0;
   bool solve = true;
   L.groups = 0;
-  if (blk < b_full) {
-    L.groups = groups;
-    if (mode) { L.a0 = 1; L.na = na - 2; L.b0 = 1; L.nb = nb - 2; }
+  if (blk < G.b_full) {
+    L.groups = G.groups;
+    if (G.mode) { L.a0 = 1; L.na = na - 2; L.b0 = 1; L.nb = nb - 2; }
     else { L.a0 = 0; L.na = na; L.b0 = 0; L.nb = nb; }
   } else {
-    blk -= b_full;
+    blk -= G.b_full;
     if (blk < nb4.x + nb4.y) {
       const int f = blk >= nb4.x;
       blk -= f ? nb4.x : 0;
@@ -346,19 +351,19 @@ __global__ void __launch_bounds__(64 * SEG_KMAX) der3d_seg_kernel(FieldSet fs, i
     } else {
       solve = false;
     }
-    T = sub;
+    T = G.sub;
     off = s;  // the sub-line scheme acts on points 1..n-2
   }
   if (solve) {
     L.nlines = L.na * L.nb;
-    seg_solve<TRI, AXIS == 0>(x + off, out + off, T, L, blk, lds);
+    seg_solve<TRI, AXIS == 0>(job, off, T, L, blk, lds);
     return;
   }
   // zeros: the four two-boundary-plane lines and both ends of the sub lines
   const int nt = blockDim.x;
   for (long t = threadIdx.x; t < 4L * n; t += nt) {
     const int line = (int)(t / n), i = (int)(t % n);
-    out[((line & 1) ? na - 1 : 0) * sa + (long)((line & 2) ? nb - 1 : 0) * sb + (long)i * s] = 0.0;
+    job.edge(((line & 1) ? na - 1 : 0) * sa + (long)((line & 2) ? nb - 1 : 0) * sb + (long)i * s);
   }
   const long ns = 2L * (na - 2) + 2L * (nb - 2);
   for (long t = threadIdx.x; t < ns; t += nt) {
@@ -366,9 +371,40 @@ __global__ void __launch_bounds__(64 * SEG_KMAX) der3d_seg_kernel(FieldSet fs, i
     if (t < 2L * (na - 2)) { a = 1 + (int)(t % (na - 2)); b = (t / (na - 2)) ? nb - 1 : 0; }
     else { const long r = t - 2L * (na - 2); b = 1 + (int)(r % (nb - 2)); a = (r / (nb - 2)) ? na - 1 : 0; }
     const long base = a * sa + b * sb;
-    out[base] = 0.0;
-    out[base + (long)(n - 1) * s] = 0.0;
+    job.edge(base);
+    job.edge(base + (long)(n - 1) * s);
   }
+}
+
+template <int AXIS, bool TRI>
+__global__ void __launch_bounds__(64 * SEG_KMAX) der3d_seg_kernel(FieldSet fs, SegGrid G) {
+  extern __shared__ double lds[];
+  int blk, fld;
+  seg_place(G, false, blk, fld);
+  const SegDer job{fs.x[fld], fs.out[fld]};
+  seg_block<AXIS, TRI>(job, G, blk, lds);
+}
+
+// One axis of the convective term of all components (SegConv): 32 lines of one
+// component per block, blocks of the three components of the same lines next to
+// each other (the advecting component they share then comes from the L2).
+// Bounds: HBM, 6 fields on the first axis and 9 on the others (stored products
+// and derivatives take 78 in all, with their kernels and the sum's), and on
+// the first, where the lines are contiguous, the waves' own latencies: 2 blocks
+// fill a CU's registers.  192 x 256 x 192: 246 + 193 + 204 us (1.8, 3.5 and
+// 3.3 TB/s), where products, 18 derivatives and the sum with the right-hand
+// sides took 1330, and right-hand sides on their own now take 207; a time
+// step 4.09 -> 3.53 ms.  At 24^3 to 64^3, three launches in turn for five with
+// the middle three beside each other: 0.42 -> 0.38 and 0.44 -> 0.41 ms a step.
+// Taken back: the right-hand sides formed here on the last axis (1.06 ms for
+// that launch; the many pointers cost the registers of the solve).
+template <int AXIS, bool TRI>
+__global__ void __launch_bounds__(64 * SEG_KMAX) conv3d_kernel(ConvArgs a, SegGrid G) {
+  extern __shared__ double lds[];
+  int c, blk;
+  seg_place(G, true, blk, c);
+  const SegConv<AXIS != 0> job{a.q[c], a.u, a.acc[c], a.out[c]};
+  seg_block<AXIS, TRI>(job, G, blk, lds);
 }
 
 // batched lines on segmented line solves: line l at x + l*ld, contiguous
@@ -383,7 +419,7 @@ __global__ void __launch_bounds__(64 * SEG_KMAX)
   L.a0 = 0; L.na = nlines; L.b0 = 0; L.nb = 1;
   L.nlines = nlines;
   L.groups = 0;
-  seg_solve<TRI, true>(x, out, T, L, blockIdx.x, lds);
+  seg_solve<TRI, true>(SegDer{x, out}, 0, T, L, blockIdx.x, lds);
 }
 
 // the same, one lane per line, for lines longer than the segmented solve
@@ -591,6 +627,60 @@ extern "C" int mf_der_lines(const mf_der *dc, int order, int sub, const double *
   return MF_OK;
 }
 
+namespace {
+// Blocks of `lines` lines along an axis: the grid's geometry and block count
+mf::SegGrid seg_grid(const mf_der *dc, int axis, int order, int lines, int nx, int ny, int nz,
+                     int *blocks) {
+  const int na = axis == 0 ? ny : nx, nb = axis == 2 ? ny : nz;
+  mf::SegGrid G;
+  std::memset(&G, 0, sizeof(G));
+  G.nx = nx; G.ny = ny; G.nz = nz;
+  G.full = dc->seg[order - 1][0];
+  G.sub = dc->seg[order - 1][1];
+  G.mode = dc->solver;
+  G.groups = axis != 0 && mf::seg_aligned(nx, lines) ? (nx + lines - 1) / lines : 0;
+  auto count = [&](long m) { return (int)((m + lines - 1) / lines); };
+  if (!G.mode) {
+    *blocks = G.b_full = G.groups ? G.groups * nb : count((long)na * nb);
+  } else {
+    G.b_full = G.groups ? G.groups * (nb - 2) : count((long)(na - 2) * (nb - 2));
+    G.nb4.x = G.nb4.y = count(na - 2);
+    G.nb4.z = G.nb4.w = count(nb - 2);
+    *blocks = G.b_full + G.nb4.x + G.nb4.y + G.nb4.z + G.nb4.w + 1;
+  }
+  return G;
+}
+}  // namespace
+
+namespace mf {
+bool conv3d_takes(const ::mf_der *const dc[3], int nx, int ny, int nz) {
+  for (int a = 0; a < 3; ++a)
+    if (!dc[a]->seg[0][0].pack) return false;
+  return seg_fits((long)nx * ny) && nx > 2 && ny > 2 && nz > 2;
+}
+
+int conv3d(const ::mf_der *dc, int axis, const ConvArgs &a, int nx, int ny, int nz, void *stream) {
+  const int n = axis == 0 ? nx : (axis == 1 ? ny : nz);
+  if (dc->n != n || !dc->solver) return fail(MF_ERR_ARG, "conv3d: not the handle of this axis");
+  int blocks;
+  const SegGrid G = seg_grid(dc, axis, 1, 32, nx, ny, nz, &blocks);
+  const size_t lds = seg_lds_doubles(n, axis == 0) * sizeof(double);
+  auto go = [&](auto ax, auto tri) {
+    hipLaunchKernelGGL((conv3d_kernel<decltype(ax)::value, decltype(tri)::value>), dim3(blocks, 3),
+                       dim3(64 * seg_count(n)), lds, (hipStream_t)stream, a, G);
+  };
+  auto pick = [&](auto ax) {
+    if (dc->tri[0]) go(ax, std::true_type());
+    else go(ax, std::false_type());
+  };
+  if (axis == 0) pick(std::integral_constant<int, 0>());
+  else if (axis == 1) pick(std::integral_constant<int, 1>());
+  else pick(std::integral_constant<int, 2>());
+  HIPCHK(hipGetLastError());
+  return MF_OK;
+}
+}  // namespace mf
+
 extern "C" int mf_der3d_batch(const mf_der *dc, int axis, int order, int nfields,
                               const double *const *x, double *const *out, int nx, int ny, int nz,
                               void *stream) {
@@ -623,27 +713,15 @@ extern "C" int mf_der3d_batch(const mf_der *dc, int axis, int order, int nfields
     blocks = b_full + b_sub + 1;
   }
   hipStream_t st = (hipStream_t)stream;
-  const mf::SegTab &SF = dc->seg[order - 1][0], &SS = dc->seg[order - 1][1];
-  if (SF.pack && (axis != 0 || mf::seg_fits((long)nx * ny))) {
+  if (dc->seg[order - 1][0].pack && (axis != 0 || mf::seg_fits((long)nx * ny))) {
     // segmented solves: 64 lines per block, one wavefront per segment
-    int4 nb4 = make_int4(0, 0, 0, 0);
-    int sb_full, sblocks;
-    const int groups = axis != 0 && mf::seg_aligned(nx) ? (nx + 63) / 64 : 0;
-    if (!mode) {
-      sb_full = groups ? groups * nb : (int)(((long)na * nb + 63) / 64);
-      sblocks = sb_full;
-    } else {
-      sb_full = groups ? groups * (nb - 2) : (int)(((long)(na - 2) * (nb - 2) + 63) / 64);
-      nb4.x = nb4.y = (na - 2 + 63) / 64;
-      nb4.z = nb4.w = (nb - 2 + 63) / 64;
-      sblocks = sb_full + nb4.x + nb4.y + nb4.z + nb4.w + 1;
-    }
+    int sblocks;
+    const mf::SegGrid G = seg_grid(dc, axis, order, 64, nx, ny, nz, &sblocks);
     const size_t lds = mf::seg_lds_doubles(F.n, axis == 0) * sizeof(double);
     const dim3 grid(sblocks, nfields), block(64 * mf::seg_count(F.n));
     auto go = [&](auto ax, auto tri) {
       hipLaunchKernelGGL((mf::der3d_seg_kernel<decltype(ax)::value, decltype(tri)::value>), grid,
-                         block, lds, st, fs, nx, ny, nz, SF, SS, mode, sb_full, nb4,
-                         groups);
+                         block, lds, st, fs, G);
     };
     auto pick = [&](auto ax) {
       if (dc->tri[order - 1]) go(ax, std::true_type());

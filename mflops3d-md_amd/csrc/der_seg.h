@@ -44,10 +44,12 @@
 namespace mf {
 
 constexpr int SEG_LEN = 32;     // longest segment
-// Whether the lines along y or z of a field of nx columns go in groups of 64
-// aligned in memory: rows of whole cache lines (16 points), and few lanes lost
-// at the rows' ends.
-inline bool seg_aligned(int nx) { return nx % 16 == 0 && 16 * ((nx + 63) / 64 * 64 - nx) <= 2 * nx; }
+// Whether the lines along y or z of a field of nx columns go in groups of
+// `lines` aligned in memory: rows of whole cache lines (16 points), and few
+// lanes lost at the rows' ends.
+inline bool seg_aligned(int nx, int lines) {
+  return nx % 16 == 0 && 16 * ((nx + lines - 1) / lines * lines - nx) <= 2 * nx;
+}
 
 // Contiguous lines: the wave shuffles 32-bit line offsets, so 64 lines that lie
 // `stride` points apart have to stay within 2^31 points.
@@ -114,8 +116,8 @@ struct SegLines {
   long sa, sb, s;
   int a0, na, b0, nb;
   int nlines;
-  // not 0: groups of 64 lines at a = 64 g .. 64 g + 63, this many for each b
-  // (lines outside a0 .. a0 + na - 1 are left out); 0: 64 lines in turn
+  // not 0: groups of a block's lines (64) at a = 64 g .. 64 g + 63, this many
+  // for each b (lines outside a0 .. a0 + na - 1 are left out); 0: 64 in turn
   int groups;
 };
 
@@ -134,13 +136,48 @@ __device__ __forceinline__ void seg_tile_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// What a block solves: the derivative of one field, 64 lines, one per lane ...
+struct SegDer {
+  static constexpr bool PAIR = false;
+  const double *__restrict__ x;
+  double *__restrict__ out;
+  __device__ __forceinline__ const double *in(bool) const { return x; }
+  __device__ __forceinline__ void edge(long o) const { out[o] = 0.0; }
+};
+
+// ... or one component's share of the convective term along one axis,
+//   out = acc + (u d(q) + d(q u)) / 2
+// on 32 lines: the lower half of the wave solves for d(q), the upper half for
+// d(q u).  Each half loads one of the two factors and they exchange them
+// (v_permlane32_swap); afterwards they exchange every other row, so that both
+// halves form and store results.
+template <bool ACC>
+struct SegConv {
+  static constexpr bool PAIR = true, HAS_ACC = ACC;
+  const double *__restrict__ q, *__restrict__ u, *__restrict__ acc;
+  double *__restrict__ out;
+  __device__ __forceinline__ const double *in(bool up) const { return up ? u : q; }
+  __device__ __forceinline__ void edge(long o) const { out[o] = 0.0; }
+};
+template <class Job>
+__host__ __device__ constexpr int seg_lines() { return Job::PAIR ? 32 : 64; }
+
+// a's upper half of the wave <-> b's lower half
+__device__ __forceinline__ void seg_swap(double &a, double &b) {
+  const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  a = __longlong_as_double(((long long)hi[0] << 32) | lo[0]);
+  b = __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+}
+
 // One wavefront's segment [s0, s0 + len).  LEN rows are unrolled; DYN: the
 // length is the runtime len <= LEN (rows beyond it are skipped), else len =
 // LEN.  HEAD: segment 0 (7-point rows 0 and 1, the alpha term of row 0);
 // TAIL: the last segment (7-point rows n-2 and n-1, the beta term of row n-1).
-// x0, out0: the block's first line; rel: this lane's line from there; lo, hi:
-// lanes lo .. hi - 1 have a line of their own (the others repeat one and
-// store nothing).  lds: the block's arrays; w, K: this segment
+// base: the block's first line; rel: this lane's line from there; lo, hi:
+// lines lo .. hi - 1 of the block are its own (the others repeat one and
+// are not stored).  lds: the block's arrays; w, K: this segment
 // and the count.
 // XT: contiguous lines (s = 1).  A lane's line then lies in memory away from
 // the next lane's, so the wave moves 16 rows x 64 lines at a time through
@@ -148,17 +185,30 @@ __device__ __forceinline__ void seg_tile_sync() {
 // lines (stored lane by lane, 8 bytes per line and instruction, HBM wrote
 // 1.56 x the field, and x took 85 us where y and z took 54-58 at
 // 201 x 256 x 187).
-template <int LEN, bool HEAD, bool TAIL, bool DYN, bool TRI, bool XT>
-__device__ __forceinline__ void seg_wave(const double *__restrict__ x0, double *__restrict__ out0,
-                                         long rel, int lo, int hi, long s, const SegTab &T, int w, int K,
-                                         int s0, int len, double *lds) {
+template <int LEN, bool HEAD, bool TAIL, bool DYN, bool TRI, bool XT, class Job>
+__device__ __forceinline__ void seg_wave(const Job &job, long base, long rel, int lo, int hi,
+                                         long s, const SegTab &T, int w, int K, int s0, int len,
+                                         double *lds) {
+  constexpr bool PAIR = Job::PAIR;
   const int n = T.n;
   const int lane = threadIdx.x & 63;
+  const bool up = PAIR && lane >= 32;       // this lane solves for d(q u)
+  const int line = PAIR ? lane & 31 : lane;
   typedef SegSlot<TRI> Slot;
   constexpr int CW = seg_cw(TRI);
   constexpr int NC = (LEN * CW + 63) / 64;  // register pairs of the rows
   constexpr int WD = seg_wave_doubles(XT), WB = XT ? 64 * SEG_TP : 128;
-  const double *xl = x0 + rel;
+  const double *xl = job.in(up) + base + rel;
+  // a loaded value as the solve takes it: the halves' factors become q and q u
+  auto factor = [&](double v) {
+    if constexpr (PAIR) {
+      double o = v;
+      seg_swap(v, o);
+      return up ? v * o : v;
+    } else {
+      return v;
+    }
+  };
   // exchange slots of wave j: forward Ef[j WD ..], backward Eb[j WD ..]
   double *Ef = lds + lane, *Eb = lds + WB + lane;
   double *tile = lds + (long)WD * w;
@@ -192,7 +242,7 @@ __device__ __forceinline__ void seg_wave(const double *__restrict__ x0, double *
       for (int q = 0; q < 16; ++q) {
         int r = s0 + 16 * t + tr;
         if (DYN) r = r > n - 1 ? n - 1 : r;
-        R[t][q] = x0[__shfl((int)rel, 4 * q + tl, 64) + r];
+        R[t][q] = job.in(PAIR && q >= 8)[base + __shfl((int)rel, 4 * q + tl, 64) + r];
       }
     // the rows next to the segment (the rows of a DYN segment's tile that lie
     // beyond its len are its successor's: nothing more to fetch)
@@ -206,10 +256,32 @@ __device__ __forceinline__ void seg_wave(const double *__restrict__ x0, double *
       for (int q = 0; q < 16; ++q) tile[(4 * q + tl) * SEG_TP + tr] = R[t][q];
       seg_tile_sync();
 #pragma unroll
-      for (int r = 0; r < 16; ++r) V[2 + 16 * t + r] = tile[lane * SEG_TP + r];
+      for (int r = 0; r < 16; ++r) V[2 + 16 * t + r] = factor(tile[lane * SEG_TP + r]);
       seg_tile_sync();
       if (t == 0) load_rows();
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (PAIR) {
+      V[0] = factor(V[0]);
+      V[1] = factor(V[1]);
+      V[LEN + 2] = factor(V[LEN + 2]);
+      V[LEN + 3] = factor(V[LEN + 3]);
+    }
+  } else if constexpr (PAIR) {
+    // the halves' pointers walk the rows (36 addresses would not fit the
+    // registers)
+    auto none = [](int k) { return (HEAD && k < 2) || (TAIL && !DYN && k >= LEN + 2); };
+    const double *xp = xl + (long)(HEAD ? 0 : s0 - 2) * s;
+#pragma unroll
+    for (int k = 0; k < LEN + 4; ++k) {
+      V[k] = none(k) ? 0.0 : *xp;
+      if (!none(k) && (!DYN || s0 - 2 + k < n - 1)) xp += s;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int k = 0; k < LEN + 4; ++k) {
+      if (!none(k)) V[k] = factor(V[k]);
+      if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
   } else {
 #pragma unroll
@@ -316,6 +388,50 @@ __device__ __forceinline__ void seg_wave(const double *__restrict__ x0, double *
   }
   Eb[w * WD] = Y[0];
   if (!TRI) Eb[w * WD + 64] = Y[1];
+  // a field at byte offset v (of the lane) from row ro of the segment
+  auto at = [&](auto *f, long ro, unsigned v) -> auto & {
+    return *(decltype(f))((char *)(f + base + (long)s0 * s + ro) + v);
+  };
+  // a pair's u and acc, 4 groups of 4 values per lane (the rows k0 + 2 j + up,
+  // or 4 lines of a 16-row tile), fetched two groups ahead of their use: the
+  // first two while the other segments finish
+  constexpr int GR = 4, NG = LEN / 8;
+  double uv[2][GR], av[2][GR];
+  // opaque to the compiler, so that the offsets of the stores are formed here
+  // rather than shared with those of the loads and held through the segment
+  long so = s;
+  int relo = (int)rel;
+  asm volatile("" : "+s"(so), "+v"(relo));
+  auto goff = [&](int g, int j) -> unsigned {
+    if constexpr (XT) {
+      const int r = 16 * (g / 2) + tr;
+      return 8u * (unsigned)(__shfl(relo, 16 * (g % 2) + 4 * j + tl, 64) + (DYN ? min(r, len - 1) : r));
+    } else {
+      const int k = 8 * g + 2 * j;
+      return 8u * (unsigned)relo + (up && (!DYN || k + 1 < len) ? 8u * (unsigned)so : 0u);
+    }
+  };
+  auto grow = [&](int g, int j) -> long {
+    const int k = 8 * g + 2 * j;
+    return XT ? 0 : (long)(DYN ? min(k, len - 1) : k) * so;
+  };
+  auto fetch = [&](int g) {
+    if constexpr (PAIR) {
+#pragma unroll
+      for (int j = 0; j < GR; ++j) {
+        uv[g % 2][j] = at(job.u, grow(g, j), goff(g, j));
+        if (Job::HAS_ACC) av[g % 2][j] = at(job.acc, grow(g, j), goff(g, j));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto share = [&](int g, int j, double dq, double dp) {
+    const double v = 0.5 * fma(uv[g % 2][j], dq, dp);
+    if constexpr (PAIR) return Job::HAS_ACC ? av[g % 2][j] + v : v;
+    return v;
+  };
+  fetch(0);
+  fetch(1);
   __syncthreads();
   v0 = v1 = 0.0;
   if (!TAIL) {
@@ -343,8 +459,6 @@ __device__ __forceinline__ void seg_wave(const double *__restrict__ x0, double *
     return xi;
   };
   if constexpr (XT) {
-    int relo = (int)rel;  // opaque: the offsets are formed here, not kept from the loads
-    asm volatile("" : "+v"(relo));
 #pragma unroll
     for (int t = 0; t < NR; ++t) {
 #pragma unroll
@@ -354,24 +468,51 @@ __device__ __forceinline__ void seg_wave(const double *__restrict__ x0, double *
       }
       seg_tile_sync();
       const bool rok = 16 * t + tr < (DYN ? len : LEN);
+      if constexpr (PAIR) {
 #pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int l = 4 * q + tl;
-        const int o = __shfl(relo, l, 64) + s0 + 16 * t + tr;
-        const double v = tile[l * SEG_TP + tr];
-        if (rok && l < hi) out0[o] = v;
-        if (q % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        for (int h = 0; h < 2; ++h) {
+          const int g = 2 * t + h;
+#pragma unroll
+          for (int j = 0; j < GR; ++j) {
+            const int l = 16 * h + 4 * j + tl;
+            const double v = share(g, j, tile[l * SEG_TP + tr], tile[(l + 32) * SEG_TP + tr]);
+            const unsigned o = goff(g, j);  // (all lanes take part)
+            if (rok && l < hi) at(job.out, 0, o) = v;
+          }
+          if (g + 2 < NG) fetch(g + 2);
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+          const int l = 4 * q + tl;
+          const int o = __shfl(relo, l, 64) + s0 + 16 * t + tr;
+          const double v = tile[l * SEG_TP + tr];
+          if (rok && l < hi) job.out[base + o] = v;
+          if (q % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
       }
       seg_tile_sync();
     }
+  } else if constexpr (PAIR) {
+    const bool act = line >= lo && line < hi;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+#pragma unroll
+      for (int j = 0; j < GR; ++j) {
+        const int k = 8 * g + 2 * j;
+        if (on(k)) {
+          double a = fixed(k), b = on(k + 1) ? fixed(k + 1) : 0.0;
+          seg_swap(a, b);  // this half's row: a = d(q), b = d(q u)
+          const double v = share(g, j, a, b);
+          if (act && (!DYN || k + up < len)) at(job.out, grow(g, j), goff(g, j)) = v;
+        }
+      }
+      if (g + 2 < NG) fetch(g + 2);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   } else {
-    // a fresh copy of the stride, opaque to the compiler, so that the store
-    // offsets are computed here rather than shared with the load offsets and
-    // held in SGPRs through the whole segment
-    long so = s;
-    asm volatile("" : "+s"(so));
-    double *po = out0 + rel + (long)s0 * so;
-    const bool act = lane >= lo && lane < hi;
+    double *po = job.out + base + rel + (long)s0 * so;
+    const bool act = line >= lo && line < hi;
 #pragma unroll
     for (int k = 0; k < LEN; ++k) {
       if (on(k)) {
@@ -383,14 +524,14 @@ __device__ __forceinline__ void seg_wave(const double *__restrict__ x0, double *
   }
 }
 
-// Solve the scheme on 64 lines per block, wave w = segment w.
-// x, out: the field and result; lines per SegLines (one family of lines).
+// Solve the scheme on 64 lines per block (32 of a pair), wave w = segment w.
+// off: added to every line's start; lines per SegLines (one family of lines).
 // lds: seg_lds_doubles(n, XT) (of the longest scheme of the launch).
 // Every wave of the block passes the same two barriers.
-template <bool TRI, bool XT>
-__device__ __forceinline__ void seg_solve(const double *__restrict__ x, double *__restrict__ out,
-                                          const SegTab &T, const SegLines &L, int lblock,
-                                          double *lds) {
+template <bool TRI, bool XT, class Job>
+__device__ __forceinline__ void seg_solve(const Job &job, long off, const SegTab &T,
+                                          const SegLines &L, int lblock, double *lds) {
+  constexpr int NL = seg_lines<Job>();
   const int n = T.n;
   const int K = T.K;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -401,30 +542,29 @@ __device__ __forceinline__ void seg_solve(const double *__restrict__ x, double *
     return;
   }
   // the block's first line, and this lane's from there
-  const int lane = threadIdx.x & 63;
+  const int line = threadIdx.x & (NL - 1);
   int lo = 0, hi;
   long base, rel;
   if (!XT && L.groups) {
-    const int ag = 64 * (lblock % L.groups), b = lblock / L.groups;
+    const int ag = NL * (lblock % L.groups), b = lblock / L.groups;
     lo = max(0, L.a0 - ag);
-    hi = min(64, L.a0 + L.na - ag);
+    hi = min(NL, L.a0 + L.na - ag);
     base = (long)ag * L.sa + (long)(L.b0 + b) * L.sb;
-    rel = min(max(lane, lo), hi - 1) * L.sa;
+    rel = min(max(line, lo), hi - 1) * L.sa;
   } else {
-    const int l0 = lblock * 64;
-    hi = min(64, L.nlines - l0);
-    const int l = l0 + min(lane, hi - 1);
+    const int l0 = lblock * NL;
+    hi = min(NL, L.nlines - l0);
+    const int l = l0 + min(line, hi - 1);
     const int a0 = l0 % L.na, b0 = l0 / L.na;
     base = (long)(L.a0 + a0) * L.sa + (long)(L.b0 + b0) * L.sb;
     rel = (long)(l % L.na - a0) * L.sa + (long)(l / L.na - b0) * L.sb;
   }
-  const double *x0 = x + base;
-  double *o0 = out + base;
+  base += off;
   const int s0 = T.len * w;
   const int len = (w == K - 1) ? n - s0 : T.len;
   auto go = [&](auto head, auto tail, auto dyn) {
     seg_wave<SEG_LEN, decltype(head)::value, decltype(tail)::value, decltype(dyn)::value, TRI, XT>(
-        x0, o0, rel, lo, hi, L.s, T, w, K, s0, len, lds);
+        job, base, rel, lo, hi, L.s, T, w, K, s0, len, lds);
   };
   typedef std::true_type yes;
   typedef std::false_type no;

@@ -30,6 +30,7 @@
 #include <string>
 #include <vector>
 
+#include "conv.h"
 #include "internal.h"
 #include "mflops/mf.h"
 
@@ -700,7 +701,14 @@ int der3(mf_ns *s, int axis, const double *x0, const double *x1, const double *x
   return mf_der3d_batch(s->dc[axis], axis, 1, 3, x, o, s->nx, s->ny, s->nz, st);
 }
 
-// nonlinear terms of the three components at level L (cached): the 9
+// Whether the nonlinear terms go axis by axis (conv3d): the skew-symmetric
+// form on lines it takes (faster at every size measured, 24^3 to 192 x 256 x
+// 192), unless the subgrid stresses want the gradients anyway.
+bool conv_by_axis(const mf_ns *s) {
+  return s->nlt == 2 && !s->les_type && !s->sgs && mf::conv3d_takes(s->dc, s->nx, s->ny, s->nz);
+}
+
+// nonlinear terms of the three components at level L (cached), otherwise: the 9
 // velocity gradients and, for the skew-symmetric form, the 9 product
 // derivatives, one batched launch per axis (6 fields: the line recurrences
 // are latency-bound, so a wider batch costs far less than a second launch)
@@ -709,6 +717,23 @@ int nonlinear(mf_ns *s, int L, hipStream_t st, const NlRhs *rhs = nullptr) {
   const long N = s->N;
   double *u = s->q[0][L], *v = s->q[1][L], *w = s->q[2][L];
   double **T = s->T;  // T[3a + c] gradients, T[9..14] products, T[15 + 3a + c] product derivatives
+  if (conv_by_axis(s)) {
+    // axis by axis (x into T[9..11], y into T[12..14], z into the level's
+    // terms): neither products nor derivatives are stored
+    for (int a = 0; a < 3; ++a) {
+      mf::ConvArgs v;
+      for (int c = 0; c < 3; ++c) {
+        v.q[c] = s->q[c][L];
+        v.acc[c] = a ? T[9 + 3 * (a - 1) + c] : nullptr;
+        v.out[c] = a < 2 ? T[9 + 3 * a + c] : s->nl[c][L];
+      }
+      v.u = s->q[a][L];
+      RC(mf::conv3d(s->dc[a], a, v, s->nx, s->ny, s->nz, st));
+    }
+    s->grad_level = -1;
+    s->nl_ok[L] = true;
+    return MF_OK;
+  }
   NlArgs n;
   std::memset(&n, 0, sizeof(n));
   n.u = u; n.v = v; n.w = w;
@@ -983,7 +1008,7 @@ int substep(mf_ns *s, int sub, int precision, double tol, bool *done, hipStream_
   // nonlinear terms of the levels the extrapolation reads, the older ones
   // first: for pt = 1 without LES the newest one's kernel also forms the
   // velocity right-hand sides (into T[0..2]), which read the older ones
-  const bool fuse_rhs = s->fused_rhs && pt == 1 && sub == 1 && !s->les_type && !s->sgs &&
+  const bool fuse_rhs = s->fused_rhs && !conv_by_axis(s) && pt == 1 && sub == 1 && !s->les_type && !s->sgs &&
                         ev.c[0] != 0.0 && ev.lev[0] == L0 && !s->nl_ok[ev.lev[0]];
   for (int m = 2; m >= 1; --m)
     if (ev.c[m] != 0.0) RC(nonlinear(s, ev.lev[m], st));

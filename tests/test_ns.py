@@ -620,3 +620,36 @@ def test_oracle_minus_div_tau_closed_form():
         ref = -sum(grad[cols[(min(i, j), max(i, j))]][j] for j in range(3))
         err = np.abs(f[c] - ref)[inner].max() / np.abs(ref[inner]).max()
         assert err < 1e-11, (c, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,so", [((20, 24, 18), 6), ((33, 36, 35), 6), ((32, 65, 34), 6),
+                                  ((34, 66, 64), 8), ((67, 33, 99), 4), ((96, 40, 98), 6),
+                                  ((144, 66, 36), 8), ((512, 24, 20), 6), ((20, 24, 513), 6)])
+def test_gpu_convective_term_by_axis(n, so):
+    """The convective term formed axis by axis against the stored products and
+    gradients, which an eddy viscosity of constant 0 asks for: lines of one
+    segment, just beyond one, of even and uneven ones, in aligned and unaligned
+    groups, tridiagonal and not; the last shape has lines that take the general
+    path on both sides.  One step's velocity holds dt times the term, whose
+    rounding is some hundred eps max|q|^2 / h (1e-12 here), and the solves'
+    own (1e-13)."""
+    import mflops as mf
+    import torch
+    assert torch.cuda.is_available()
+    mf.load()
+    gx, gy, gz, u, v, w, bc = _channel(n)
+    rng = np.random.default_rng(7)
+    q = [np.asfortranarray(a + 0.3 * rng.standard_normal(a.shape)) for a in (u, v, w)]
+    out = []
+    for les in (0, 1):
+        print("run ns convective term", n, so, "les", les, flush=True)
+        s = _gpu_ns(mf, gx, gy, gz, *q, bc, 3000.0, 1e-2, so=so)
+        s.set_flow_rate(True, 2.0 / 3000.0)
+        if les:
+            s.set_les(1, 0.0)
+        s.step(1, mf.MF_FP64)
+        out.append([mf.to_host(t) for t in s.get()[:3]])
+    for a, b in zip(*out):
+        assert np.isfinite(a).all()
+        assert np.abs(a - b).max() < 1e-11 * np.abs(b).max()
