@@ -522,7 +522,7 @@ def run_md(args):
         bd.append(torch.tensor(np.concatenate([b.ravel(order="F") for b in bc]), device="cuda"))
         exact.append(U)
     u = [mf.fortran_zeros(g.shape) for g in gd]
-    # matvec rate (the GMRES inner product is one pass over all blocks)
+    # mf_md_matvec's rate (one pass over all blocks; the solve applies them factored)
     x = torch.ones(h.ninf, dtype=torch.float64, device="cuda")
     y = torch.empty_like(x)
     h.matvec(x, y)
