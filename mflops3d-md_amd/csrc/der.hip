@@ -1,6 +1,6 @@
 // Compact finite-difference derivatives on gfx950.
 //
-// Lines of up to 512 points take the segmented solve (der_seg.h), 3-D fields
+// Lines of up to 528 points take the segmented solve (der_seg.h), 3-D fields
 // and batches of contiguous lines alike.  Longer ones (and contiguous lines
 // that lie more than 2^25 points apart) take the kernels of this file:
 // one lane owns one grid line and runs the reference's per-line algorithm:
@@ -315,7 +315,7 @@ __device__ __forceinline__ void seg_place(const SegGrid &G, bool inner, int &blk
   fld = inner ? t % nf : t / G.b_full;
 }
 
-template <int AXIS, bool TRI, class Job>
+template <int AXIS, bool TRI, bool LONG, class Job>
 __device__ __forceinline__ void seg_block(const Job &job, const SegGrid &G, int blk, double *lds) {
   const int nx = G.nx, ny = G.ny, nz = G.nz;
   const int4 nb4 = G.nb4;
@@ -356,7 +356,7 @@ __device__ __forceinline__ void seg_block(const Job &job, const SegGrid &G, int 
   }
   if (solve) {
     L.nlines = L.na * L.nb;
-    seg_solve<TRI, AXIS == 0>(job, off, T, L, blk, lds);
+    seg_solve<TRI, AXIS == 0, LONG>(job, off, T, L, blk, lds);
     return;
   }
   // zeros: the four two-boundary-plane lines and both ends of the sub lines
@@ -376,13 +376,13 @@ __device__ __forceinline__ void seg_block(const Job &job, const SegGrid &G, int 
   }
 }
 
-template <int AXIS, bool TRI>
+template <int AXIS, bool TRI, bool LONG>
 __global__ void __launch_bounds__(64 * SEG_KMAX) der3d_seg_kernel(FieldSet fs, SegGrid G) {
   extern __shared__ double lds[];
   int blk, fld;
   seg_place(G, false, blk, fld);
   const SegDer job{fs.x[fld], fs.out[fld]};
-  seg_block<AXIS, TRI>(job, G, blk, lds);
+  seg_block<AXIS, TRI, LONG>(job, G, blk, lds);
 }
 
 // One axis of the convective term of all components (SegConv): 32 lines of one
@@ -404,12 +404,12 @@ __global__ void __launch_bounds__(64 * SEG_KMAX) conv3d_kernel(ConvArgs a, SegGr
   int c, blk;
   seg_place(G, true, blk, c);
   const SegConv<AXIS != 0> job{a.q[c], a.u, a.acc[c], a.out[c]};
-  seg_block<AXIS, TRI>(job, G, blk, lds);
+  seg_block<AXIS, TRI, false>(job, G, blk, lds);
 }
 
 // batched lines on segmented line solves: line l at x + l*ld, contiguous
 // points (der/dder/der_s/dder_s)
-template <bool TRI>
+template <bool TRI, bool LONG>
 __global__ void __launch_bounds__(64 * SEG_KMAX)
     der_lines_seg_kernel(const double *__restrict__ x, double *__restrict__ out, int nlines,
                          long ld, SegTab T) {
@@ -419,7 +419,7 @@ __global__ void __launch_bounds__(64 * SEG_KMAX)
   L.a0 = 0; L.na = nlines; L.b0 = 0; L.nb = 1;
   L.nlines = nlines;
   L.groups = 0;
-  seg_solve<TRI, true>(SegDer{x, out}, 0, T, L, blockIdx.x, lds);
+  seg_solve<TRI, true, LONG>(SegDer{x, out}, 0, T, L, blockIdx.x, lds);
 }
 
 // the same, one lane per line, for lines longer than the segmented solve
@@ -447,7 +447,7 @@ struct mf_der {
   double *dbuf = nullptr;      // device tables, then one scratch line of n
   double *scratch = nullptr;   // surplus lanes' output line
   mf::LineTab tab[2][2];       // [order-1][sub]
-  mf::SegTab seg[2][2];        // the segmented solve's tables (lines of up to 512 points)
+  mf::SegTab seg[2][2];        // the segmented solve's tables (lines it takes)
   bool tri[2] = {false, false};  // [order-1]: tridiagonal factors, full and sub scheme
   std::vector<double> host[2][2][2];  // [order-1][sub][0: dl_lu(n,5), 1: dr(n,7)]
 };
@@ -611,12 +611,16 @@ extern "C" int mf_der_lines(const mf_der *dc, int order, int sub, const double *
     const dim3 grid((nlines + 63) / 64), block(64 * mf::seg_count(S.n));
     const size_t lds = mf::seg_lds_doubles(S.n, true) * sizeof(double);
     const int o = sub ? 1 : 0;
-    if (dc->tri[order - 1])
-      hipLaunchKernelGGL(mf::der_lines_seg_kernel<true>, grid, block, lds, (hipStream_t)stream,
-                         x + o, out + o, nlines, (long)ld, S);
-    else
-      hipLaunchKernelGGL(mf::der_lines_seg_kernel<false>, grid, block, lds, (hipStream_t)stream,
-                         x + o, out + o, nlines, (long)ld, S);
+    auto go = [&](auto tri, auto lng) {
+      hipLaunchKernelGGL((mf::der_lines_seg_kernel<decltype(tri)::value, decltype(lng)::value>), grid,
+                         block, lds, (hipStream_t)stream, x + o, out + o, nlines, (long)ld, S);
+    };
+    auto pick = [&](auto tri) {
+      if (S.len > mf::SEG_LEN) go(tri, std::true_type());
+      else go(tri, std::false_type());
+    };
+    if (dc->tri[order - 1]) pick(std::true_type());
+    else pick(std::false_type());
     HIPCHK(hipGetLastError());
     return MF_OK;
   }
@@ -655,7 +659,7 @@ mf::SegGrid seg_grid(const mf_der *dc, int axis, int order, int lines, int nx, i
 namespace mf {
 bool conv3d_takes(const ::mf_der *const dc[3], int nx, int ny, int nz) {
   for (int a = 0; a < 3; ++a)
-    if (!dc[a]->seg[0][0].pack) return false;
+    if (!dc[a]->seg[0][0].pack || dc[a]->seg[0][0].len > SEG_LEN) return false;
   return seg_fits((long)nx * ny) && nx > 2 && ny > 2 && nz > 2;
 }
 
@@ -719,13 +723,18 @@ extern "C" int mf_der3d_batch(const mf_der *dc, int axis, int order, int nfields
     const mf::SegGrid G = seg_grid(dc, axis, order, 64, nx, ny, nz, &sblocks);
     const size_t lds = mf::seg_lds_doubles(F.n, axis == 0) * sizeof(double);
     const dim3 grid(sblocks, nfields), block(64 * mf::seg_count(F.n));
-    auto go = [&](auto ax, auto tri) {
-      hipLaunchKernelGGL((mf::der3d_seg_kernel<decltype(ax)::value, decltype(tri)::value>), grid,
-                         block, lds, st, fs, G);
+    auto go = [&](auto ax, auto tri, auto lng) {
+      hipLaunchKernelGGL((mf::der3d_seg_kernel<decltype(ax)::value, decltype(tri)::value,
+                                               decltype(lng)::value>),
+                         grid, block, lds, st, fs, G);
+    };
+    auto scheme = [&](auto ax, auto tri) {
+      if (G.full.len > mf::SEG_LEN) go(ax, tri, std::true_type());
+      else go(ax, tri, std::false_type());
     };
     auto pick = [&](auto ax) {
-      if (dc->tri[order - 1]) go(ax, std::true_type());
-      else go(ax, std::false_type());
+      if (dc->tri[order - 1]) scheme(ax, std::true_type());
+      else scheme(ax, std::false_type());
     };
     if (axis == 0) pick(std::integral_constant<int, 0>());
     else if (axis == 1) pick(std::integral_constant<int, 1>());

@@ -43,7 +43,8 @@
 
 namespace mf {
 
-constexpr int SEG_LEN = 32;     // longest segment
+constexpr int SEG_LEN = 32;     // longest segment, on lines of up to 16 of them
+constexpr int SEG_LONG = 33;    // longest on the lines just beyond (an instance of its own)
 // Whether the lines along y or z of a field of nx columns go in groups of
 // `lines` aligned in memory: rows of whole cache lines (16 points), and few
 // lanes lost at the rows' ends.
@@ -60,10 +61,16 @@ constexpr int SEG_PACK = 512;   // coefficient doubles per segment
 constexpr int SEG_CHAIN = 64;   // doubles per chain table (4 per segment)
 
 // Segmentation of a line of n points: K segments of seg_len(n) rows, the last
-// one the rest (for 33 <= n <= 512 at least 11 rows: it holds the 7-point
+// one the rest (for 33 <= n <= 528 at least 11 rows: it holds the 7-point
 // closure's inputs and row n-4).  Even segments, since a block takes as long
-// as its longest.
-__host__ __device__ inline int seg_count(int n) { return (n + SEG_LEN - 1) / SEG_LEN; }
+// as its longest.  Lines of 513 to 528 points (2^9 intervals and a few more)
+// take 16 segments of up to 33 rows: 513 x 64 x 65, one derivative along x / y / z
+// 300 / 299 / 293 us one lane per line, 25 / 85 / 82 us in segments (512 points:
+// 24 / 80 / 80 us).
+__host__ __device__ inline int seg_count(int n) {
+  const int K = (n + SEG_LEN - 1) / SEG_LEN;
+  return K > SEG_KMAX && n <= SEG_KMAX * SEG_LONG ? SEG_KMAX : K;
+}
 __host__ __device__ inline int seg_len(int n) { return (n + seg_count(n) - 1) / seg_count(n); }
 
 // LDS doubles per wave: the forward and backward exchange arrays, 2 x 64
@@ -100,7 +107,7 @@ struct SegSlot {
 };
 __host__ __device__ constexpr int seg_cw(bool tri) { return tri ? 10 : 14; }
 constexpr int SEG_XHEAD = 496, SEG_XTAIL = 500, SEG_XALPHA = 504, SEG_XBETA = 505;
-static_assert(SEG_LEN * 14 <= SEG_XHEAD, "a segment's rows fit the pack");
+static_assert(SEG_LONG * 14 <= SEG_XHEAD, "a segment's rows fit the pack");
 static_assert(4 * SEG_KMAX <= SEG_CHAIN, "the chain tables fit one register pair");
 // Chain tables, 4 doubles per segment j: forward A, B of its last row but one
 // and of its last row; backward C, D of its first and second row.
@@ -233,7 +240,7 @@ __device__ __forceinline__ void seg_wave(const Job &job, long base, long rel, in
   // two after it (last segment of exactly LEN rows) are never read; a
   // runtime-length segment clamps into the line
   double V[LEN + 4];
-  constexpr int NR = LEN / 16;  // 16-row tiles
+  constexpr int NR = LEN / 16;  // 16-row tiles (rows beyond them go lane by lane)
   if constexpr (XT) {
     double R[NR][16];
 #pragma unroll
@@ -248,8 +255,9 @@ __device__ __forceinline__ void seg_wave(const Job &job, long base, long rel, in
     // beyond its len are its successor's: nothing more to fetch)
     V[0] = HEAD ? 0.0 : xl[s0 - 2];
     V[1] = HEAD ? 0.0 : xl[s0 - 1];
-    V[LEN + 2] = TAIL ? 0.0 : xl[s0 + LEN > n - 1 ? n - 1 : s0 + LEN];
-    V[LEN + 3] = TAIL ? 0.0 : xl[s0 + LEN + 1 > n - 1 ? n - 1 : s0 + LEN + 1];
+#pragma unroll
+    for (int r = 16 * NR; r < LEN + 2; ++r)
+      V[2 + r] = TAIL && r >= LEN ? 0.0 : xl[s0 + r > n - 1 ? n - 1 : s0 + r];
 #pragma unroll
     for (int t = 0; t < NR; ++t) {
 #pragma unroll
@@ -396,6 +404,7 @@ __device__ __forceinline__ void seg_wave(const Job &job, long base, long rel, in
   // or 4 lines of a 16-row tile), fetched two groups ahead of their use: the
   // first two while the other segments finish
   constexpr int GR = 4, NG = LEN / 8;
+  static_assert(!PAIR || LEN % 16 == 0, "a pair's groups are whole tiles");
   double uv[2][GR], av[2][GR];
   // opaque to the compiler, so that the offsets of the stores are formed here
   // rather than shared with those of the loads and held through the segment
@@ -493,6 +502,15 @@ __device__ __forceinline__ void seg_wave(const Job &job, long base, long rel, in
       }
       seg_tile_sync();
     }
+    if constexpr (16 * NR < LEN) {
+      const bool act = line >= lo && line < hi;
+#pragma unroll
+      for (int r = 16 * NR; r < LEN; ++r)
+        if (on(r)) {
+          const double xi = fixed(r);
+          if (act) job.out[base + relo + s0 + r] = xi;
+        }
+    }
   } else if constexpr (PAIR) {
     const bool act = line >= lo && line < hi;
 #pragma unroll
@@ -525,10 +543,11 @@ __device__ __forceinline__ void seg_wave(const Job &job, long base, long rel, in
 }
 
 // Solve the scheme on 64 lines per block (32 of a pair), wave w = segment w.
+// LONG: segments of up to SEG_LONG rows.
 // off: added to every line's start; lines per SegLines (one family of lines).
 // lds: seg_lds_doubles(n, XT) (of the longest scheme of the launch).
 // Every wave of the block passes the same two barriers.
-template <bool TRI, bool XT, class Job>
+template <bool TRI, bool XT, bool LONG, class Job>
 __device__ __forceinline__ void seg_solve(const Job &job, long off, const SegTab &T,
                                           const SegLines &L, int lblock, double *lds) {
   constexpr int NL = seg_lines<Job>();
@@ -563,12 +582,16 @@ __device__ __forceinline__ void seg_solve(const Job &job, long off, const SegTab
   const int s0 = T.len * w;
   const int len = (w == K - 1) ? n - s0 : T.len;
   auto go = [&](auto head, auto tail, auto dyn) {
-    seg_wave<SEG_LEN, decltype(head)::value, decltype(tail)::value, decltype(dyn)::value, TRI, XT>(
-        job, base, rel, lo, hi, L.s, T, w, K, s0, len, lds);
+    seg_wave<LONG ? SEG_LONG : SEG_LEN, decltype(head)::value, decltype(tail)::value,
+             decltype(dyn)::value, TRI, XT>(job, base, rel, lo, hi, L.s, T, w, K, s0, len, lds);
   };
   typedef std::true_type yes;
   typedef std::false_type no;
-  if (K == 1) {
+  if constexpr (LONG) {
+    if (w == 0) go(yes(), no(), yes());
+    else if (w < K - 1) go(no(), no(), yes());
+    else go(no(), yes(), yes());
+  } else if (K == 1) {
     go(yes(), yes(), yes());
   } else if (len == SEG_LEN) {
     if (w == 0) go(yes(), no(), no());

@@ -101,6 +101,51 @@ def test_derivatives_shapes(shape, so):
     _der_case(mf, gs, f, so, label=str(shape))
 
 
+# lines of 16 segments of up to 33 rows (513 to 528 points, with sub-lines of 32
+# and of 33), and of one lane per line beyond, along each axis in turn
+@pytest.mark.parametrize("shape", [(513, 10, 66), (66, 515, 10), (10, 66, 528),
+                                   (529, 9, 66), (66, 530, 9), (9, 66, 601)])
+@pytest.mark.parametrize("so", [6, 8])
+def test_derivatives_long_lines(shape, so):
+    mf, torch = _mf()
+    rng = np.random.default_rng(sum(shape) + so)
+    gs = [o.grid_uniform(shape[0], 0, 1), o.grid_tanh(shape[1], 0, 2, 1.8),
+          o.grid_asin(shape[2], -0.5, 0.5)]
+    f = np.asfortranarray(rng.standard_normal(shape))
+    _der_case(mf, gs, f, so, label=str(shape))
+
+
+def test_derivatives_just_beyond_512_points():
+    """2^9 intervals and a few more take the segmented solve too.  The times of
+    513 and 528 points are 1.04 to 1.09 of that of 512 (one lane per line: 3.7 to
+    12 times it; bar 3)."""
+    mf, torch = _mf()
+
+    def best(shape, axis):
+        dc = mf.DerivativeCoefficients(o.grid_uniform(shape[axis], 0, 1), solver=True, so=6)
+        x, out = mf.fortran_zeros(shape), mf.fortran_zeros(shape)
+        x.fill_(1.0)
+        t = []
+        for _ in range(12):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            for _ in range(5):
+                mf.derivative(dc, x, axis, 1, out)
+            e[1].record()
+            e[1].synchronize()
+            t.append(e[0].elapsed_time(e[1]))
+        return min(t)
+
+    for axis in range(3):
+        t = {}
+        for n in (512, 513, 528):
+            shape = [64, 65, 64]
+            shape[axis] = n
+            t[n] = best(tuple(shape), axis)
+        print("axis %d: %s" % (axis, {n: "%.1f us" % (200 * v) for n, v in t.items()}), flush=True)
+        assert t[513] < 3 * t[512] and t[528] < 3 * t[512]
+
+
 def test_derivatives_white_noise():
     """Pure noise input: the worst case for cancellation."""
     mf, torch = _mf()
@@ -129,10 +174,10 @@ def test_der_lines():
         _check("lines " + name, got, ex, ora)
 
 
-# one segment, even and uneven segments, 16 full ones, and the one-lane kernel
-# beyond; groups of 64 lines full, short by one and just begun; lines apart by
+# one segment, even and uneven segments, 16 full ones, 16 of up to 33 rows, and
+# the one-lane kernel beyond; groups of 64 lines full, short by one and just begun; lines apart by
 # more than their length
-@pytest.mark.parametrize("n", [10, 32, 33, 64, 66, 321, 481, 512, 513])
+@pytest.mark.parametrize("n", [10, 32, 33, 64, 66, 321, 481, 512, 513, 528, 529])
 @pytest.mark.parametrize("so", [6, 8])
 def test_der_lines_segments(n, so):
     mf, torch = _mf()
