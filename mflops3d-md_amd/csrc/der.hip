@@ -468,8 +468,9 @@ namespace {
 constexpr int kLinePack = 13;
 void pack_scheme(int n, const std::vector<double> &dl, const std::vector<double> &dr, bool tri,
                  std::vector<double> &dst) {
-  const bool seg = mf::seg_count(n) <= mf::SEG_KMAX;
-  dst.assign((size_t)kLinePack * n + (seg ? mf::seg_table_doubles(n) : 0), 0.0);
+  const int K = mf::seg_count(n, tri);
+  const bool seg = K <= mf::SEG_KMAX;
+  dst.assign((size_t)kLinePack * n + (seg ? mf::seg_table_doubles(K) : 0), 0.0);
   for (int i = 0; i < n; ++i)
     for (int m = 0; m < 7; ++m) dst[(size_t)7 * i + m] = dr[i + (size_t)n * m];
   double *p = &dst[(size_t)7 * n];
@@ -583,8 +584,10 @@ extern "C" int mf_der_create(const double *grid, int n, int solver_mode, int so,
       T.alpha = h->host[o][sub][0][0];                       // dl(1,1)
       T.beta = h->host[o][sub][0][4 * (size_t)m + m - 1];    // dl(m,5) after pentalu
       T.n = m;
-      if (pk.size() > (size_t)kLinePack * m) 
-        h->seg[o][sub] = mf::SegTab{b + (size_t)kLinePack * m, m, mf::seg_count(m), mf::seg_len(m)};
+      if (pk.size() > (size_t)kLinePack * m) {
+        const int K = mf::seg_count(m, h->tri[o]);
+        h->seg[o][sub] = mf::SegTab{b + (size_t)kLinePack * m, m, K, mf::seg_len(m, K)};
+      }
       off += pk.size();
     }
   *out = h;
@@ -608,8 +611,8 @@ extern "C" int mf_der_lines(const mf_der *dc, int order, int sub, const double *
   const mf::LineTab &T = dc->tab[order - 1][sub ? 1 : 0];
   const mf::SegTab &S = dc->seg[order - 1][sub ? 1 : 0];
   if (S.pack && mf::seg_fits(ld)) {
-    const dim3 grid((nlines + 63) / 64), block(64 * mf::seg_count(S.n));
-    const size_t lds = mf::seg_lds_doubles(S.n, true) * sizeof(double);
+    const dim3 grid((nlines + 63) / 64), block(64 * S.K);
+    const size_t lds = mf::seg_lds_doubles(S.K, true) * sizeof(double);
     const int o = sub ? 1 : 0;
     auto go = [&](auto tri, auto lng) {
       hipLaunchKernelGGL((mf::der_lines_seg_kernel<decltype(tri)::value, decltype(lng)::value>), grid,
@@ -668,10 +671,10 @@ int conv3d(const ::mf_der *dc, int axis, const ConvArgs &a, int nx, int ny, int 
   if (dc->n != n || !dc->solver) return fail(MF_ERR_ARG, "conv3d: not the handle of this axis");
   int blocks;
   const SegGrid G = seg_grid(dc, axis, 1, 32, nx, ny, nz, &blocks);
-  const size_t lds = seg_lds_doubles(n, axis == 0) * sizeof(double);
+  const size_t lds = seg_lds_doubles(G.full.K, axis == 0) * sizeof(double);
   auto go = [&](auto ax, auto tri) {
     hipLaunchKernelGGL((conv3d_kernel<decltype(ax)::value, decltype(tri)::value>), dim3(blocks, 3),
-                       dim3(64 * seg_count(n)), lds, (hipStream_t)stream, a, G);
+                       dim3(64 * G.full.K), lds, (hipStream_t)stream, a, G);
   };
   auto pick = [&](auto ax) {
     if (dc->tri[0]) go(ax, std::true_type());
@@ -721,8 +724,8 @@ extern "C" int mf_der3d_batch(const mf_der *dc, int axis, int order, int nfields
     // segmented solves: 64 lines per block, one wavefront per segment
     int sblocks;
     const mf::SegGrid G = seg_grid(dc, axis, order, 64, nx, ny, nz, &sblocks);
-    const size_t lds = mf::seg_lds_doubles(F.n, axis == 0) * sizeof(double);
-    const dim3 grid(sblocks, nfields), block(64 * mf::seg_count(F.n));
+    const size_t lds = mf::seg_lds_doubles(G.full.K, axis == 0) * sizeof(double);
+    const dim3 grid(sblocks, nfields), block(64 * G.full.K);
     auto go = [&](auto ax, auto tri, auto lng) {
       hipLaunchKernelGGL((mf::der3d_seg_kernel<decltype(ax)::value, decltype(tri)::value,
                                                decltype(lng)::value>),

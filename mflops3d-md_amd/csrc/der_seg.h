@@ -60,18 +60,23 @@ constexpr int SEG_KMAX = 16;    // segments per line (wavefronts per block)
 constexpr int SEG_PACK = 512;   // coefficient doubles per segment
 constexpr int SEG_CHAIN = 64;   // doubles per chain table (4 per segment)
 
-// Segmentation of a line of n points: K segments of seg_len(n) rows, the last
-// one the rest (for 33 <= n <= 528 at least 11 rows: it holds the 7-point
+// Segmentation of a line of n points: K segments of seg_len(n, K) rows, the last
+// one the rest (of several at least 8 rows: it holds the 7-point
 // closure's inputs and row n-4).  Even segments, since a block takes as long
 // as its longest.  Lines of 513 to 528 points (2^9 intervals and a few more)
 // take 16 segments of up to 33 rows: 513 x 64 x 65, one derivative along x / y / z
 // 300 / 299 / 293 us one lane per line, 25 / 85 / 82 us in segments (512 points:
-// 24 / 80 / 80 us).
-__host__ __device__ inline int seg_count(int n) {
+// 24 / 80 / 80 us).  Pentadiagonal lines of 17 to 32 points take two segments, since
+// their rows' 28 lane reads make one long wave: 32^3 along x / y / z 12.0 / 13.0 /
+// 13.4 -> 9.8 / 8.9 / 8.9 us, 49 152 lines of 32 points 14.8 -> 12.4 us (400 000 of
+// them, where the rows read twice count, 46.6 -> 49.2 us).  Tridiagonal ones keep
+// one segment, which is as fast there and 10% faster on 400 000 lines.
+inline int seg_count(int n, bool tri) {
+  if (!tri && n >= 17 && n <= SEG_LEN) return 2;
   const int K = (n + SEG_LEN - 1) / SEG_LEN;
   return K > SEG_KMAX && n <= SEG_KMAX * SEG_LONG ? SEG_KMAX : K;
 }
-__host__ __device__ inline int seg_len(int n) { return (n + seg_count(n) - 1) / seg_count(n); }
+inline int seg_len(int n, int K) { return (n + K - 1) / K; }
 
 // LDS doubles per wave: the forward and backward exchange arrays, 2 x 64
 // each; on contiguous lines the wave's 64 x 16 transpose tile, whose start
@@ -79,12 +84,10 @@ __host__ __device__ inline int seg_len(int n) { return (n + seg_count(n) - 1) / 
 // last barrier), and the backward exchange
 constexpr int SEG_TP = 17;  // pitch of the transpose tile
 __host__ __device__ constexpr int seg_wave_doubles(bool xt) { return xt ? 64 * SEG_TP + 128 : 256; }
-// dynamic LDS doubles of a block running a scheme of n points
-__host__ __device__ inline int seg_lds_doubles(int n, bool xt) {
-  return seg_wave_doubles(xt) * seg_count(n);
-}
+// dynamic LDS doubles of a block running a scheme of K segments
+inline int seg_lds_doubles(int K, bool xt) { return seg_wave_doubles(xt) * K; }
 // doubles of a scheme's table: the segments' packs, then the two chain tables
-inline size_t seg_table_doubles(int n) { return (size_t)SEG_PACK * seg_count(n) + 2 * SEG_CHAIN; }
+inline size_t seg_table_doubles(int K) { return (size_t)SEG_PACK * K + 2 * SEG_CHAIN; }
 
 // The right-hand side sum_m dr_m f_m of an interior row is formed on the
 // differences of its window,
@@ -545,7 +548,7 @@ __device__ __forceinline__ void seg_wave(const Job &job, long base, long rel, in
 // Solve the scheme on 64 lines per block (32 of a pair), wave w = segment w.
 // LONG: segments of up to SEG_LONG rows.
 // off: added to every line's start; lines per SegLines (one family of lines).
-// lds: seg_lds_doubles(n, XT) (of the longest scheme of the launch).
+// lds: seg_lds_doubles(K, XT) (of the longest scheme of the launch).
 // Every wave of the block passes the same two barriers.
 template <bool TRI, bool XT, bool LONG, class Job>
 __device__ __forceinline__ void seg_solve(const Job &job, long off, const SegTab &T,
@@ -612,13 +615,13 @@ inline void seg_tables(int n, const double *dr, const double *p, const double *f
                        const double *d, const double *e, const double *rc, double alpha,
                        double beta, bool tri, double *out) {
   typedef long double real;
-  const int K = seg_count(n), CW = seg_cw(tri);
+  const int K = seg_count(n, tri), len = seg_len(n, K), CW = seg_cw(tri);
   double *fch = out + (size_t)SEG_PACK * K, *bch = fch + SEG_CHAIN;
-  std::fill(out, out + seg_table_doubles(n), 0.0);
+  std::fill(out, out + seg_table_doubles(K), 0.0);
   std::vector<real> R[4];  // A, B, C, D
   for (int u = 0; u < 4; ++u) R[u].assign(n, 0);
   for (int w = 0; w < K; ++w) {
-    const int s0 = seg_len(n) * w, e0 = (w == K - 1) ? n : s0 + seg_len(n);
+    const int s0 = len * w, e0 = (w == K - 1) ? n : s0 + len;
     for (int u = 0; u < 2 && w > 0; ++u) {
       real m2 = u ? 0 : 1, m1 = u ? 1 : 0;  // y_{s0-2}, y_{s0-1}
       for (int i = s0; i < e0; ++i) {

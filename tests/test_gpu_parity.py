@@ -83,10 +83,11 @@ def test_derivatives_c1():
     _der_case(mf, (gx, gy, gz), u, 6, label="c1")
 
 
-# line lengths cover one to eleven segments of up to 32 rows, and sub-lines
-# with fewer segments than the full lines (33, 65, 130)
+# line lengths cover one to eleven segments of up to 32 rows (pentadiagonal
+# lines two from 17 points on), and sub-lines with fewer segments than the full
+# lines (18, 33, 65, 130)
 @pytest.mark.parametrize("shape", [(9, 10, 11), (33, 17, 40), (70, 65, 10), (130, 12, 9),
-                                   (39, 340, 38)])
+                                   (39, 340, 38), (17, 32, 19), (16, 18, 31)])
 @pytest.mark.parametrize("so", [4, 6, 8])
 def test_derivatives_shapes(shape, so):
     mf, torch = _mf()
@@ -177,7 +178,7 @@ def test_der_lines():
 # one segment, even and uneven segments, 16 full ones, 16 of up to 33 rows, and
 # the one-lane kernel beyond; groups of 64 lines full, short by one and just begun; lines apart by
 # more than their length
-@pytest.mark.parametrize("n", [10, 32, 33, 64, 66, 321, 481, 512, 513, 528, 529])
+@pytest.mark.parametrize("n", [10, 16, 17, 19, 22, 32, 33, 64, 66, 321, 481, 512, 513, 528, 529])
 @pytest.mark.parametrize("so", [6, 8])
 def test_der_lines_segments(n, so):
     mf, torch = _mf()

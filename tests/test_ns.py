@@ -623,7 +623,7 @@ def test_oracle_minus_div_tau_closed_form():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,so", [((20, 24, 18), 6), ((33, 36, 35), 6), ((32, 65, 34), 6),
+@pytest.mark.parametrize("n,so", [((20, 24, 18), 6), ((31, 66, 20), 8), ((33, 36, 35), 6), ((32, 65, 34), 6),
                                   ((34, 66, 64), 8), ((67, 33, 99), 4), ((96, 40, 98), 6),
                                   ((144, 66, 36), 8), ((512, 24, 20), 6), ((20, 24, 513), 6)])
 def test_gpu_convective_term_by_axis(n, so):
