@@ -25,9 +25,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-#include <cmath>
 #include <type_traits>
+
+#include "gemm_tile.h"
 
 namespace mf {
 
@@ -170,10 +170,97 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ A, long lda,
     if (s + d < KS) mma_end(d, s + d);
 }
 
+// The same for a K-contiguous B, 16 k at a time (K >= 16): in step r of four,
+// lane (c, g) takes k = 16 q + 4 g + r, so that it loads the four steps' values
+// of B as one vector (at any alignment of T).  One value a step touches 16 cache
+// lines for 256 bytes where T is 32 bits wide, and that bound the FP32 x
+// transform: 124 us at 254^3 on 64 x 64 tiles, 61 at 192 x 256 x 192 on 64 x 48.
+// With vectors, four quads ahead, 32 x 32 tiles do best: 96 and 44 us (staged
+// through LDS 101 and 46); 3.5 us for 4.7 at 64^3 on 16 x 16.
+template <typename T, int MI, int NI, int Q>
+__device__ __forceinline__ void gemm_tile_quads(const T *__restrict__ A, long lda,
+                                                const T *__restrict__ B, long ldb, int M, int N,
+                                                int K, int m0, int n0,
+                                                typename Mfma<T>::acc_t (&acc)[MI][NI]) {
+  typedef typename Mfma<T>::acc_t acc_t;
+  typedef T vec_t __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int a = 0; a < MI; ++a)
+#pragma unroll
+    for (int b = 0; b < NI; ++b) acc[a][b] = (acc_t){0, 0, 0, 0};
+
+  // The last 16 k are K - 16 .. K - 1; the first `over` of them, which the quad
+  // before holds, are set to zero.
+  const int KQ = (K + 15) / 16, over = 16 * KQ - K;
+  const T *pa[MI], *pb[NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) pa[i] = A + min(m0 + 16 * i + c, M - 1) + lda * (4 * g);
+#pragma unroll
+  for (int i = 0; i < NI; ++i) pb[i] = B + (long)min(n0 + 16 * i + c, N - 1) * ldb + 4 * g;
+  T af[Q][4][MI];
+  vec_t bf[Q][NI];
+  // k from quad q to the next
+  auto step = [&](int q) { return q + 2 > KQ ? 0 : (q + 2 == KQ ? 16 - over : 16); };
+  auto fetch_a = [&](int d, int r, int q) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) af[d][r][i] = *pa[i];
+    const long da = r < 3 ? lda : (step(q) - 3) * lda;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) pa[i] += da;
+  };
+  auto fetch_b = [&](int d, int q) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) bf[d][i] = *(const vec_t *)pb[i];
+    const int db = step(q);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) pb[i] += db;
+  };
+  auto mma = [&](int d, int r) {
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+      for (int ni = 0; ni < NI; ++ni)
+        acc[mi][ni] = Mfma<T>::op(bf[d][ni][r], af[d][r][mi], acc[mi][ni]);
+  };
+#pragma unroll
+  for (int d = 0; d < Q; ++d) {
+    fetch_b(d, d);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) fetch_a(d, r, d);
+  }
+  int q = 0;
+  for (; q + Q < KQ; q += Q) {
+#pragma unroll
+    for (int d = 0; d < Q; ++d) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        mma(d, r);
+        fetch_a(d, r, q + d + Q);
+      }
+      fetch_b(d, q + d + Q);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < Q; ++d)
+    if (q + d < KQ) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (q + d + 1 == KQ && 4 * g + r < over) {
+#pragma unroll
+          for (int i = 0; i < MI; ++i) af[d][r][i] = (T)0;
+#pragma unroll
+          for (int i = 0; i < NI; ++i) bf[d][i][r] = (T)0;
+        }
+        mma(d, r);
+      }
+    }
+}
+
 // A: M-contiguous; B: K-contiguous (KB) or N-contiguous.  tm x tn x batch
 // tiles, one per wave: the M tiles of a column group in turn when the field is
-// B, the N tiles of a row group when it is A.
-template <typename T, typename TC, int MI, int NI, int D, bool KB, int EPI>
+// B, the N tiles of a row group when it is A.  QUADS: the products by gemm_tile_quads, D / 4 quads ahead.
+template <typename T, typename TC, int MI, int NI, int D, bool KB, bool QUADS, int EPI>
 __global__ void __launch_bounds__(256, 2)
     gemm_mode_kernel(const T *__restrict__ A, long lda, long sA, const T *__restrict__ B, long ldb,
                      TC *__restrict__ C, long ldc, long sC, int M, int N, int K, int tm, int tn,
@@ -192,7 +279,10 @@ __global__ void __launch_bounds__(256, 2)
   if (EPI == EPI_FIELDS) C = (TC *)ep.out[ib];
 
   acc_t acc[MI][NI];
-  gemm_tile<T, MI, NI, D, KB>(A, lda, B, ldb, M, N, K, m0, n0, acc);
+  if constexpr (QUADS)
+    gemm_tile_quads<T, MI, NI, D / 4>(A, lda, B, ldb, M, N, K, m0, n0, acc);
+  else
+    gemm_tile<T, MI, NI, D, KB>(A, lda, B, ldb, M, N, K, m0, n0, acc);
   // epilogue: lane holds C(m0+16mi+lane%16, n0+16ni+row(lane,r)).
   // Index splits (m -> i1,i2; n -> j,k) take one 32-bit division per lane and
   // then advance with wrap-around.
@@ -257,48 +347,22 @@ __global__ void __launch_bounds__(256, 2)
   }
 }
 
-// Tile of a product, in MFMA blocks: the one whose waves take the least time
-// on the busiest SIMD, a k-step of a wave costing its MFMAs (64 cycles each)
-// or its loads (512 B each, a CU's L1 delivering 64 B a cycle to 4 SIMDs),
-// whichever is more, and each wave the latency of its first loads.  At 254
-// points 64 x 64 tiles (4 waves per SIMD); 48 wide where that pads less (130
-// columns in three); a 62^3 field 16 x 16 tiles, since 64-wide ones would leave
-// fifteen SIMDs of sixteen empty.  Measured against block tiles staged through
-// LDS (one barrier pair per 16-deep step, two blocks per CU), bit for bit the
-// same results: a 256^3 FP64 solve 1.397 -> 1.051 ms, a 64^3 one 121 -> 37 us,
-// training targets 256^3 -> 64^3 1.90 -> 1.33 ms.
-struct GemmTile {
-  int mi, ni;
-};
-inline GemmTile gemm_tile_of(int M, int N, int K, int batch, int ncu) {
-  static const GemmTile all[] = {{4, 4}, {4, 3}, {3, 4}, {3, 3}, {4, 2}, {2, 4}, {2, 2}, {1, 1}};
-  GemmTile best = all[0];
-  double least = 0.0;
-  for (const GemmTile &t : all) {
-    const double w = (double)((M + 16 * t.mi - 1) / (16 * t.mi)) *
-                     ((N + 16 * t.ni - 1) / (16 * t.ni)) * batch;
-    const double per = std::ceil(w / (4.0 * ncu));
-    const double step = std::max(64.0 * t.mi * t.ni, 32.0 * (t.mi + t.ni));
-    const double cost = per * ((K + 3) / 4) * step + 2000.0 * std::ceil(per / 2.0);
-    if (least == 0.0 || cost < least) {
-      least = cost;
-      best = t;
-    }
-  }
-  return best;
-}
-
 // C = A B (per batch) with the epilogue EPI, enqueued on st.
 template <typename T, typename TC, bool KB, int EPI>
 void gemm_launch(const T *A, long lda, long sA, const T *B, long ldb, TC *C, long ldc, long sC,
                  int M, int N, int K, int batch, const EpiArgs &ep, int ncu, hipStream_t st) {
-  const GemmTile t = gemm_tile_of(M, N, K, batch, ncu);
+  // FP32: x by quads; y and z with more k-steps ahead, since a step's MFMAs take
+  // half the time (a z transform at 254^3 on 64 x 64 tiles 106 -> 90 us, at
+  // 192 x 256 x 192 on 64 x 48 ones 50 -> 45)
+  constexpr bool F32 = sizeof(T) == 4, X32 = KB && F32;
+  const bool quads = X32 && K >= 16;
+  const GemmTile t = X32 ? gemm_tile_x32(M, N, K, batch, ncu) : gemm_tile_of(M, N, K, batch, ncu);
   const int tm = (M + 16 * t.mi - 1) / (16 * t.mi), tn = (N + 16 * t.ni - 1) / (16 * t.ni);
   const long waves = (long)tm * tn * batch;
   const dim3 grid((unsigned)((waves + 3) / 4));
-  auto go = [&](auto mi, auto ni, auto d) {
+  auto go = [&](auto mi, auto ni, auto d, auto qd) {
     hipLaunchKernelGGL((gemm_mode_kernel<T, TC, decltype(mi)::value, decltype(ni)::value,
-                                         decltype(d)::value, KB, EPI>),
+                                         decltype(d)::value, KB, decltype(qd)::value, EPI>),
                        grid, dim3(256), 0, st, A, lda, sA, B, ldb, C, ldc, sC, M, N, K, tm, tn,
                        waves, ep);
   };
@@ -306,17 +370,26 @@ void gemm_launch(const T *A, long lda, long sA, const T *B, long ldb, TC *C, lon
   typedef std::integral_constant<int, 2> I2;
   typedef std::integral_constant<int, 3> I3;
   typedef std::integral_constant<int, 4> I4;
+  typedef std::integral_constant<int, F32 ? 6 : 4> D6;
+  typedef std::integral_constant<int, F32 ? 8 : 4> D8;
   typedef std::integral_constant<int, 8> I8;
   typedef std::integral_constant<int, 16> I16;
-  switch (10 * t.mi + t.ni) {
-    case 44: go(I4(), I4(), I4()); break;
-    case 43: go(I4(), I3(), I4()); break;
-    case 34: go(I3(), I4(), I4()); break;
-    case 33: go(I3(), I3(), I4()); break;
-    case 42: go(I4(), I2(), I4()); break;
-    case 24: go(I2(), I4(), I4()); break;
-    case 22: go(I2(), I2(), I8()); break;
-    default: go(I1(), I1(), I16()); break;
+  typedef std::false_type no;
+  if constexpr (X32) {
+    if (!quads) go(I1(), I1(), I16(), no());
+    else if (t.mi == 2) go(I2(), I2(), I16(), std::true_type());
+    else go(I1(), I1(), I16(), std::true_type());
+  } else {
+    switch (10 * t.mi + t.ni) {
+      case 44: go(I4(), I4(), D8(), no()); break;
+      case 43: go(I4(), I3(), D6(), no()); break;
+      case 34: go(I3(), I4(), D6(), no()); break;
+      case 33: go(I3(), I3(), D8(), no()); break;
+      case 42: go(I4(), I2(), D8(), no()); break;
+      case 24: go(I2(), I4(), D6(), no()); break;
+      case 22: go(I2(), I2(), I8(), no()); break;
+      default: go(I1(), I1(), I16(), no()); break;
+    }
   }
 }
 
