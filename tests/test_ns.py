@@ -380,47 +380,72 @@ def test_ns_advective_form_matches_oracle():
     _compare(mf, dev, orc, 1e-10, "nlt=1")
 
 
+def _launches(torch, name, run):
+    """Launches of kernels of that name while run() runs."""
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        run()
+        torch.cuda.synchronize()
+    return sum(name in e.name for e in prof.events())
+
+
+# kw, eddy viscosity: the default (the convective term axis by axis); and the
+# routes with stored gradients, whose derivative batches go over the streams:
+# the advective form, an eddy viscosity, and lines of more than 512 points
+CONVECTIVE = [((40, 48, 36), {}, 0, False), ((40, 48, 36), {"nlt": 1}, 0, True),
+              ((40, 48, 36), {}, 1, True), ((20, 24, 513), {}, 0, True)]
+
+
 @pytest.mark.gpu
+@pytest.mark.parametrize("shape,kw,les,stored", CONVECTIVE)
 @pytest.mark.parametrize("prec", [0, 3], ids=["fp64", "fp16x2"])
-def test_ns_concurrent_velocity_solves_match_sequential(monkeypatch, prec):
+def test_ns_concurrent_velocity_solves_match_sequential(monkeypatch, prec, shape, kw, les, stored):
     """The three velocity solves on three handles and streams (the default)
     against one handle in turn (MF_NS_CONCURRENT=0): the same kernels on the
     same data, so the fields agree bit for bit."""
     import mflops as mf
+    import torch
     mf.load()
-    gx, gy, gz, u, v, w, bc = _channel((40, 48, 36))
+    gx, gy, gz, u, v, w, bc = _channel(shape)
     re, dt, steps = 3000.0, 1e-3, 3
     runs = {}
     for conc in ("1", "0"):
-        print("run ns concurrent=%s precision=%d" % (conc, prec), flush=True)
+        print("run ns concurrent=%s precision=%d %s %s les=%d" % (conc, prec, shape, kw, les),
+              flush=True)
         monkeypatch.setenv("MF_NS_CONCURRENT", conc)
-        dev = _gpu_ns(mf, gx, gy, gz, u, v, w, bc, re, dt)
+        dev = _gpu_ns(mf, gx, gy, gz, u, v, w, bc, re, dt, **kw)
         dev.set_flow_rate(True, 2.0 / re)
-        dev.step(steps, prec, tol=1e-13)
+        if les:
+            dev.set_les(les, 0.02)
+        n = _launches(torch, "conv3d_kernel", lambda: dev.step(steps, prec, tol=1e-13))
+        assert (n == 0) == stored, n
         runs[conc] = [mf.to_host(t) for t in dev.get()]
     for name, a, b in zip(("u", "v", "w", "p", "phi"), runs["1"], runs["0"]):
         assert np.array_equal(a, b), (name, np.abs(a - b).max())
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tou", [1, 2, 3])
-def test_ns_fused_right_hand_sides_match_separate(monkeypatch, tou):
+@pytest.mark.parametrize("tou,shape,kw", [(1, (40, 48, 36), {"nlt": 1}), (2, (40, 48, 36), {"nlt": 1}),
+                                          (3, (40, 48, 36), {"nlt": 1}), (2, (20, 24, 513), {})])
+def test_ns_fused_right_hand_sides_match_separate(monkeypatch, tou, shape, kw):
     """The first presolve's velocity right-hand sides formed inside the
-    nonlinear-term kernel (pt = 1, the default) against rhs_kernel
-    (MF_NS_FUSED_RHS=0): the same arithmetic in the same order, so the
-    fields agree bit for bit."""
+    nonlinear-term kernel (pt = 1; the advective form, or lines of more than 512
+    points) against rhs_kernel (MF_NS_FUSED_RHS=0), which it then replaces: the
+    same arithmetic in the same order, so the fields agree bit for bit."""
     import mflops as mf
+    import torch
     mf.load()
-    gx, gy, gz, u, v, w, bc = _channel((40, 48, 36))
+    gx, gy, gz, u, v, w, bc = _channel(shape)
     re, dt, steps = 3000.0, 1e-3, 4
-    runs = {}
+    runs, rhs = {}, {}
     for fused in ("1", "0"):
-        print("run ns fused_rhs=%s tou=%d" % (fused, tou), flush=True)
+        print("run ns fused_rhs=%s tou=%d %s %s" % (fused, tou, shape, kw), flush=True)
         monkeypatch.setenv("MF_NS_FUSED_RHS", fused)
-        dev = _gpu_ns(mf, gx, gy, gz, u, v, w, bc, re, dt, tou=tou, top=tou)
+        dev = _gpu_ns(mf, gx, gy, gz, u, v, w, bc, re, dt, tou=tou, top=tou, **kw)
         dev.set_flow_rate(True, 2.0 / re)
-        dev.step(steps, mf.MF_FP64)
+        rhs[fused] = _launches(torch, "rhs_kernel", lambda: dev.step(steps, mf.MF_FP64))
         runs[fused] = [mf.to_host(t) for t in dev.get()]
+    print("  rhs_kernel launches", rhs, flush=True)
+    assert rhs["1"] < rhs["0"]
     for name, a, b in zip(("u", "v", "w", "p", "phi"), runs["1"], runs["0"]):
         assert np.array_equal(a, b), (name, np.abs(a - b).max())
 
