@@ -154,12 +154,15 @@ __global__ void __launch_bounds__(64 * MLP_WAVES, 2)
     mlp_grad_kernel(const float *__restrict__ X, const float *__restrict__ T, long n,
                     const unsigned short *__restrict__ wb, const float *__restrict__ p,
                     double *__restrict__ part) {
-  __shared__ float S[3][H][MLP_PITCH];             // h2 then dh1 | dh2 | h1
-  __shared__ float SX[I0 + 1][MLP_PITCH];          // inputs and a row of ones
-  __shared__ float SD[O][MLP_PITCH];               // dY
-  __shared__ float W2[H][MLP_PITCH];               // widened; rows forward, columns backward
-  __shared__ unsigned short W3[O][MLP_WP], W3t[H][8];
-  __shared__ float B2[H];
+  // read four values at a time (mlp_f4, mlp_widen4): aligned bases and pitches
+  __shared__ alignas(16) float S[3][H][MLP_PITCH];     // h2 then dh1 | dh2 | h1
+  __shared__ alignas(16) float SX[I0 + 1][MLP_PITCH];  // inputs and a row of ones
+  __shared__ alignas(16) float SD[O][MLP_PITCH];       // dY
+  __shared__ alignas(16) float W2[H][MLP_PITCH];       // widened; rows forward, columns backward
+  __shared__ alignas(16) unsigned short W3[O][MLP_WP], W3t[H][8];
+  __shared__ alignas(16) float B2[H];
+  static_assert(MLP_PITCH * sizeof(float) % sizeof(mlp_f4) == 0 &&
+                MLP_WP * sizeof(unsigned short) % sizeof(uint2) == 0, "rows stay aligned");
   const int tid = threadIdx.x, l = tid & 63, c = l & 15, g = l >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   for (int t = tid; t < NW2; t += 64 * MLP_WAVES) W2[t / H][t % H] = bf2f(wb[NW1 + t]);
