@@ -742,6 +742,7 @@ int mlp_grad(mf_mlp *h, const float *X, const float *T, long n, hipStream_t st) 
       LESCHK(hipStreamSynchronize(st));
       (void)hipFree(h->part);
       h->part = nullptr;
+      h->part_blocks = 0;  // should the allocation fail, the next call tries again
     }
     LESCHK(hipMalloc(&h->part, (size_t)nb * (NPARAM + 1) * sizeof(double)));
     h->part_blocks = nb;
