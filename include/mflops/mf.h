@@ -179,7 +179,11 @@ int mf_influence_impulses(mf_solver3d *sc, const mf_der *dx, const mf_der *dy,
  * solver and three solver-mode derivative handles per subdomain and
  * assembles the influence matrix (md_influence_matrix_set) on the device, as
  * one dense block per subdomain over the unknowns of its interfaces; sigma
- * is fixed at creation (the matrix depends on it).  Synchronous. */
+ * is fixed at creation (the matrix depends on it).  The blocks are what
+ * mf_md_matvec multiplies by and mf_md_write_matrix stores; mf_md_solve applies
+ * the same matrix from its one-axis factors, which the solvers hold, and
+ * reads the blocks only when they were formed by unit-impulse solves
+ * (MF_INFL_IMPULSES=1 in the environment of the create call).  Synchronous. */
 typedef struct mf_md mf_md;
 typedef struct mf_md_report {
   int iterations;   /* GMRES iterations                                  */
@@ -195,7 +199,8 @@ int mf_md_info(const mf_md *h, int *nsub, long long *ninf, long long *matrix_byt
 int mf_md_matvec(mf_md *h, const double *x, double *y, void *stream);
 /* Solve: g[s], u[s] are device full-size fields of subdomain s; bc[s] its
  * boundary arrays [bcx(n2,n3,2) | bcy(n1,n3,2) | bcz(n1,n2,2)] (outer faces
- * used, interface faces ignored).  The interface system is solved by
+ * used, interface faces ignored).  The interface system (its matrix from
+ * factors, equal to the blocks to rounding; see mf_md_create) is solved by
  * restarted GMRES(30) from x = 0 until the relative residual is <= tol
  * (<= 0 selects 1e-10) or max_iter iterations (<= 0: 1000); then every
  * subdomain is solved with the interface values, FP64.  x_iface (optional,
@@ -216,7 +221,9 @@ int mf_md_set_guess(mf_md *h, int enable);
  * (nd, bct, so, sigma, a hash of the slab sizes and grids, sizes) then the
  * dense blocks.  mf_md_create_cached reads the blocks from path when its
  * header matches the arguments, else assembles them as mf_md_create and
- * writes path; *loaded (optional) tells which. */
+ * writes path; *loaded (optional) tells which.  As with mf_md_create, the
+ * blocks, read or assembled, serve mf_md_matvec; mf_md_solve takes them as its
+ * matrix only with MF_INFL_IMPULSES=1. */
 int mf_md_write_matrix(const mf_md *h, const char *path);
 int mf_md_create_cached(const int nd[3], const int *npts, const double *grids, const int bct[6],
                         int so, double sigma, const char *path, int *loaded, mf_md **out);
