@@ -389,9 +389,11 @@ __global__ void __launch_bounds__(64 * SEG_KMAX) der3d_seg_kernel(FieldSet fs, S
 // component per block, blocks of the three components of the same lines next to
 // each other (the advecting component they share then comes from the L2).
 // Bounds: HBM, 6 fields on the first axis and 9 on the others (stored products
-// and derivatives take 78 in all, with their kernels and the sum's), and on
-// the first, where the lines are contiguous, the waves' own latencies: 2 blocks
-// fill a CU's registers.  192 x 256 x 192: 246 + 193 + 204 us (1.8, 3.5 and
+// and derivatives take 78 in all, with their kernels and the sum's), and
+// registers: a pair's values, results and addresses need more than the 128
+// that launch bounds for 16 waves leave, so that a lane keeps 161 to 185 of them
+// (240 to 243 pentadiagonal) in scratch memory, 268 bytes a lane on the first
+// axis.  192 x 256 x 192: 246 + 193 + 204 us (1.8, 3.5 and
 // 3.3 TB/s), where products, 18 derivatives and the sum with the right-hand
 // sides took 1330, and right-hand sides on their own now take 207; a time
 // step 4.09 -> 3.53 ms.  At 24^3 to 64^3, three launches in turn for five with

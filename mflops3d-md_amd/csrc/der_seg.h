@@ -25,6 +25,13 @@
 // and reach the FMAs through v_readlane, which has no latency to wait for:
 // 28 lane reads and 15 FP64 operations per row.  (Scalar loads, four rows per wait on a
 // 24 KB table that the 16 KB scalar cache does not hold, kept a wave waiting.)
+// Lane reads cost issue slots instead: on fields that stay in cache, pentadiagonal
+// lines of 64 to 200 points along y and z take 5 to 20% longer than with scalar
+// loads (38 x 200 x 200, one derivative along z, 13.4 us then and 16.5 now), all
+// else less.  Blocks of up to 16 waves leave a wave 128 registers: the solves
+// along y and z keep within them, those of contiguous lines put 7 to 9
+// (tridiagonal) or 26 to 32 registers of a lane into scratch memory, and pairs
+// 161 to 185 or 240 to 243.
 // Where the factored matrix is tridiagonal (p = e = 0: the schemes of order 6
 // and below) a second instance drops p, e, A, D and one of the two exchanged
 // values: 20 lane reads and 11 operations.
@@ -47,7 +54,9 @@ constexpr int SEG_LEN = 32;     // longest segment, on lines of up to 16 of them
 constexpr int SEG_LONG = 33;    // longest on the lines just beyond (an instance of its own)
 // Whether the lines along y or z of a field of nx columns go in groups of
 // `lines` aligned in memory: rows of whole cache lines (16 points), and few
-// lanes lost at the rows' ends.
+// lanes lost at the rows' ends.  Six fields of 192 x 256 x 192 along y / z 253 / 272
+// -> 238 / 253 us, three of 256^3 212 / 227 -> 191 / 200 us; the same time either
+// way on fields that stay in cache (64^3, 496 x 64 x 60).
 inline bool seg_aligned(int nx, int lines) {
   return nx % 16 == 0 && 16 * ((nx + lines - 1) / lines * lines - nx) <= 2 * nx;
 }

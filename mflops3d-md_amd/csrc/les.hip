@@ -143,10 +143,10 @@ inline unsigned nblk(long n) { return (unsigned)((n + 255) / 256); }
 // ---- learned-closure data path ----
 // The x pass of three filtered fields at once: w1_f = F B_f for the fields
 // (G = 0) u, v, w, (1) uu, uv, uw or (2) vv, vw, ww, formed from u, v, w as
-// they are loaded; or of one field, (3) u or (4) uv.  One wave takes 16 MI filtered points of 16 columns, three
-// accumulators deep: the matrix's operands serve all three fields, and no
-// product field is written.  Bounded by the FP64 matrix rate (24 MFMAs of 64
-// cycles on 10 loads per step at 64 points); 256^3 -> 64^3 with its y and z
+// they are loaded; or of one field, (3) u or (4) uv.  One wave takes 16 MI
+// filtered points of 16 columns, three accumulators deep: the matrix's operands
+// serve all three fields, and no product field is written.  Bounded by the FP64
+// matrix rate (12 MFMAs of 64 cycles on 7 loads per step at 64 points); 256^3 -> 64^3 with its y and z
 // passes 1.26 -> 0.62 ms for all nine fields (a pass over memory per product,
 // and a GEMM of its own for each field and axis, before).
 constexpr int FX_D = 4;  // k-steps in flight

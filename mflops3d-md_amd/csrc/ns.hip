@@ -620,7 +620,7 @@ struct mf_ns {
   std::vector<double> gx, gy, gz;
   int grad_level = -1;  // level whose velocity gradients T[0..8] hold
   // the first presolve's velocity right-hand sides formed by nl_kernel
-  // (pt = 1, no LES; MF_NS_FUSED_RHS=0: by rhs_kernel)
+  // (pt = 1, no LES, terms not axis by axis; MF_NS_FUSED_RHS=0: by rhs_kernel)
   bool fused_rhs = true;
   // LES (navier_LES): model, constant squared, fields -les_f (3) and nu,
   // squared spacings
@@ -703,7 +703,11 @@ int der3(mf_ns *s, int axis, const double *x0, const double *x1, const double *x
 
 // Whether the nonlinear terms go axis by axis (conv3d): the skew-symmetric
 // form on lines it takes (faster at every size measured, 24^3 to 192 x 256 x
-// 192), unless the subgrid stresses want the gradients anyway.
+// 192), unless the subgrid stresses want the nine gradients, which would then
+// be a batch of their own.  An FP64 step with a closure as it is / axis by axis:
+// 24^3 440-457 / 457-470 us, 64^3 467-484 / 487-528, 96^3 703-826 / 745-869; but
+// 128^3 1.27-1.52 / 1.23-1.50 ms and 192 x 256 x 192 5.46-6.68 / 5.20-6.42 ms, which
+// is not made use of.
 bool conv_by_axis(const mf_ns *s) {
   return s->nlt == 2 && !s->les_type && !s->sgs && mf::conv3d_takes(s->dc, s->nx, s->ny, s->nz);
 }
@@ -1006,8 +1010,9 @@ int substep(mf_ns *s, int sub, int precision, double tol, bool *done, hipStream_
   }
   NSCHK(hipGetLastError());
   // nonlinear terms of the levels the extrapolation reads, the older ones
-  // first: for pt = 1 without LES the newest one's kernel also forms the
-  // velocity right-hand sides (into T[0..2]), which read the older ones
+  // first: for pt = 1 without LES the newest one's kernel, where it is nl_kernel
+  // (the advective form, or lines conv3d does not take), also forms the velocity
+  // right-hand sides (into T[0..2]), which read the older ones
   const bool fuse_rhs = s->fused_rhs && !conv_by_axis(s) && pt == 1 && sub == 1 && !s->les_type && !s->sgs &&
                         ev.c[0] != 0.0 && ev.lev[0] == L0 && !s->nl_ok[ev.lev[0]];
   for (int m = 2; m >= 1; --m)
