@@ -9,8 +9,9 @@
 // plus dcoef x_f on the faces of t's own axis.  That is O(n^3) work and
 // O(n^2) memory per subdomain, where the dense block is O(n^4) doubles to
 // read per product: at 2 x 2 x 2 subdomains of 48-96 points 8.6 GB and 1.72 ms
-// (5 TB/s) against six launches; a solve (9 iterations) 20.4 -> 2.8 ms.  The four transforms of all faces of
-// all subdomains run as grouped launches of one-wave 16 x 16 tiles
+// (5 TB/s) against six launches; a solve (9 iterations) 20.4 -> 2.8 ms, 2.0 with
+// one wait per iteration.  The four transforms of all faces of all subdomains run
+// as grouped launches of one-wave 16 x 16 tiles
 // (gemm_tile), bounded by their latency at these sizes, as is the spectral
 // sum, which forms R anew for each of the three axes it sums along rather than
 // storing U.
